@@ -179,35 +179,57 @@ struct TraceResult {
 	float b1, b2;
 };
 
-// Per-lane traversal stack: the first nLds entries in LDS (entries `stride`
-// ints apart, so a wave's 64 lanes hit 64 banks), deeper entries in a global
-// overflow area laid out lane-fastest (entries `ovStride` ints apart:
+// Per-lane traversal stack: the first nLds entries in LDS, deeper entries in a
+// global overflow area laid out lane-fastest (entries `ovStride` ints apart:
 // coalesced when the lanes of a wave spill together).  A small LDS footprint
-// keeps the traversal kernels at high occupancy; deep stacks are rare but
-// stay exact.  nLds is uniform over the launch (kShortStack by default).
+// keeps the traversal kernels at high occupancy; deep stacks are rare but stay
+// exact.  nLds is uniform over the launch.
 //
-// Each lane owns nLds + 1 LDS slots.  Every push writes LDS slot
-// min(sp, nLds) - the extra slot absorbs the pushes that belong to the
-// overflow area - and every pop reads that slot, so the common case is one
-// ds_write / ds_read; only entries at sp >= nLds also take a (rarely
-// entered) branch to global memory.  A pointer chosen between LDS and
-// global memory would compile to flat loads and stores on every access.
+// Each wave owns nLds + kStackPad rows of 64 ints, lane-fastest, so a wave's
+// 64 lanes hit 64 banks, entry e of a lane is e * 256 bytes from its first, and
+// the three entries a node can push go to constant offsets from one address.
+// A push writes all three rows whatever the number of children to keep: the
+// valid ones come first, the rows above are overwritten by later pushes, and
+// the pad rows take them at the top of the area.  Lanes past nLds send their
+// wave through a path that also serves the overflow area; the common path has
+// one compare for it.  (A push at a time, each with its own address, bound and
+// branch, took 21 vector instructions for the three; this takes 10.)  With the
+// loops per node kind below: 2^20 incoherent closest and 2^20 shadow rays in the
+// 1.31 M-triangle field 1369 against 1550 us, the 36-triangle Cornell box at
+// 256x256, 16 samples 3.91 against 4.18 ms, the field's 1080p frame 3.72
+// against 3.77 ms.
 constexpr int kShortStack = 16;
+constexpr int kStackPad	  = 3;
 struct LaneStack {
-	int *lds;
-	int stride;
+	int *lds; // this lane's entry 0
 	int *ovf;
 	int ovStride;
 	int nLds;
-	// LDS slot min(sp, nLds) * stride: both factors are below 2^23, so the
-	// full-rate 24-bit multiply gives the product
-	KRR_DEV int slot(int sp) const { return __mul24(min(sp, nLds), stride); }
-	KRR_DEV void put(int sp, int v) const {
-		lds[slot(sp)] = v;
-		if (sp >= nLds) ovf[(size_t) (sp - nLds) * ovStride] = v;
+	KRR_DEV void put(int e, int v) const {
+		if (e < nLds) lds[e * 64] = v;
+		else ovf[(size_t) (e - nLds) * ovStride] = v;
 	}
-	KRR_DEV int get(int sp) const {
-		int v = lds[slot(sp)];
+	// Pushes the hit children c1 (nearest) to c3 in the order c3, c2, c1;
+	// h3 implies h2 implies h1.
+	KRR_DEV void push(int &sp, bool h1, bool h2, bool h3, int c1, int c2, int c3) const {
+		const int e0 = h3 ? c3 : (h2 ? c2 : c1), e1 = h3 ? c2 : c1;
+		const int n	 = sp + (h1 ? 1 : 0) + (h2 ? 1 : 0) + (h3 ? 1 : 0);
+		if (__builtin_expect(__ballot(n > nLds) == 0, 1)) { // sp <= nLds: the three rows are inside the area
+			int *p = lds + sp * 64;
+			p[0]   = e0;
+			p[64]  = e1;
+			p[128] = c1;
+		} else {
+			if (h1) put(sp, e0);
+			if (h2) put(sp + 1, e1);
+			if (h3) put(sp + 2, c1);
+		}
+		sp = n;
+	}
+	KRR_DEV int pop(int &sp) const {
+		sp--;
+		if (__builtin_expect(__ballot(sp >= nLds) == 0, 1)) return lds[sp * 64];
+		int v = lds[min(sp, nLds) * 64];
 		// keeps the LDS read a ds_read: without the barrier the compiler folds
 		// both reads into one flat load of a selected address
 		asm volatile("" : "+v"(v));
@@ -271,11 +293,18 @@ KRR_DEV SlabRay slabRay(const f3 &o, const f3 &d) {
 constexpr float kWiden = 1.00000036f;			 // 1 + 2*gamma(3)
 constexpr float kTie   = 1.00000095367431640625f; // 1 + 2^-20
 
+// Which nodes a traversal reads: float nodes from global memory, float nodes
+// with the top of the tree in LDS ("lds_nodes"), quantised nodes.  Uniform over
+// a launch; each kind has a loop of its own (a branch per node visit kept the
+// loads' registers apart from the slab test's and cost moves between them).
+enum class Nodes { Float, FloatLds, Quantized };
+
 // Slab test of the four children of inner node `entry` against [0, tlim]:
 // k[i] = entry distance of child i, +inf when missed; c[i] = its reference.
-// Float nodes are read from LDS for entries below nLdsNodes (the block's copy
+// FloatLds nodes are read from LDS for entries below nLdsNodes (the block's copy
 // of the top of the tree), from global memory otherwise: seven 16-byte loads
 // of the node's 128-byte line (the six planes the ray needs and the children).
+template <Nodes NODES>
 KRR_DEV void nodeTest(const TraceBvh &bvh, const SlabRay &sr, int entry, float tlim, const float4 *nodeLds, int nLdsNodes, float &k0,
 					  float &k1, float &k2, float &k3, int &c0, int &c1, int &c2, int &c3) {
 #define KRR_SLAB(kc, px, qx, py, qy, pz, qz)                                                                                                   \
@@ -284,7 +313,7 @@ KRR_DEV void nodeTest(const TraceBvh &bvh, const SlabRay &sr, int entry, float t
 		const float t1 = fminf(fminf(fminf(fmaf(qx, sr.ix, sr.bfx), fmaf(qy, sr.iy, sr.bfy)), fmaf(qz, sr.iz, sr.bfz)) * kWiden, tlim);         \
 		kc			   = t0 <= t1 ? t0 : __builtin_inff();                                                                                      \
 	}
-	if (bvh.qnodes) {
+	if constexpr (NODES == Nodes::Quantized) {
 		// One 64-byte quantised node: {org, e, valid}, planes lox hix loy
 		// hiy, planes loz hiz + children 0 1, children 2 3.  Plane c of a
 		// dword is byte c; org + q 2^e is exact (one fma, no rounding).
@@ -316,7 +345,7 @@ KRR_DEV void nodeTest(const TraceBvh &bvh, const SlabRay &sr, int entry, float t
 	} else {
 		float4 nx, fx, ny, fy, nz, fz;
 		int4 ch;
-		if (entry < nLdsNodes) {
+		if (NODES == Nodes::FloatLds && entry < nLdsNodes) {
 			const float4 *np = nodeLds + (uint32_t) entry * 8u;
 			nx				 = np[sr.nX >> 4];
 			fx				 = np[(sr.nX ^ 16u) >> 4];
@@ -387,8 +416,8 @@ KRR_DEV void nodeTest(const TraceBvh &bvh, const SlabRay &sr, int entry, float t
 // testing the leaves of a node on the spot, slot by slot, made the wave run
 // up to four leaf blocks per node visit, each for the few lanes whose child in
 // that slot was a hit leaf.  The closest hit does not depend on the order.
-template <bool ANY, bool COUNT, bool ALPHA = false>
-KRR_DEV TraceResult traverse(const TraceBvh &bvh, const f3 &o, const f3 &d, float tmax, const LaneStack &stack,
+template <bool ANY, bool COUNT, bool ALPHA, Nodes NODES>
+KRR_DEV TraceResult traverseNodes(const TraceBvh &bvh, const f3 &o, const f3 &d, float tmax, const LaneStack &stack,
 							 uint32_t &nodeVisits, uint32_t &triTests) {
 	TraceResult res{tmax, -1, 0.f, 0.f};
 	const RayPre rp	 = rayPre(o, d);
@@ -423,24 +452,29 @@ KRR_DEV TraceResult traverse(const TraceBvh &bvh, const f3 &o, const f3 &d, floa
 				}
 			}
 			if (sp == 0) break;
-			entry = stack.get(--sp);
+			entry = stack.pop(sp);
 			continue;
 		}
 		if (COUNT) nodeVisits++;
 		float k0, k1, k2, k3;
 		int c0, c1, c2, c3;
-		nodeTest(bvh, sr, entry, res.t * kTie, nullptr, 0, k0, k1, k2, k3, c0, c1, c2, c3);
+		nodeTest<NODES>(bvh, sr, entry, res.t * kTie, nullptr, 0, k0, k1, k2, k3, c0, c1, c2, c3);
 		if (k0 == __builtin_inff()) {
 			if (sp == 0) break;
-			entry = stack.get(--sp);
+			entry = stack.pop(sp);
 			continue;
 		}
-		if (k3 != __builtin_inff()) stack.put(sp++, c3);
-		if (k2 != __builtin_inff()) stack.put(sp++, c2);
-		if (k1 != __builtin_inff()) stack.put(sp++, c1);
+		stack.push(sp, k1 != __builtin_inff(), k2 != __builtin_inff(), k3 != __builtin_inff(), c1, c2, c3);
 		entry = c0;
 	}
 	return res;
+}
+
+template <bool ANY, bool COUNT, bool ALPHA = false>
+KRR_DEV TraceResult traverse(const TraceBvh &bvh, const f3 &o, const f3 &d, float tmax, const LaneStack &stack, uint32_t &nodeVisits,
+							 uint32_t &triTests) {
+	if (bvh.qnodes) return traverseNodes<ANY, COUNT, ALPHA, Nodes::Quantized>(bvh, o, d, tmax, stack, nodeVisits, triTests);
+	return traverseNodes<ANY, COUNT, ALPHA, Nodes::Float>(bvh, o, d, tmax, stack, nodeVisits, triTests);
 }
 
 // Default refill threshold of the persistent launch (pass param
@@ -496,10 +530,9 @@ KRR_DEV void travInit(TravState &s, const TraceBvh &bvh, float tmax) {
 // leafShare % of the traversing lanes hold one, inner nodes otherwise; the
 // other lanes wait.  A mixed iteration runs both code paths, each for part of
 // the wave.  Each ray still takes its own entries in its own order.
-template <bool COUNT, bool ALPHA>
-KRR_DEV void traverseSteps(const TraceBvh &bvh, const f3 &o, const f3 &d, const bool any, bool &going, TravState &s,
-						   const LaneStack &stack, const int minLanes, uint32_t &nodeVisits, uint32_t &triTests,
-						   const float4 *nodeLds = nullptr, int nLdsNodes = 0, int leafShare = 0) {
+template <bool COUNT, bool ALPHA, Nodes NODES>
+KRR_DEV void traverseStepsNodes(const TraceBvh &bvh, const f3 &o, const f3 &d, const bool any, bool &going, TravState &s, const LaneStack &stack,
+								const int minLanes, uint32_t &nodeVisits, uint32_t &triTests, const float4 *nodeLds, int nLdsNodes, int leafShare) {
 	const RayPre rp	 = rayPre(o, d);
 	const SlabRay sr = slabRay(o, d);
 	while (true) {
@@ -548,26 +581,33 @@ KRR_DEV void traverseSteps(const TraceBvh &bvh, const f3 &o, const f3 &d, const 
 				going = false;
 				continue;
 			}
-			s.entry = stack.get(--s.sp);
+			s.entry = stack.pop(s.sp);
 			continue;
 		}
 		if (COUNT) nodeVisits++;
 		float k0, k1, k2, k3;
 		int c0, c1, c2, c3;
-		nodeTest(bvh, sr, s.entry, s.t * kTie, nodeLds, nLdsNodes, k0, k1, k2, k3, c0, c1, c2, c3);
+		nodeTest<NODES>(bvh, sr, s.entry, s.t * kTie, nodeLds, nLdsNodes, k0, k1, k2, k3, c0, c1, c2, c3);
 		if (k0 == __builtin_inff()) {
 			if (s.sp == 0) {
 				going = false;
 				continue;
 			}
-			s.entry = stack.get(--s.sp);
+			s.entry = stack.pop(s.sp);
 			continue;
 		}
-		if (k3 != __builtin_inff()) stack.put(s.sp++, c3);
-		if (k2 != __builtin_inff()) stack.put(s.sp++, c2);
-		if (k1 != __builtin_inff()) stack.put(s.sp++, c1);
+		stack.push(s.sp, k1 != __builtin_inff(), k2 != __builtin_inff(), k3 != __builtin_inff(), c1, c2, c3);
 		s.entry = c0;
 	}
+}
+
+template <bool COUNT, bool ALPHA>
+KRR_DEV void traverseSteps(const TraceBvh &bvh, const f3 &o, const f3 &d, const bool any, bool &going, TravState &s, const LaneStack &stack,
+						   const int minLanes, uint32_t &nodeVisits, uint32_t &triTests, const float4 *nodeLds, int nLdsNodes, int leafShare) {
+	if (bvh.qnodes) traverseStepsNodes<COUNT, ALPHA, Nodes::Quantized>(bvh, o, d, any, going, s, stack, minLanes, nodeVisits, triTests, nullptr, 0, leafShare);
+	else if (nLdsNodes > 0)
+		traverseStepsNodes<COUNT, ALPHA, Nodes::FloatLds>(bvh, o, d, any, going, s, stack, minLanes, nodeVisits, triTests, nodeLds, nLdsNodes, leafShare);
+	else traverseStepsNodes<COUNT, ALPHA, Nodes::Float>(bvh, o, d, any, going, s, stack, minLanes, nodeVisits, triTests, nullptr, 0, leafShare);
 }
 
 } // namespace krr

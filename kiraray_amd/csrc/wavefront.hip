@@ -1113,7 +1113,7 @@ k_megakernel_refill(WfParams P0, DevScene sc, TraceBvh bvh, RayQueueDev q, const
 	const LaneStack stack = laneStack(bvh, ldsStack, ovf);
 	WfParams P			  = P0;
 	// the top P.ldsNodes nodes of the tree, copied into LDS behind the stack
-	float4 *nodeLds = reinterpret_cast<float4 *>(ldsStack + (size_t) (bvh.stackLds + 1) * blockDim.x);
+	float4 *nodeLds = reinterpret_cast<float4 *>(ldsStack + (size_t) (bvh.stackLds + kStackPad) * blockDim.x);
 	if (P.ldsNodes > 0) {
 		const float4 *src = reinterpret_cast<const float4 *>(bvh.nodes);
 		for (int i = (int) threadIdx.x; i < P.ldsNodes * 8; i += (int) blockDim.x) nodeLds[i] = src[i];
@@ -1392,7 +1392,9 @@ struct AccelData {
 	int maxDepth	= 0;
 	double buildSeconds = 0;
 	bool onDevice		= false; // built by the GPU builder
-	int ldsEntries() const { return std::min(stackSize, stackLds); }
+	// entries kept in LDS: "stack_lds_entries" less the two rows the pad has
+	// beyond one, so that the LDS a setting takes does not depend on the pad
+	int ldsEntries() const { return std::min(stackSize, std::max(0, stackLds - (kStackPad - 1))); }
 	TraceBvh dev() const {
 		return TraceBvh{nodes.as<Bvh4Node>(), tris.as<LeafTri>(), ldsEntries(), (int) std::min<int64_t>(INT32_MAX, nNodes + nLeafTris),
 						alphaTri.as<AlphaTri>(), alphaSrc.as<AlphaSrc>(), quantized ? qnodes.as<Bvh4QNode>() : nullptr};
@@ -1608,8 +1610,7 @@ template <class K> int persistentGrid(K kernel, int block, size_t lds, int maxBl
 
 // LDS bytes per block of the short traversal stack, and ints per grid thread
 // of its global overflow.
-// nLds entries + one slot that absorbs the pushes bound for the overflow area
-size_t stackLds(const AccelData &a, int block) { return (size_t) (a.ldsEntries() + 1) * block * sizeof(int); }
+size_t stackLds(const AccelData &a, int block) { return (size_t) (a.ldsEntries() + kStackPad) * block * sizeof(int); }
 size_t stackOverflowInts(const AccelData &a) { return (size_t) (a.stackSize - a.ldsEntries()); }
 
 // A fraction of a persistent grid (at least one block).
@@ -2522,7 +2523,7 @@ int krr_wf_render(krr_wf *wf, float *film_dev, void *hip_stream) {
 	const int tb	   = wf->traceBlockSize;
 	const int gTmax	   = (N + tb - 1) / tb;
 	const size_t lds   = stackLds(wf->accel, tb);
-	if ((size_t) (bvh.stackLds + 1) * tb * sizeof(int) != lds) return krr::fail(KRR_ERR_INVALID_ARG, "krr_wf_render: stack layout mismatch");
+	if ((size_t) (bvh.stackLds + kStackPad) * tb * sizeof(int) != lds) return krr::fail(KRR_ERR_INVALID_ARG, "krr_wf_render: stack layout mismatch");
 	const bool count   = wf->countTraversal;
 	const bool media   = wf->enableMedium && wf->sceneHasMedia;
 	const bool plain   = !wf->sceneTextured;
@@ -3323,7 +3324,7 @@ int krr_mk_render(krr_mk *mk, float *film_dev, void *hip_stream) {
 		if (!mk->rays.p) KRR_HIP(mk->rays.alloc(2 * sizeof(unsigned long long)));
 		mk->gridKey = key;
 	}
-	if ((size_t) (bvh.stackLds + 1) * tb * sizeof(int) != lds) return krr::fail(KRR_ERR_INVALID_ARG, "krr_mk_render: stack layout mismatch");
+	if ((size_t) (bvh.stackLds + kStackPad) * tb * sizeof(int) != lds) return krr::fail(KRR_ERR_INVALID_ARG, "krr_mk_render: stack layout mismatch");
 	PtArgs a;
 	a.sc		  = wf->ds;
 	a.bvh		  = bvh;
