@@ -254,7 +254,8 @@ def kernel_rooflines(cfg, prm, steps, tot, cnt):
     max_depth = prm["max_depth"]
     NODE_B = NODE_BYTES[prm.get("node_format", "float")]
     wdepths = prm["wavefront_depths"]
-    mega_launches = steps * spp if wdepths <= max_depth else 0
+    # with every depth in the persistent launch, one launch runs all samples of a frame
+    mega_launches = (steps if wdepths == 0 else steps * spp) if wdepths <= max_depth else 0
     wf_closest = cnt["closest_rays"] - cnt["megakernel_closest_rays"]
     wf_shadow = cnt["shadow_rays"] - cnt["megakernel_shadow_rays"]
     out = {}

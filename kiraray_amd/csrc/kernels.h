@@ -98,7 +98,11 @@ KRR_DEV uint32_t trainHash(uint32_t pixel) {
 }
 
 struct CameraDev {
-	float filmH, focalLength, focalDistance, lensRadius, aspect;
+	// tan(atan2(film height / 2, focal length)) by detmath on the host: the same
+	// bits as on the device, where each camera ray computed it anew in about
+	// 150 FP64 instructions
+	float tanFov;
+	float focalDistance, lensRadius, aspect;
 	float M[12];
 	int medium;
 };
@@ -118,6 +122,7 @@ struct WfParams {
 	uint32_t sampleIndex; // frameIndex * spp (as uint)
 	int refillLanes;	  // persistent launch without media: end a traversal round below this many traversing lanes (1..64)
 	int ldsNodes;		  // refill launch: tree nodes 0..ldsNodes-1 are read from a per-block copy in LDS
+	int chain;			  // persistent launch: samples of a pixel run one after the other by the lane that takes it up
 	int leafShare;		  // refill launch: leaf-only iterations once this percent of traversing lanes hold a leaf (0: off)
 };
 
@@ -258,8 +263,7 @@ KRR_DEV RayItem cameraRay(const CameraDev &cam, int W, int H, int x, int y, Pcg 
 	const float p1	 = (float) y + 0.5f + cs[1];
 	const float ndc0 = (2.f * p0) / (float) W + (-1.f);
 	const float ndc1 = (2.f * p1) / (float) H + (-1.f);
-	const float fov	 = detmath::atan2f(cam.filmH * 0.5f, cam.focalLength);
-	const f3 fd		 = normalize(f3(detmath::tanf(fov) * cam.aspect * ndc0, detmath::tanf(fov) * ndc1, -1.f));
+	const f3 fd		 = normalize(f3(cam.tanFov * cam.aspect * ndc0, cam.tanFov * ndc1, -1.f));
 	f3 o, d;
 	if (cam.lensRadius > 1e-5f) {
 		float ax, ay;

@@ -156,22 +156,6 @@ KRR_DEV void storePathRegs(const PixelStateDev &px, int pixel, const PathRegs &p
 	px.rng[pixel] = pr.rng;
 }
 
-// Camera ray of global pixel i for the current sample (k_camera per view);
-// the pixel's radiance (zero unless the reference's spp loop keeps it) and
-// sampler state after the camera draws go to pr.
-KRR_DEV RayItem viewCameraRay(const WfParams &P, const ViewsDev &V, const PixelStateDev &px, int i, PathRegs &pr, bool media) {
-	const int v		= findView(V, i);
-	const int local = i - V.start[v];
-	const ViewDev &vw = V.view[v];
-	pr				  = loadPathRegs(px, i, media);
-	if (!P.legacySpp) pr.L = f3();
-	Pcg s{pr.rng, P.inc};
-	RayItem r = cameraRay(vw.cam, vw.W, vw.H, local % vw.W, local / vw.W, s);
-	r.pixel	  = i;
-	pr.rng	  = s.state;
-	return r;
-}
-
 // Film write of every view (k_film per view).
 __global__ void k_film_views(WfParams P, ViewsDev V, PixelStateDev px) {
 	const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -180,7 +164,12 @@ __global__ void k_film_views(WfParams P, ViewsDev V, PixelStateDev px) {
 	const int local	  = i - V.start[v];
 	const ViewDev &vw = V.view[v];
 	const int x = local % vw.W, y = local / vw.W;
-	const float4 p = px.pixel[i];
+	float4 p	   = px.pixel[i];
+	const float4 L = px.L[i]; // the frame's last sample, as in k_film
+	p.x			   = p.x + L.x;
+	p.y			   = p.y + L.y;
+	p.z			   = p.z + L.z;
+	px.pixel[i]	   = p;
 	float r = p.x / (float) P.spp, g = p.y / (float) P.spp, b = p.z / (float) P.spp;
 	if (P.enableClamp) {
 		r = clampf(r, 0.f, P.clampMax);
@@ -989,6 +978,75 @@ __global__ void k_mega_begin(Counters *cnt) {
 	cnt->closestLaunches += 1;
 }
 
+// Takes up the next path of each idle lane of the persistent launch: the next
+// sample of the lane's pixel while `left` samples remain, else the first
+// sample of the next pixel (one atomic per wave for all such lanes), or with
+// neither VIEWS nor camFetch the next item of the ray queue.  Camera rays are
+// made here (generateCameraRays, integrator.cpp:166-179).  Returns true on
+// the lanes that start a path.
+//
+// A pixel's P.chain samples run one after the other in the lane that took the
+// pixel, because each sample's draws continue the pixel's sampler where the
+// last one left it.  One launch per sample makes every sample wait for the
+// longest path of the one before, and the lanes whose path has ended with it:
+// one launch per frame instead took 2.26 against 3.91 ms for 16 samples of the
+// 256x256 Cornell box, 10.7 against 13.8 ms for 2 of the 720p volume, 1.56
+// against 2.11 ms for 2 of a textured 853x479 field and 8.37 against 9.27 ms for
+// 2 of 32 views (3.3 M pixels) of the icosphere field.
+template <bool MEDIA, bool VIEWS>
+KRR_DEV bool fetchPath(const WfParams &P, const ViewsDev &V, const PixelStateDev &px, const RayQueueDev &q, const CameraDev &cam, int camFetch,
+					   int startDepth, int count, int *work, bool &active, bool &exhausted, int &left, RayItem &r, PathRegs &pr) {
+	int pix = r.pixel;
+	if (!exhausted) {
+		const bool need = !active && left == 0;
+		const int i		= wavePush(work, need);
+		if (__ballot(need && i >= count)) exhausted = true;
+		if (need && i < count) {
+			if (VIEWS || camFetch) {
+				pix	 = px.order ? px.order[i] : i;
+				pr	 = loadPathRegs(px, pix, MEDIA);
+				left = P.chain;
+			} else {
+				r	   = loadRayItem(q, (px.order && startDepth == 0) ? px.order[i] : i);
+				pr	   = loadPathRegs(px, r.pixel, MEDIA);
+				active = true;
+				return true;
+			}
+		}
+	}
+	if (active || left == 0) return false;
+	left--;
+	if (!P.legacySpp) pr.L = f3();
+	Pcg s{pr.rng, P.inc};
+	if (VIEWS) {
+		const int v		  = findView(V, pix);
+		const int local	  = pix - V.start[v];
+		const ViewDev &vw = V.view[v];
+		r				  = cameraRay(vw.cam, vw.W, vw.H, local % vw.W, local / vw.W, s);
+	} else r = cameraRay(cam, P.W, P.H, pix % P.W, pix / P.W, s);
+	r.pixel = pix;
+	pr.rng	= s.state;
+	active	= true;
+	return true;
+}
+
+// End of a path of the persistent launch: with samples of the pixel left, the
+// radiance goes to the pixel sum (k_accumulate's addition) and the sampler
+// stays in registers; the last sample leaves both to memory, for k_film or
+// k_accumulate.
+KRR_DEV void endPath(const PixelStateDev &px, int pixel, const PathRegs &pr, int left, int depth) {
+	if (left > 0) {
+		float4 p		= px.pixel[pixel];
+		p.x				= p.x + pr.L.x;
+		p.y				= p.y + pr.L.y;
+		p.z				= p.z + pr.L.z;
+		px.pixel[pixel] = p;
+		return;
+	}
+	storePathRegs(px, pixel, pr);
+	if (px.plen) px.plen[pixel] = (uint8_t) min(depth, 255);
+}
+
 // Tail of the sample: every path left in the queue after the wavefront depths
 // runs to completion in one thread - closest trace, shade, shadow trace,
 // next depth - in the same per-path stage order as the wavefront, so the
@@ -1020,31 +1078,14 @@ __global__ void k_megakernel(WfParams P0, DevScene sc, TraceBvh bvh, RayQueueDev
 	const int count = (VIEWS || camFetch) ? P.N : *countPtr;
 	uint32_t nv = 0, nt = 0, snv = 0, snt = 0, nClosest = 0, nShadow = 0;
 	bool active = false, exhausted = false, trainPath = false;
-	int depth	= startDepth;
+	int depth = startDepth, left = 0;
 	RayItem r;
-	PathRegs pr; // the path's pixel state, in registers until the path ends
+	r.pixel = 0;
+	PathRegs pr; // the path's pixel state, in registers until the pixel's last path of this launch ends
 	while (true) {
-		if (!exhausted) {
-			const int i = wavePush(&cnt->work[2], !active);
-			if (__ballot(!active && i >= count)) exhausted = true;
-			if (!active && i < count) {
-				if (VIEWS) r = viewCameraRay(P, V, px, px.order ? px.order[i] : i, pr, MEDIA);
-				else if (camFetch) {
-					const int pix = px.order ? px.order[i] : i;
-					pr			  = loadPathRegs(px, pix, MEDIA);
-					if (!P.legacySpp) pr.L = f3();
-					Pcg cs{pr.rng, P.inc};
-					r		= cameraRay(cam, P.W, P.H, pix % P.W, pix / P.W, cs);
-					r.pixel = pix;
-					pr.rng	= cs.state;
-				} else {
-					r  = loadRayItem(q, (px.order && startDepth == 0) ? px.order[i] : i);
-					pr = loadPathRegs(px, r.pixel, MEDIA);
-				}
-				depth	  = startDepth;
-				active	  = true;
-				trainPath = NRC && trainHash((uint32_t) r.pixel) % (uint32_t) nrc.trainMod == (uint32_t) nrc.phase;
-			}
+		if (fetchPath<MEDIA, VIEWS>(P, V, px, q, cam, camFetch, startDepth, count, &cnt->work[2], active, exhausted, left, r, pr)) {
+			depth	  = startDepth;
+			trainPath = NRC && trainHash((uint32_t) r.pixel) % (uint32_t) nrc.trainMod == (uint32_t) nrc.phase;
 		}
 		if (__ballot(active) == 0) break;
 		if (!active) continue;
@@ -1070,8 +1111,7 @@ __global__ void k_megakernel(WfParams P0, DevScene sc, TraceBvh bvh, RayQueueDev
 			r = nx;
 			depth++;
 		} else {
-			storePathRegs(px, r.pixel, pr);
-			if (px.plen) px.plen[r.pixel] = (uint8_t) min(depth, 255);
+			endPath(px, r.pixel, pr, left, depth);
 			active = false;
 		}
 	}
@@ -1128,44 +1168,31 @@ k_megakernel_refill(WfParams P0, DevScene sc, TraceBvh bvh, RayQueueDev q, const
 	uint32_t nv = 0, nt = 0, nClosest = 0, nShadow = 0;
 	bool active = false, exhausted = false, trainPath = false;
 	bool going = false, shadowRay = false, pendingNext = false;
-	int depth = startDepth, trainSlot = -1;
+	int depth = startDepth, trainSlot = -1, left = 0;
 	RayItem r; // the path's current vertex ray; while its shadow ray is in flight, the next one
+	r.pixel = 0;
 	PathRegs pr;
 	f3 to, td;	 // the ray in flight
 	f3 contrib;	 // the shadow ray's radiance when unoccluded
 	TravState ts;
 	while (true) {
-		if (!exhausted) {
-			const int i = wavePush(&cnt->work[2], !active);
-			if (__ballot(!active && i >= count)) exhausted = true;
-			if (!active && i < count) {
-				if (VIEWS) r = viewCameraRay(P, V, px, px.order ? px.order[i] : i, pr, false);
-				else if (camFetch) {
-					const int pix = px.order ? px.order[i] : i;
-					pr			  = loadPathRegs(px, pix, false);
-					if (!P.legacySpp) pr.L = f3();
-					Pcg cs{pr.rng, P.inc};
-					r		= cameraRay(cam, P.W, P.H, pix % P.W, pix / P.W, cs);
-					r.pixel = pix;
-					pr.rng	= cs.state;
-				} else {
-					r  = loadRayItem(q, (px.order && startDepth == 0) ? px.order[i] : i);
-					pr = loadPathRegs(px, r.pixel, false);
-				}
-				depth	  = startDepth;
-				active	  = true;
-				trainPath = NRC && trainHash((uint32_t) r.pixel) % (uint32_t) nrc.trainMod == (uint32_t) nrc.phase;
-				to		  = r.o;
-				td		  = r.d;
-				shadowRay = false;
-				going	  = true;
-				travInit(ts, bvh, __builtin_inff());
-				nClosest++;
-			}
+		if (fetchPath<false, VIEWS>(P, V, px, q, cam, camFetch, startDepth, count, &cnt->work[2], active, exhausted, left, r, pr)) {
+			depth	  = startDepth;
+			trainPath = NRC && trainHash((uint32_t) r.pixel) % (uint32_t) nrc.trainMod == (uint32_t) nrc.phase;
+			to		  = r.o;
+			td		  = r.d;
+			shadowRay = false;
+			going	  = true;
+			travInit(ts, bvh, __builtin_inff());
+			nClosest++;
 		}
-		if (__ballot(active) == 0) break;
-		traverseSteps<COUNT, !PLAIN>(bvh, to, td, shadowRay, going, ts, stack, exhausted ? 1 : P.refillLanes, nv, nt, nodeLds, P.ldsNodes,
-									 P.leafShare);
+		const int nActive = __popcll(__ballot(active));
+		if (nActive == 0) break;
+		// every active lane has a ray in flight here, and the threshold is at
+		// most their number: each round finishes at least one ray
+		const bool drain   = exhausted && __ballot(left > 0) == 0;
+		const int minLanes = drain ? 1 : max(1, (nActive * P.refillLanes) >> 6);
+		traverseSteps<COUNT, !PLAIN>(bvh, to, td, shadowRay, going, ts, stack, minLanes, nv, nt, nodeLds, P.ldsNodes, P.leafShare);
 		if (!active || going) continue;
 		bool next = false; // go on with the path's next closest ray
 		if (shadowRay) {
@@ -1205,8 +1232,7 @@ k_megakernel_refill(WfParams P0, DevScene sc, TraceBvh bvh, RayQueueDev q, const
 			travInit(ts, bvh, __builtin_inff());
 			nClosest++;
 		} else {
-			storePathRegs(px, r.pixel, pr);
-			if (px.plen) px.plen[r.pixel] = (uint8_t) min(depth, 255);
+			endPath(px, r.pixel, pr, left, depth);
 			active = false;
 		}
 	}
@@ -1613,6 +1639,23 @@ template <class K> int persistentGrid(K kernel, int block, size_t lds, int maxBl
 size_t stackLds(const AccelData &a, int block) { return (size_t) (a.ldsEntries() + kStackPad) * block * sizeof(int); }
 size_t stackOverflowInts(const AccelData &a) { return (size_t) (a.stackSize - a.ldsEntries()); }
 
+// Launch of a persistent path kernel over `paths` pixels: the resident blocks,
+// or as many as the paths fill.
+struct PathGrid {
+	int blocks = 1;
+	// The order the paths are taken up in (k_tile_keys) counts only when some
+	// wait for a lane; when every path starts at once, its six launches (25 us)
+	// are left out: 742 against 753 us for a 64x64 frame of 4 samples.
+	bool ordered = true;
+};
+
+PathGrid pathGrid(int resident, int tb, int64_t paths) {
+	PathGrid g;
+	g.blocks  = (int) std::max<int64_t>(1, std::min<int64_t>(resident, (paths + tb - 1) / tb));
+	g.ordered = paths > (int64_t) tb * g.blocks;
+	return g;
+}
+
 // A fraction of a persistent grid (at least one block).
 int scaledGrid(int g, float frac) { return std::max(1, (int) std::lround((double) g * (double) frac)); }
 
@@ -1691,7 +1734,7 @@ struct krr_wf {
 	std::string nrcConfig; // JSON for krr_nrc_create
 	krr_nrc *nrc = nullptr;
 	DevBuf nrcQuery, nrcTrainBuf, nrcBatchV, nrcBatchT;
-	int gMegaNrc = 1;
+	PathGrid gMegaNrc;
 	// persistent launches: fraction of the resident blocks launched
 	float occupancy = 1.f;
 	// multi-view frame (krr_wf_set_views / krr_wf_render_views): pixel state
@@ -1701,7 +1744,7 @@ struct krr_wf {
 	uint64_t viewsVersion = 0, sceneVersion = 0;
 	DevBuf viewBuf, viewStart, frameBuf, vL, vPixel, vRng, vChannel, vNrcQuery;
 	uint64_t viewsGridKey = ~0ull;
-	int gMegaViews = 1;
+	PathGrid gMegaViews;
 	// the multi-view frame is recorded once into a graph and replayed
 	bool useGraph = true;
 	hipStream_t capStream = nullptr;
@@ -1734,7 +1777,8 @@ struct krr_wf {
 	krr_camera cam{};
 	uint64_t frameIndex = 0;
 	uint64_t gridKey	= ~0ull;
-	int gClosest = 1, gShadow = 1, gShade = 1, gMega = 1;
+	int gClosest = 1, gShadow = 1, gShade = 1;
+	PathGrid gMega;
 	bool beginPending	= false;
 	hipStream_t lastStream = nullptr;
 	krr_stats stats{};
@@ -2142,13 +2186,13 @@ WfParams frameParams(const krr_wf *wf, int W, int H, int N, uint64_t frameIndex)
 	P.refillLanes  = refillLanesOf(wf);
 	P.ldsNodes	   = ldsNodeCount(wf);
 	P.leafShare	   = wf->leafShare;
+	P.chain		   = 1;
 	return P;
 }
 
 CameraDev cameraDev(const krr_camera &c) {
 	CameraDev cam;
-	cam.filmH		  = c.film_size[1];
-	cam.focalLength	  = c.focal_length;
+	cam.tanFov		  = detmath::tanf(detmath::atan2f(c.film_size[1] * 0.5f, c.focal_length));
 	cam.focalDistance = c.focal_distance;
 	cam.lensRadius	  = c.lens_radius;
 	cam.aspect		  = c.aspect_ratio;
@@ -2509,7 +2553,7 @@ int krr_wf_render(krr_wf *wf, float *film_dev, void *hip_stream) {
 	hipStream_t st = (hipStream_t) hip_stream;
 	wf->lastStream = st;
 	const int N		   = wf->W * wf->H;
-	const WfParams P   = frameParams(wf, wf->W, wf->H, N, wf->frameIndex);
+	WfParams P		   = frameParams(wf, wf->W, wf->H, N, wf->frameIndex);
 	const CameraDev cam = cameraDev(wf->cam);
 
 	PixelStateDev px{wf->L.as<float4>(), wf->pixel.as<float4>(), wf->rng.as<uint64_t>(), wf->channel.as<int>(), wf->order.as<int>(),
@@ -2539,12 +2583,13 @@ int krr_wf_render(krr_wf *wf, float *film_dev, void *hip_stream) {
 		else wf->gShadow = count ? persistentGrid(k_trace_shadow<true>, tb, lds, gTmax) : persistentGrid(k_trace_shadow<false>, tb, lds, gTmax);
 		wf->gShade = media ? persistentGrid(k_shade<true>, bs, 0, (int) gN) : persistentGrid(k_shade<false>, bs, 0, (int) gN);
 		const size_t nodeBytes = (size_t) ldsNodeCount(wf) * sizeof(Bvh4Node);
-		wf->gMega = withMega<false>(media, count, false, plain, refill, [&](auto k) { return decltype(k)::grid(tb, lds, gTmax, nodeBytes); });
-		if (wf->nrcOn)
-			wf->gMegaNrc = withMega<false>(media, count, true, plain, refill, [&](auto k) { return decltype(k)::grid(tb, lds, gTmax, nodeBytes); });
-		wf->gMega	 = scaledGrid(wf->gMega, wf->occupancy);
-		wf->gMegaNrc = scaledGrid(wf->gMegaNrc, wf->occupancy);
-		const int gMax = std::max(std::max(std::max(wf->gClosest, wf->gShadow), wf->gMega), wf->nrcOn ? wf->gMegaNrc : 0);
+		auto mega = [&](bool nrc) {
+			const int resident = withMega<false>(media, count, nrc, plain, refill, [&](auto k) { return decltype(k)::grid(tb, lds, 1 << 20, nodeBytes); });
+			return pathGrid(scaledGrid(resident, wf->occupancy), tb, N);
+		};
+		wf->gMega = mega(false);
+		if (wf->nrcOn) wf->gMegaNrc = mega(true);
+		const int gMax = std::max(std::max(std::max(wf->gClosest, wf->gShadow), wf->gMega.blocks), wf->nrcOn ? wf->gMegaNrc.blocks : 0);
 		if (int rc = reserveOverflow(wf->ovf, wf->accel, (size_t) gMax * tb)) return rc;
 		wf->gridKey = shapeKey;
 	}
@@ -2587,7 +2632,12 @@ int krr_wf_render(krr_wf *wf, float *film_dev, void *hip_stream) {
 		nrc.trainMod   = wf->nrcTrainMod;
 		nrc.phase	   = (int) (wf->frameIndex % (uint64_t) wf->nrcTrainMod);
 	}
-	for (int s = 0; s < wf->spp; s++) {
+	// With every depth in the persistent launch, one launch runs all samples of
+	// the frame; the radiance cache answers its queries between samples.
+	const PathGrid &pg = wf->nrcOn ? wf->gMegaNrc : wf->gMega;
+	if (wf->wavefrontDepths == 0 && !wf->nrcOn) P.chain = wf->spp;
+	if (!pg.ordered) px.order = nullptr;
+	for (int s = 0; s < wf->spp; s += P.chain) {
 		// with every depth in the persistent launch, it makes the camera rays itself
 		if (wf->wavefrontDepths > 0) hipLaunchKernelGGL(k_camera, dim3(gN), dim3(bs), 0, st, P, cam, px, rayQueue(wf, 0), cnt);
 		for (int depth = 0; depth <= wf->maxDepth; depth++) {
@@ -2595,7 +2645,7 @@ int krr_wf_render(krr_wf *wf, float *film_dev, void *hip_stream) {
 			const RayQueueDev cq = rayQueue(wf, cur);
 			if (depth >= wf->wavefrontDepths) { // the rest of every path in one launch
 				hipLaunchKernelGGL(k_mega_begin, dim3(1), dim3(1), 0, st, cnt);
-				if (depth == 0) { // camera paths: the order from the last sample's path lengths
+				if (depth == 0 && pg.ordered) { // camera paths: the order from the last sample's path lengths
 					const int tilesX = (wf->W + 7) / 8, nTiles = tilesX * ((wf->H + 7) / 8), nBlk = (nTiles + kTileBlock - 1) / kTileBlock;
 					uint8_t *key = wf->tileKey.as<uint8_t>();
 					int *tc = wf->tileCnt.as<int>(), *hist = wf->tileHist.as<int>(), *sorted = wf->tileSorted.as<int>(), *off = wf->tileOff.as<int>();
@@ -2607,11 +2657,10 @@ int krr_wf_render(krr_wf *wf, float *film_dev, void *hip_stream) {
 					hipLaunchKernelGGL(k_tile_pixels, dim3(nTiles), dim3(64), 0, st, sorted, off, wf->W, wf->H, tilesX, wf->order.as<int>());
 				}
 				timed(4, [&] {
-					const unsigned g = (unsigned) wf->gMega;
 					const int camFetch = depth == 0 ? 1 : 0; // k_camera skipped: the kernel makes the camera rays
 					const int *cp	 = (const int *) &cnt->rayCount[cur];
 					withMega<false>(media, count, wf->nrcOn, plain, refill, [&](auto k) {
-						decltype(k)::launch(wf->nrcOn ? (unsigned) wf->gMegaNrc : g, tb, lds, st, P, wf->ds, bvh, cq, cp, px, ovf, cnt,
+						decltype(k)::launch((unsigned) pg.blocks, tb, lds, st, P, wf->ds, bvh, cq, cp, px, ovf, cnt,
 											wf->nrcOn ? nrc : NrcDev{}, ViewsDev{}, depth, cam, camFetch);
 						return 0;
 					});
@@ -2657,7 +2706,7 @@ int krr_wf_render(krr_wf *wf, float *film_dev, void *hip_stream) {
 			if (nrcRc) return nrcRc;
 		}
 		// the last sample is added to the pixel sums by the film write
-		if (s + 1 < wf->spp) hipLaunchKernelGGL(k_accumulate, dim3(gN), dim3(bs), 0, st, N, px);
+		if (s + P.chain < wf->spp) hipLaunchKernelGGL(k_accumulate, dim3(gN), dim3(bs), 0, st, N, px);
 	}
 	if (wf->nrcOn) { // one training step per frame on the recorded vertices
 		timed(5, [&] { nrcRc = nrcTrainDevice(wf->nrc, wf->nrcBatchV.as<float>(), wf->nrcBatchT.as<float>(), &cnt->nrcTrainDone, wf->nrcBatch, wf->nrcSteps, st);
@@ -2692,7 +2741,7 @@ PixelStateDev viewsPx(krr_wf *wf) {
 struct ViewsLaunch {
 	TraceBvh bvh;
 	size_t lds;
-	unsigned grid;
+	PathGrid grid;
 	bool media, count, nrc;
 };
 
@@ -2708,15 +2757,14 @@ int viewsLaunch(krr_wf *wf, int N, bool nrc, ViewsLaunch &L) {
 						 ((uint64_t) wf->stackLdsEntries << 43) ^ (L.count ? 2 : 0) ^ (L.media ? 1 : 0) ^ (nrc ? 4 : 0) ^ (wf->sceneTextured ? 0 : 8) ^
 						 (refillLanesOf(wf) > 0 ? 16 : 0) ^ ((uint64_t) ldsNodeCount(wf) << 5) ^ ((uint64_t) (wf->occupancy * 1024.f) << 32);
 	if (key != wf->viewsGridKey) {
-		const int maxBlocks = std::max(1, (N + tb - 1) / tb);
 		const size_t nodeBytes = (size_t) ldsNodeCount(wf) * sizeof(Bvh4Node);
-		const int g = withMega<true>(L.media, L.count, nrc, !wf->sceneTextured, refillLanesOf(wf) > 0,
-									 [&](auto k) { return decltype(k)::grid(tb, L.lds, maxBlocks, nodeBytes); });
-		wf->gMegaViews		= scaledGrid(g, wf->occupancy);
-		if (int rc = reserveOverflow(wf->ovf, wf->accel, (size_t) wf->gMegaViews * tb)) return rc;
+		const int resident = withMega<true>(L.media, L.count, nrc, !wf->sceneTextured, refillLanesOf(wf) > 0,
+											[&](auto k) { return decltype(k)::grid(tb, L.lds, 1 << 20, nodeBytes); });
+		wf->gMegaViews = pathGrid(scaledGrid(resident, wf->occupancy), tb, N);
+		if (int rc = reserveOverflow(wf->ovf, wf->accel, (size_t) wf->gMegaViews.blocks * tb)) return rc;
 		wf->viewsGridKey = key;
 	}
-	L.grid = (unsigned) wf->gMegaViews;
+	L.grid = wf->gMegaViews;
 	return KRR_OK;
 }
 
@@ -2725,9 +2773,9 @@ int viewsLaunch(krr_wf *wf, int N, bool nrc, ViewsLaunch &L) {
 // views' pixels (plus the cache queries), accumulate, the cache's training,
 // the film write of every view.  `trial` stops after the first persistent
 // launch and writes no film (autotuner).
-int enqueueViews(krr_wf *wf, const WfParams &P, const ViewsLaunch &L, hipStream_t st, bool timing, bool trial) {
-	const ViewsDev V	   = viewsDev(wf);
-	const PixelStateDev px = viewsPx(wf);
+int enqueueViews(krr_wf *wf, WfParams P, const ViewsLaunch &L, hipStream_t st, bool timing, bool trial) {
+	const ViewsDev V = viewsDev(wf);
+	PixelStateDev px = viewsPx(wf);
 	Counters *cnt		   = wf->counters.as<Counters>();
 	const int tb		   = wf->traceBlockSize;
 	const unsigned gN	   = (unsigned) ((P.N + wf->blockSize - 1) / wf->blockSize);
@@ -2758,9 +2806,11 @@ int enqueueViews(krr_wf *wf, const WfParams &P, const ViewsLaunch &L, hipStream_
 	if (L.nrc) hipLaunchKernelGGL(k_nrc_begin, dim3(1), dim3(1), 0, st, cnt, wf->nrcBatch);
 	hipLaunchKernelGGL(k_begin_views, dim3(gN), dim3(wf->blockSize), 0, st, P, V, px);
 	int rc = KRR_OK;
-	for (int s = 0; s < wf->spp; s++) {
+	if (!L.nrc) P.chain = wf->spp; // as in krr_wf_render
+	if (!L.grid.ordered) px.order = nullptr;
+	for (int s = 0; s < wf->spp; s += P.chain) {
 		hipLaunchKernelGGL(k_mega_begin, dim3(1), dim3(1), 0, st, cnt);
-		{ // the order of this sample's camera paths, from the last sample's path lengths (k_tile_keys)
+		if (L.grid.ordered) { // the order of this sample's camera paths, from the last sample's path lengths (k_tile_keys)
 			const int nT = wf->vTiles, nBlk = (nT + kTileBlock - 1) / kTileBlock;
 			uint8_t *key = wf->vTileKey.as<uint8_t>();
 			int *tc = wf->vTileCnt.as<int>(), *hist = wf->vTileHist.as<int>(), *sorted = wf->vTileSorted.as<int>(), *off = wf->vTileOff.as<int>();
@@ -2773,7 +2823,7 @@ int enqueueViews(krr_wf *wf, const WfParams &P, const ViewsLaunch &L, hipStream_
 		}
 		timed(4, [&] {
 			withMega<true>(L.media, L.count, L.nrc, !wf->sceneTextured, refillLanesOf(wf) > 0, [&](auto k) {
-				decltype(k)::launch(L.grid, tb, L.lds, st, P, wf->ds, L.bvh, RayQueueDev{}, nullptr, px, ovf, cnt, nrc, V);
+				decltype(k)::launch((unsigned) L.grid.blocks, tb, L.lds, st, P, wf->ds, L.bvh, RayQueueDev{}, nullptr, px, ovf, cnt, nrc, V);
 				return 0;
 			});
 		});
@@ -2787,7 +2837,8 @@ int enqueueViews(krr_wf *wf, const WfParams &P, const ViewsLaunch &L, hipStream_
 			});
 			if (rc) return rc;
 		}
-		hipLaunchKernelGGL(k_accumulate, dim3(gN), dim3(wf->blockSize), 0, st, P.N, px);
+		// the last sample is added to the pixel sums by the film write
+		if (s + P.chain < wf->spp) hipLaunchKernelGGL(k_accumulate, dim3(gN), dim3(wf->blockSize), 0, st, P.N, px);
 	}
 	if (L.nrc) {
 		timed(5, [&] { rc = nrcTrainDevice(wf->nrc, wf->nrcBatchV.as<float>(), wf->nrcBatchT.as<float>(), &cnt->nrcTrainDone, wf->nrcBatch, wf->nrcSteps, st); });
@@ -2979,7 +3030,7 @@ int krr_wf_autotune(krr_wf *wf, int64_t trial_paths, char *report, int32_t cap, 
 				hipLaunchKernelGGL(k_mega_begin, dim3(1), dim3(1), 0, st, wf->counters.as<Counters>());
 				KRR_HIP(hipEventRecord(e0, st));
 				withMega<true>(L.media, false, false, !wf->sceneTextured, refillLanesOf(wf) > 0, [&](auto k) {
-					decltype(k)::launch(L.grid, wf->traceBlockSize, L.lds, st, P, wf->ds, L.bvh, RayQueueDev{}, nullptr, tpx,
+					decltype(k)::launch((unsigned) L.grid.blocks, wf->traceBlockSize, L.lds, st, P, wf->ds, L.bvh, RayQueueDev{}, nullptr, tpx,
 										wf->ovf.as<int>(), wf->counters.as<Counters>(), NrcDev{}, viewsDev(wf));
 					return 0;
 				});

@@ -1,0 +1,39 @@
+"""A pixel's samples in one persistent launch.
+
+With every depth in the persistent launch (wavefront_depths 0) a lane runs
+all samples of the pixel it takes up, one after the other; with
+wavefront_depths 1 each sample is a launch of its own.  Both keep the order
+of the draws and of the radiance additions, so the films must be equal bit
+for bit, for frames smaller and larger than the launch's lanes, with and
+without ray refill, in media, and with the reference's running sum.
+"""
+import numpy as np
+import pytest
+
+from conftest import CORNELL, icosphere_scene
+from test_gpu_render import gpu_render
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("w,h,spp,more", [
+    (1, 1, 5, {}), (7, 3, 2, {}), (65, 1, 3, {"refill_lanes": 64}), (129, 67, 3, {"legacy_spp_accumulate": True}),
+    (129, 67, 4, {"refill_lanes": 8, "trace_block_size": 64, "occupancy": 0.01}), (1033, 517, 2, {"refill_lanes": 16}), (1033, 517, 2, {})])
+def test_chained_samples_equal_launches_per_sample(krr, gpu, w, h, spp, more):
+    print(f"case: cornell {w}x{h} {spp} spp {more}", flush=True)
+    s = krr.Scene(CORNELL)
+    params = dict({"spp": spp, "max_depth": 6}, **more)
+    a, sa = gpu_render(krr, gpu, s, w, h, params, frame_index=3, frames=2)
+    b, sb = gpu_render(krr, gpu, s, w, h, dict(params, wavefront_depths=1), frame_index=3, frames=2)
+    assert sa["closest_rays"] == sb["closest_rays"] and sa["shadow_rays"] == sb["shadow_rays"]
+    assert np.array_equal(a, b)
+
+
+def test_chained_samples_in_media(krr, gpu):
+    print("case: icosphere field in a grid medium, 97x51, 3 spp", flush=True)
+    s = krr.Scene(icosphere_scene(count=64, level=2, res=(97, 51), media=True, grid_res=48))
+    params = {"spp": 3, "max_depth": 12, "rr_min_depth": 3}
+    a, sa = gpu_render(krr, gpu, s, 97, 51, params)
+    b, sb = gpu_render(krr, gpu, s, 97, 51, dict(params, wavefront_depths=1))
+    assert sa["closest_rays"] == sb["closest_rays"] and sa["shadow_rays"] == sb["shadow_rays"]
+    assert np.array_equal(a, b)
