@@ -123,6 +123,7 @@ struct WfParams {
 	int refillLanes;	  // persistent launch without media: end a traversal round below this many traversing lanes (1..64)
 	int ldsNodes;		  // refill launch: tree nodes 0..ldsNodes-1 are read from a per-block copy in LDS
 	int chain;			  // persistent launch: samples of a pixel run one after the other by the lane that takes it up
+	int fetchLanes;		  // persistent launch: lanes of a wave that take up paths (64, fewer when the paths are few)
 	int leafShare;		  // refill launch: leaf-only iterations once this percent of traversing lanes hold a leaf (0: off)
 };
 

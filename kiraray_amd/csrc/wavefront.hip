@@ -998,7 +998,7 @@ KRR_DEV bool fetchPath(const WfParams &P, const ViewsDev &V, const PixelStateDev
 					   int startDepth, int count, int *work, bool &active, bool &exhausted, int &left, RayItem &r, PathRegs &pr) {
 	int pix = r.pixel;
 	if (!exhausted) {
-		const bool need = !active && left == 0;
+		const bool need = !active && left == 0 && laneId() < P.fetchLanes;
 		const int i		= wavePush(work, need);
 		if (__ballot(need && i >= count)) exhausted = true;
 		if (need && i < count) {
@@ -1640,19 +1640,33 @@ size_t stackLds(const AccelData &a, int block) { return (size_t) (a.ldsEntries()
 size_t stackOverflowInts(const AccelData &a) { return (size_t) (a.stackSize - a.ldsEntries()); }
 
 // Launch of a persistent path kernel over `paths` pixels: the resident blocks,
-// or as many as the paths fill.
+// or as many as the paths fill, and the lanes of each wave that take up paths.
+//
+// A frame with fewer paths than lanes leaves most of the chip idle when its
+// paths fill waves of 64, and each wave runs every stage for as long as its
+// slowest lane.  Spread over more waves, a path waits for fewer others: the
+// fewest lanes per wave, a power of two, that still hold every path at once in
+// the resident waves, or in half of them for small trees whose nodes sit in the
+// L1 (two waves then share a SIMD that four would crowd).  us per frame with 64
+// lanes / all resident waves / half of them: Cornell 64x64 704 / 445 / 420,
+// 256x256 2208 / 2332 / 2055; 1.31 M-triangle field 64x48 1069 / 526 / 559,
+// 160x90 1902 / 1417 / 1613, 320x180 1256 / 1141 / 1261; grid medium 240x135
+// 7119 / 4743 / 5622.
 struct PathGrid {
-	int blocks = 1;
+	int blocks = 1, lanes = 64;
 	// The order the paths are taken up in (k_tile_keys) counts only when some
 	// wait for a lane; when every path starts at once, its six launches (25 us)
 	// are left out: 742 against 753 us for a 64x64 frame of 4 samples.
 	bool ordered = true;
 };
 
-PathGrid pathGrid(int resident, int tb, int64_t paths) {
+PathGrid pathGrid(int resident, int tb, int64_t paths, bool smallTree) {
 	PathGrid g;
-	g.blocks  = (int) std::max<int64_t>(1, std::min<int64_t>(resident, (paths + tb - 1) / tb));
-	g.ordered = paths > (int64_t) tb * g.blocks;
+	const int64_t waves = (int64_t) resident * (tb / 64) / (smallTree ? 2 : 1);
+	while (g.lanes > 1 && waves * (g.lanes / 2) >= paths) g.lanes /= 2;
+	const int64_t perBlock = (int64_t) g.lanes * (tb / 64);
+	g.blocks  = (int) std::max<int64_t>(1, std::min<int64_t>(resident, (paths + perBlock - 1) / perBlock));
+	g.ordered = paths > perBlock * g.blocks;
 	return g;
 }
 
@@ -2187,6 +2201,7 @@ WfParams frameParams(const krr_wf *wf, int W, int H, int N, uint64_t frameIndex)
 	P.ldsNodes	   = ldsNodeCount(wf);
 	P.leafShare	   = wf->leafShare;
 	P.chain		   = 1;
+	P.fetchLanes   = 64;
 	return P;
 }
 
@@ -2585,7 +2600,7 @@ int krr_wf_render(krr_wf *wf, float *film_dev, void *hip_stream) {
 		const size_t nodeBytes = (size_t) ldsNodeCount(wf) * sizeof(Bvh4Node);
 		auto mega = [&](bool nrc) {
 			const int resident = withMega<false>(media, count, nrc, plain, refill, [&](auto k) { return decltype(k)::grid(tb, lds, 1 << 20, nodeBytes); });
-			return pathGrid(scaledGrid(resident, wf->occupancy), tb, N);
+			return pathGrid(scaledGrid(resident, wf->occupancy), tb, N, !media && !refill);
 		};
 		wf->gMega = mega(false);
 		if (wf->nrcOn) wf->gMegaNrc = mega(true);
@@ -2635,7 +2650,10 @@ int krr_wf_render(krr_wf *wf, float *film_dev, void *hip_stream) {
 	// With every depth in the persistent launch, one launch runs all samples of
 	// the frame; the radiance cache answers its queries between samples.
 	const PathGrid &pg = wf->nrcOn ? wf->gMegaNrc : wf->gMega;
-	if (wf->wavefrontDepths == 0 && !wf->nrcOn) P.chain = wf->spp;
+	if (wf->wavefrontDepths == 0) {
+		P.fetchLanes = pg.lanes;
+		if (!wf->nrcOn) P.chain = wf->spp;
+	}
 	if (!pg.ordered) px.order = nullptr;
 	for (int s = 0; s < wf->spp; s += P.chain) {
 		// with every depth in the persistent launch, it makes the camera rays itself
@@ -2760,7 +2778,7 @@ int viewsLaunch(krr_wf *wf, int N, bool nrc, ViewsLaunch &L) {
 		const size_t nodeBytes = (size_t) ldsNodeCount(wf) * sizeof(Bvh4Node);
 		const int resident = withMega<true>(L.media, L.count, nrc, !wf->sceneTextured, refillLanesOf(wf) > 0,
 											[&](auto k) { return decltype(k)::grid(tb, L.lds, 1 << 20, nodeBytes); });
-		wf->gMegaViews = pathGrid(scaledGrid(resident, wf->occupancy), tb, N);
+		wf->gMegaViews = pathGrid(scaledGrid(resident, wf->occupancy), tb, N, !L.media && refillLanesOf(wf) == 0);
 		if (int rc = reserveOverflow(wf->ovf, wf->accel, (size_t) wf->gMegaViews.blocks * tb)) return rc;
 		wf->viewsGridKey = key;
 	}
@@ -2805,7 +2823,8 @@ int enqueueViews(krr_wf *wf, WfParams P, const ViewsLaunch &L, hipStream_t st, b
 	hipLaunchKernelGGL(k_reset_totals, dim3(1), dim3(1), 0, st, cnt);
 	if (L.nrc) hipLaunchKernelGGL(k_nrc_begin, dim3(1), dim3(1), 0, st, cnt, wf->nrcBatch);
 	hipLaunchKernelGGL(k_begin_views, dim3(gN), dim3(wf->blockSize), 0, st, P, V, px);
-	int rc = KRR_OK;
+	int rc		 = KRR_OK;
+	P.fetchLanes = L.grid.lanes;
 	if (!L.nrc) P.chain = wf->spp; // as in krr_wf_render
 	if (!L.grid.ordered) px.order = nullptr;
 	for (int s = 0; s < wf->spp; s += P.chain) {

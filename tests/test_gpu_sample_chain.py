@@ -37,3 +37,18 @@ def test_chained_samples_in_media(krr, gpu):
     b, sb = gpu_render(krr, gpu, s, 97, 51, dict(params, wavefront_depths=1))
     assert sa["closest_rays"] == sb["closest_rays"] and sa["shadow_rays"] == sb["shadow_rays"]
     assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("w,h,spp,more", [(3, 1, 2, {}), (64, 64, 2, {}), (130, 127, 1, {"refill_lanes": 64}), (251, 190, 1, {"refill_lanes": 1}),
+                                          (301, 203, 1, {"refill_lanes": 12, "trace_block_size": 256}), (40, 30, 1, {"nrc": {"train_mod": 4}})])
+def test_few_paths_in_many_waves(krr, gpu, w, h, spp, more):
+    """Frames of fewer paths than the launch has lanes are spread over more
+    waves with fewer lanes each; a launch held to few blocks ("occupancy")
+    fills its waves.  Both trace the same paths."""
+    print(f"case: field {w}x{h} {spp} spp {more}", flush=True)
+    s = krr.Scene(icosphere_scene(count=64, level=2, res=(w, h)))
+    params = dict({"spp": spp, "max_depth": 8, "refill_lanes": 8}, **more)
+    a, sa = gpu_render(krr, gpu, s, w, h, params)
+    b, sb = gpu_render(krr, gpu, s, w, h, dict(params, occupancy=0.01))
+    assert sa["closest_rays"] == sb["closest_rays"] and sa["shadow_rays"] == sb["shadow_rays"]
+    assert np.array_equal(a, b)
