@@ -16,9 +16,8 @@
 //    nodes of a level together: bounds, bins (LDS per block, merged with
 //    integer atomics on order-preserving float encodings), split choice, and
 //    a stable partition (per-block counts, a per-node scan, a scatter);
-//  * every node of at most kSmall references roots a subtree that one wave
-//    builds alone: bins in the wave's LDS, ballots for the stable partition,
-//    a depth-first stack in global memory;
+//  * every node of at most kSmall references roots a subtree that one block
+//    builds alone in LDS, level by level, a node per wave;
 //  * the binary tree is collapsed into 4-wide nodes level by level (open the
 //    child with the largest surface area until four children), nodes of a
 //    level numbered by a prefix sum, children of a node contiguous;
@@ -32,6 +31,7 @@
 #include <cstdint>
 #include <cstring>
 #include <limits>
+#include <type_traits>
 #include <vector>
 
 #include "bvh.h"
@@ -41,7 +41,7 @@ namespace krr {
 namespace bvhdev {
 
 constexpr int NB	   = 16;   // SAH bins per axis (the host builder's default)
-constexpr int kSmall   = 1024; // nodes of at most this many references are built by one wave
+constexpr int kSmall   = 1024; // nodes of at most this many references are built by one block
 constexpr int kChunk   = 2048; // references per block in the level-synchronous phase
 constexpr int kThreads = 256;
 
@@ -431,155 +431,229 @@ __global__ void k_level_nodes(Level L, int nNodes, const int *childBase, Nodes2 
 	else writeNode(N, L.node[t], bb, childBase[t], childBase[t] + 1, 0, 0);
 }
 
-// --------------------------------------------- small subtrees, one per wave
+// -------------------------------------------- small subtrees, one per block
 
 struct SmallTask {
 	int node, first, count, nodeBase; // descendants take nodeBase, nodeBase + 1, ...
 };
 
-// One wave (one 64-thread block) builds the subtree of one task depth first,
-// with the task's references, the partition scratch and the stack of pending
-// right children in LDS.  Per node: one pass bins the references, one pass
-// partitions them (the left count comes from the bins) and accumulates both
-// children's bounds; the left child is processed next with those bounds, a
-// popped right child first recomputes its own.
-__device__ inline void waveBox(Box &b) {
-	for (int a = 0; a < 3; a++) {
-		b.lo[a] = waveMin(b.lo[a]);
-		b.hi[a] = waveMax(b.hi[a]);
+// One block builds the subtree of one task level by level, each wave taking
+// nodes of the level in turn; references (as local indices), primitive boxes
+// and the node lists stay in LDS (44 KB).
+//
+// A subtree of 1,024 triangles has about 1,000 nodes, most of two or three
+// references, and a node's chain of passes is what bounds it: latency, not
+// bandwidth.  So a node's work is spread over the lanes instead of repeated by
+// each: lane (axis, bin) of 48 walks the node's references (broadcast LDS
+// reads) and keeps its own bin's box and count, prefix and suffix boxes over the
+// 16 bins are DPP scans within a row of 16 lanes, and each lane prices the split
+// after its bin.  Minima, maxima and counts are exact in any order and the
+// areas and costs are the host builder's expressions, so the tree is the same.
+// One wave per subtree, with LDS atomics for the bins and every lane going
+// through all 45 splits, took 14.9 ms for the 504 subtrees of 328 K triangles;
+// this takes 1.23 ms, and is bound by vector issue (about 900 instructions a
+// node).
+constexpr int kSmallThreads = 512;
+
+// v combined over 16 lanes (a DPP row) by f, the result in each of them; over
+// the wave when wide.
+template <class F> __device__ inline float rowReduce(float v, F f, bool wide) {
+	auto dpp = [&](auto ctrl) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), ctrl.value, 0xf, 0xf, true)); };
+	v = f(v, dpp(std::integral_constant<int, 0xB1>{}));	 // lanes xor 1 (quad_perm 1 0 3 2)
+	v = f(v, dpp(std::integral_constant<int, 0x4E>{}));	 // lanes xor 2 (quad_perm 2 3 0 1)
+	v = f(v, dpp(std::integral_constant<int, 0x141>{})); // row_half_mirror
+	v = f(v, dpp(std::integral_constant<int, 0x140>{})); // row_mirror
+	if (wide) {
+		v = f(v, __shfl_xor(v, 16));
+		v = f(v, __shfl_xor(v, 32));
 	}
+	return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
 }
 
-__global__ void __launch_bounds__(64) k_small(const SmallTask *tasks, int nTasks, Prims P, int *refs, Nodes2 N, float nodeCost, int maxLeaf) {
-	__shared__ int sRef[kSmall], sTmp[kSmall];
-	__shared__ int2 sStack[kSmall]; // {node, first << 11 | count}, first relative to the task
-	__shared__ Bins B;
-	const int ti = blockIdx.x, lane = threadIdx.x;
+// Inclusive scan over the 16 lanes of a row, from lane 0 up (CTRL0 0x110,
+// row_shr) or from lane 15 down (0x100, row_shl); lanes without a source take
+// the identity.
+template <int CTRL0, class F> __device__ inline int rowScan(int v, int identity, F f) {
+	v = f(v, __builtin_amdgcn_update_dpp(identity, v, CTRL0 + 1, 0xf, 0xf, false));
+	v = f(v, __builtin_amdgcn_update_dpp(identity, v, CTRL0 + 2, 0xf, 0xf, false));
+	v = f(v, __builtin_amdgcn_update_dpp(identity, v, CTRL0 + 4, 0xf, 0xf, false));
+	v = f(v, __builtin_amdgcn_update_dpp(identity, v, CTRL0 + 8, 0xf, 0xf, false));
+	return v;
+}
+template <int CTRL0> __device__ inline Box rowScanBox(Box b) {
+	auto lo = [](int x, int y) { return __float_as_int(fminf(__int_as_float(x), __int_as_float(y))); };
+	auto hi = [](int x, int y) { return __float_as_int(fmaxf(__int_as_float(x), __int_as_float(y))); };
+	for (int a = 0; a < 3; a++) {
+		b.lo[a] = __int_as_float(rowScan<CTRL0>(__float_as_int(b.lo[a]), __float_as_int(__builtin_inff()), lo));
+		b.hi[a] = __int_as_float(rowScan<CTRL0>(__float_as_int(b.hi[a]), __float_as_int(-__builtin_inff()), hi));
+	}
+	return b;
+}
+
+__global__ void __launch_bounds__(kSmallThreads) k_small(const SmallTask *tasks, int nTasks, Prims P, int *refs, Nodes2 N, float nodeCost, int maxLeaf) {
+	__shared__ float4 sLo[kSmall], sHi[kSmall]; // boxes of the task's primitives, in the order of the references at the start
+	__shared__ uint16_t sRef[kSmall], sTmp[kSmall];
+	__shared__ int2 sList[2][kSmall / 2]; // nodes of a level with at least two references: {node, first << 11 | count}
+	__shared__ int sCount[2], sNodes;
+	const int ti = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+	constexpr int waves = kSmallThreads / 64;
 	if (ti >= nTasks) return;
 	const SmallTask tk = tasks[ti];
-	for (int i = lane; i < tk.count; i += 64) sRef[i] = refs[tk.first + i];
+	auto sBox = [&](int r) {
+		const float4 l = sLo[r], h = sHi[r];
+		Box b;
+		b.lo[0] = l.x, b.lo[1] = l.y, b.lo[2] = l.z;
+		b.hi[0] = h.x, b.hi[1] = h.y, b.hi[2] = h.z;
+		return b;
+	};
+	for (int i = threadIdx.x; i < tk.count; i += kSmallThreads) {
+		const int r = refs[tk.first + i];
+		float4 l = P.lo[r];
+		l.w	   = __int_as_float(r); // the reference travels with its box
+		sLo[i] = l;
+		sHi[i] = P.hi[r];
+		sRef[i] = (uint16_t) i;
+	}
+	if (threadIdx.x == 0) {
+		sList[0][0] = make_int2(tk.node, tk.count);
+		sCount[0]	= 1;
+		sNodes		= 0;
+	}
 	__syncthreads();
-	int sp = 0, nextNode = tk.nodeBase;
-	int node = tk.node, first = 0, count = tk.count; // first relative to the task
-	bool haveBounds = false;
-	Box bb, cb;
-	while (true) {
-		if (!haveBounds) { // bounds and centroid bounds of the node
+	if (tk.count < 2) { // a single reference is a leaf, as in the loop below
+		if (threadIdx.x == 0 && tk.count == 1) writeNode(N, tk.node, sBox(0), -1, -1, tk.first, 1);
+		return;
+	}
+	const int axis = min(lane >> 4, 2), bin = lane & 15;
+	const bool binLane = lane < 48, ax0 = axis == 0, ax1 = axis == 1;
+	// each level has fewer references per node than the one above, so there are
+	// at most tk.count levels
+	for (int cur = 0;; cur ^= 1) {
+		const int nLevel = sCount[cur];
+		if (nLevel == 0) break;
+		__syncthreads();
+		if (threadIdx.x == 0) sCount[cur ^ 1] = 0;
+		__syncthreads();
+		for (int q = wave; q < nLevel; q += waves) {
+			const int2 e	= sList[cur][q];
+			const int node	= __builtin_amdgcn_readfirstlane(e.x);
+			const int first = __builtin_amdgcn_readfirstlane(e.y) >> 11, count = __builtin_amdgcn_readfirstlane(e.y) & 2047;
+			// bounds and centroid bounds
+			Box bb, cb;
 			bb.reset();
 			cb.reset();
 			for (int i = first + lane; i < first + count; i += 64) {
-				Box pb;
-				float c[3];
-				primBox(P, sRef[i], pb, c);
+				const Box pb = sBox(sRef[i]);
 				bb.grow(pb);
 				for (int a = 0; a < 3; a++) {
-					cb.lo[a] = fminf(cb.lo[a], c[a]);
-					cb.hi[a] = fmaxf(cb.hi[a], c[a]);
+					const float c = 0.5f * (pb.lo[a] + pb.hi[a]);
+					cb.lo[a]	  = fminf(cb.lo[a], c);
+					cb.hi[a]	  = fmaxf(cb.hi[a], c);
 				}
 			}
-			waveBox(bb);
-			waveBox(cb);
-		}
-		int d = 1;
-		Split s{-1, -1, 0.f};
-		float scale[3];
-		if (count > 1) {
-			binsReset(B, lane, 64);
-			__syncthreads();
+			const bool wide = count > 16;
+			auto mn = [](float x, float y) { return fminf(x, y); };
+			auto mx = [](float x, float y) { return fmaxf(x, y); };
 			for (int a = 0; a < 3; a++) {
-				const float ext = cb.hi[a] - cb.lo[a];
-				scale[a]		= ext > 0 ? NB / ext : 0.f;
+				bb.lo[a] = rowReduce(bb.lo[a], mn, wide);
+				bb.hi[a] = rowReduce(bb.hi[a], mx, wide);
+				cb.lo[a] = rowReduce(cb.lo[a], mn, wide);
+				cb.hi[a] = rowReduce(cb.hi[a], mx, wide);
 			}
-			for (int i = first + lane; i < first + count; i += 64) {
-				Box pb;
-				float c[3];
-				primBox(P, sRef[i], pb, c);
-				for (int a = 0; a < 3; a++) {
-					if (!(scale[a] > 0)) continue;
-					const int k = binOf(c[a], cb.lo[a], scale[a]);
-					atomicAdd(&B.cnt[a][k], 1);
-					for (int e = 0; e < 3; e++) {
-						atomicMin(&B.lo[a][k][e], ordF(pb.lo[e]));
-						atomicMax(&B.hi[a][k][e], ordF(pb.hi[e]));
-					}
+			// this lane's bin
+			const float cLo = ax0 ? cb.lo[0] : (ax1 ? cb.lo[1] : cb.lo[2]), cHi = ax0 ? cb.hi[0] : (ax1 ? cb.hi[1] : cb.hi[2]);
+			const float ext = cHi - cLo, scale = ext > 0 ? NB / ext : 0.f;
+			const bool mine = binLane && scale > 0;
+			Box own;
+			own.reset();
+			int cnt = 0;
+#pragma unroll 4
+			for (int i = first; i < first + count; i++) {
+				const int r	   = sRef[i];
+				const float4 l = sLo[r], h = sHi[r];
+				const float c = 0.5f * ((ax0 ? l.x : (ax1 ? l.y : l.z)) + (ax0 ? h.x : (ax1 ? h.y : h.z)));
+				if (mine && binOf(c, cLo, scale) == bin) {
+					own.lo[0] = fminf(own.lo[0], l.x), own.lo[1] = fminf(own.lo[1], l.y), own.lo[2] = fminf(own.lo[2], l.z);
+					own.hi[0] = fmaxf(own.hi[0], h.x), own.hi[1] = fmaxf(own.hi[1], h.y), own.hi[2] = fmaxf(own.hi[2], h.z);
+					cnt++;
 				}
 			}
-			__syncthreads();
-			s = chooseSplit(B, cb, bb.area(), nodeCost); // every lane, same result
-			d = decide(s, count, maxLeaf);
-		}
-		if (d == 1) {
-			if (lane == 0) writeNode(N, node, bb, -1, -1, tk.first + first, count);
-			__syncthreads(); // bins read before the next node resets them
-			if (sp == 0) break;
-			const int2 e = sStack[--sp];
-			node		 = e.x;
-			first		 = e.y >> 11;
-			count		 = e.y & 2047;
-			haveBounds	 = false;
-			continue;
-		}
-		// left count from the bins (binned split) or half (middle split)
-		int nLeft = count / 2;
-		if (d == 0) {
-			nLeft = 0;
-			for (int k = 0; k <= s.bin; k++) nLeft += B.cnt[s.axis][k];
-		}
-		__syncthreads(); // bins read before the next node resets them
-		// stable partition into sTmp, with the left child's bounds
-		Box lb, lc;
-		lb.reset();
-		lc.reset();
-		int nl = 0, nr = 0;
-		for (int base = first; base < first + count; base += 64) {
-			const int i	 = base + lane;
-			const bool v = i < first + count;
-			bool left	 = false;
-			int r		 = 0;
-			Box pb;
-			float c[3];
-			if (v) {
-				r = sRef[i];
-				primBox(P, r, pb, c);
-				left = d == 2 ? i < first + count / 2 : binOf(c[s.axis], cb.lo[s.axis], scale[s.axis]) <= s.bin;
-				if (left) {
-					lb.grow(pb);
-					for (int a = 0; a < 3; a++) {
-						lc.lo[a] = fminf(lc.lo[a], c[a]);
-						lc.hi[a] = fmaxf(lc.hi[a], c[a]);
+			// the split after this bin: prefix up to it, suffix from the next one
+			auto add = [](int x, int y) { return x + y; };
+			const Box pre = rowScanBox<0x110>(own);
+			Box suf		  = rowScanBox<0x100>(own);
+			const int nPre = rowScan<0x110>(cnt, 0, add);
+			int nSuf	   = rowScan<0x100>(cnt, 0, add);
+			// lane k takes the suffix from bin k + 1
+			for (int a = 0; a < 3; a++) {
+				suf.lo[a] = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(suf.lo[a]), 0x101, 0xf, 0xf, true));
+				suf.hi[a] = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(suf.hi[a]), 0x101, 0xf, 0xf, true));
+			}
+			nSuf		 = __builtin_amdgcn_update_dpp(0, nSuf, 0x101, 0xf, 0xf, true);
+			float cost	 = __builtin_inff();
+			const bool ok = mine && bin < NB - 1 && nPre != 0 && nSuf != 0;
+			if (ok) cost = nodeCost + (pre.area() * nPre + suf.area() * nSuf) / fmaxf(bb.area(), 1e-30f);
+			if (!(cost < __builtin_inff())) cost = __builtin_inff(); // not a number: never the minimum
+			// the first minimum in axis-major, bin-minor order
+			const float best = rowReduce(cost, mn, true);
+			Split s{-1, -1, __builtin_inff()};
+			if (best < __builtin_inff()) {
+				const int w = __ffsll((unsigned long long) __ballot(cost == best)) - 1;
+				s			= Split{w >> 4, w & 15, best};
+			}
+			const int d = decide(s, count, maxLeaf);
+			if (d == 1) {
+				if (lane == 0) writeNode(N, node, bb, -1, -1, tk.first + first, count);
+				continue;
+			}
+			// stable partition; the left count from the bins (binned split) or half
+			int nLeft = count / 2;
+			if (d == 0) {
+				nLeft = __builtin_amdgcn_readlane(nPre, s.axis * 16 + s.bin);
+				const float sLoA = s.axis == 0 ? cb.lo[0] : (s.axis == 1 ? cb.lo[1] : cb.lo[2]), sHiA = s.axis == 0 ? cb.hi[0] : (s.axis == 1 ? cb.hi[1] : cb.hi[2]);
+				const float sScale = NB / (sHiA - sLoA);
+				int nl = 0, nr = 0;
+				uint16_t *dst = count <= 64 ? sRef : sTmp; // a node of one pass is read whole before it is written
+				for (int base = first; base < first + count; base += 64) {
+					const int i	 = base + lane;
+					const bool v = i < first + count;
+					int r		 = 0;
+					bool left	 = false;
+					if (v) {
+						r				= sRef[i];
+						const float4 l = sLo[r], h = sHi[r];
+						const float c = 0.5f * (s.axis == 0 ? l.x + h.x : (s.axis == 1 ? l.y + h.y : l.z + h.z));
+						left		  = binOf(c, sLoA, sScale) <= s.bin;
 					}
+					const uint64_t lm = __ballot(v && left), rm = __ballot(v && !left);
+					const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+					const int slot = left ? first + nl + __popcll(lm & below) : first + nLeft + nr + __popcll(rm & below);
+					if (v && slot < first + count) dst[slot] = (uint16_t) r; // always in range: nl ends equal to nLeft
+					nl += __popcll(lm);
+					nr += __popcll(rm);
+				}
+				if (count > 64) {
+					__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+					for (int i = first + lane; i < first + count; i += 64) sRef[i] = sTmp[i];
 				}
 			}
-			const uint64_t lm = __ballot(v && left), rm = __ballot(v && !left);
-			const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-			const int slot = v ? (left ? first + nl + __popcll(lm & below) : first + nLeft + nr + __popcll(rm & below)) : -1;
-			if (slot >= first && slot < first + count) sTmp[slot] = r; // always in range when nl ends equal to nLeft
-			nl += __popcll(lm);
-			nr += __popcll(rm);
+			__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); // other lanes' sRef entries are read from here on
+			// children: two or more references go to the next level's list, a
+			// single one is a leaf.  A side is never empty (binned splits skip
+			// empty sides, middle splits halve at least 9 references).
+			if (lane == 0) {
+				const int l = tk.nodeBase + 2 * atomicAdd(&sNodes, 1);
+				writeNode(N, node, bb, l, l + 1, 0, 0);
+				for (int k = 0; k < 2; k++) {
+					const int f = k ? first + nLeft : first, c = k ? count - nLeft : nLeft;
+					if (c > 1) sList[cur ^ 1][atomicAdd(&sCount[cur ^ 1], 1)] = make_int2(l + k, (f << 11) | c);
+					else writeNode(N, l + k, sBox(sRef[f]), -1, -1, tk.first + f, 1);
+				}
+			}
 		}
 		__syncthreads();
-		for (int i = first + lane; i < first + count; i += 64) sRef[i] = sTmp[i];
-		__syncthreads();
-		// nl == nLeft by construction; a side is never empty (binned splits
-		// skip empty sides, middle splits halve at least 9 references)
-		const int l = nextNode, rgt = nextNode + 1;
-		nextNode += 2;
-		if (lane == 0) {
-			writeNode(N, node, bb, l, rgt, 0, 0);
-			sStack[sp] = make_int2(rgt, ((first + nLeft) << 11) | (count - nLeft));
-		}
-		sp++;
-		__syncthreads();
-		waveBox(lb);
-		waveBox(lc);
-		node	   = l;
-		count	   = nLeft;
-		bb		   = lb;
-		cb		   = lc;
-		haveBounds = true;
 	}
-	__syncthreads();
-	for (int i = lane; i < tk.count; i += 64) refs[tk.first + i] = sRef[i];
+	for (int i = threadIdx.x; i < tk.count; i += kSmallThreads) refs[tk.first + i] = __float_as_int(sLo[sRef[i]].w);
 }
 
 // ------------------------------------------------------------- collapse
@@ -893,7 +967,7 @@ int buildBvh4Device(const float *pos, int64_t nVerts, const int32_t *idx, int64_
 	if (!small.empty()) {
 		Buf bSmall;
 		BVHD_HIP(upload(bSmall, small, st));
-		hipLaunchKernelGGL(k_small, dim3((unsigned) small.size()), dim3(64), 0, st, (const SmallTask *) bSmall.as<SmallTask>(),
+		hipLaunchKernelGGL(k_small, dim3((unsigned) small.size()), dim3(kSmallThreads), 0, st, (const SmallTask *) bSmall.as<SmallTask>(),
 						   (int) small.size(), P, refs.as<int>(), N, cost, maxLeaf);
 		BVHD_HIP(hipGetLastError());
 		BVHD_HIP(hipStreamSynchronize(st));

@@ -134,3 +134,27 @@ def test_render_parity_either_builder(krr, oracle, gpu):
         wf.close()
     assert np.array_equal(imgs[0][0], imgs[1][0])
     assert imgs[0][1:] == imgs[1][1:]
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 8, 9, 16, 17, 64, 65, 127, 1023, 1024, 1025, 2500])
+@pytest.mark.parametrize("kind", ["spread", "grid", "one_point"])
+def test_subtree_sizes(krr, oracle, gpu, n, kind):
+    """Triangle counts around the sizes where a subtree's passes change (one
+    row of lanes, one wave, one block), spread out, with many equal centroids,
+    and all around one point (middle splits): the host's tree, the brute
+    force's hits."""
+    print(f"case: device BVH of {n} triangles, {kind}", flush=True)
+    rng = np.random.default_rng(n)
+    c = rng.random((n, 1, 3)) if kind == "spread" else np.floor(rng.random((n, 1, 3)) * 4) / 4 if kind == "grid" else np.full((n, 1, 3), 0.5)
+    edge = np.array([[0.05, 0.0, 0.0], [-0.025, 0.05, 0.0], [-0.025, -0.05, 0.0]])
+    pos = np.ascontiguousarray((c + edge * (0.5 + rng.random((n, 1, 1)))).reshape(-1, 3), np.float32)
+    idx = np.arange(3 * n, dtype=np.int32).reshape(-1, 3)
+    desc, keep = _soup_desc(krr, pos, idx)
+    rays = _rays_towards_triangles(pos, idx, 2000, rng, np.array([-0.2, -0.2, -1.0]), np.array([1.2, 1.2, 2.0]), jitter=0.02)
+    gd, vd, infod = _gpu_closest(krr, gpu, _Desc(desc), rays, {"builder": "device"})
+    if kind == "spread":  # no equal centroids: the host's unstable order reaches no middle split
+        _, _, infoh = _gpu_closest(krr, gpu, _Desc(desc), rays, {"builder": "host"})
+        assert infod["nodes"] == infoh["nodes"] and infod["max_depth"] == infoh["max_depth"]
+    assert infod["leaf_tris"] == n
+    _assert_same_hits(gd, oracle.trace_closest(desc, rays))
+    assert np.array_equal(vd, oracle.trace_any(desc, rays))
