@@ -14,13 +14,14 @@
 // GPU organisation:
 //  * large nodes (> kSmall references) are processed level by level, all
 //    nodes of a level together: bounds, bins (LDS per block, merged with
-//    integer atomics on order-preserving float encodings), split choice, and
-//    a stable partition (per-block counts, a per-node scan, a scatter);
+//    integer atomics on order-preserving float encodings), split choice, a
+//    stable partition between two reference buffers (per-block counts, a
+//    scatter), and the next level's list made on the device;
 //  * every node of at most kSmall references roots a subtree that one block
 //    builds alone in LDS, level by level, a node per wave;
 //  * the binary tree is collapsed into 4-wide nodes level by level (open the
 //    child with the largest surface area until four children), nodes of a
-//    level numbered by a prefix sum, children of a node contiguous;
+//    level numbered by block sums and a scan, children of a node contiguous;
 //  * leaf triangles are stored in reference order, so a binary leaf
 //    [first, first + count) is directly its triangle range.
 #include <hip/hip_runtime.h>
@@ -103,49 +104,68 @@ struct Split {
 	float cost;
 };
 
-// SAH over the bins exactly as the host builder (bvh.cpp Builder2::build):
-// suffix boxes from the top bin down, prefix boxes from bin 0 up, strict '<'.
-__device__ Split chooseSplit(const Bins &b, const Box &cb, float pA, float nodeCost) {
-	Split s{-1, -1, __builtin_inff()};
-	for (int a = 0; a < 3; a++) {
-		const float ext = cb.hi[a] - cb.lo[a];
-		if (!(ext > 0)) continue;
-		float rightArea[NB];
-		int rightCnt[NB];
-		Box acc;
-		acc.reset();
-		int c = 0;
-		for (int k = NB - 1; k >= 1; k--) {
-			Box bk;
-			for (int e = 0; e < 3; e++) {
-				bk.lo[e] = unordF(b.lo[a][k][e]);
-				bk.hi[e] = unordF(b.hi[a][k][e]);
-			}
-			acc.grow(bk);
-			c += b.cnt[a][k];
-			rightArea[k] = acc.area();
-			rightCnt[k]	 = c;
-		}
-		acc.reset();
-		c = 0;
-		for (int k = 0; k < NB - 1; k++) {
-			Box bk;
-			for (int e = 0; e < 3; e++) {
-				bk.lo[e] = unordF(b.lo[a][k][e]);
-				bk.hi[e] = unordF(b.hi[a][k][e]);
-			}
-			acc.grow(bk);
-			c += b.cnt[a][k];
-			if (c == 0 || rightCnt[k + 1] == 0) continue;
-			const float cost = nodeCost + (acc.area() * c + rightArea[k + 1] * rightCnt[k + 1]) / fmaxf(pA, 1e-30f);
-			if (cost < s.cost) {
-				s.cost = cost;
-				s.axis = a;
-				s.bin  = k;
-			}
-		}
+// v combined over 16 lanes (a DPP row) by f, the result in each of them; over
+// the wave when wide.
+template <class F> __device__ inline float rowReduce(float v, F f, bool wide) {
+	auto dpp = [&](auto ctrl) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), ctrl.value, 0xf, 0xf, true)); };
+	v = f(v, dpp(std::integral_constant<int, 0xB1>{}));	 // lanes xor 1 (quad_perm 1 0 3 2)
+	v = f(v, dpp(std::integral_constant<int, 0x4E>{}));	 // lanes xor 2 (quad_perm 2 3 0 1)
+	v = f(v, dpp(std::integral_constant<int, 0x141>{})); // row_half_mirror
+	v = f(v, dpp(std::integral_constant<int, 0x140>{})); // row_mirror
+	if (wide) {
+		v = f(v, __shfl_xor(v, 16));
+		v = f(v, __shfl_xor(v, 32));
 	}
-	return s;
+	return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
+}
+
+// Inclusive scan over the 16 lanes of a row, from lane 0 up (CTRL0 0x110,
+// row_shr) or from lane 15 down (0x100, row_shl); lanes without a source take
+// the identity.
+template <int CTRL0, class F> __device__ inline int rowScan(int v, int identity, F f) {
+	v = f(v, __builtin_amdgcn_update_dpp(identity, v, CTRL0 + 1, 0xf, 0xf, false));
+	v = f(v, __builtin_amdgcn_update_dpp(identity, v, CTRL0 + 2, 0xf, 0xf, false));
+	v = f(v, __builtin_amdgcn_update_dpp(identity, v, CTRL0 + 4, 0xf, 0xf, false));
+	v = f(v, __builtin_amdgcn_update_dpp(identity, v, CTRL0 + 8, 0xf, 0xf, false));
+	return v;
+}
+template <int CTRL0> __device__ inline Box rowScanBox(Box b) {
+	auto lo = [](int x, int y) { return __float_as_int(fminf(__int_as_float(x), __int_as_float(y))); };
+	auto hi = [](int x, int y) { return __float_as_int(fmaxf(__int_as_float(x), __int_as_float(y))); };
+	for (int a = 0; a < 3; a++) {
+		b.lo[a] = __int_as_float(rowScan<CTRL0>(__float_as_int(b.lo[a]), __float_as_int(__builtin_inff()), lo));
+		b.hi[a] = __int_as_float(rowScan<CTRL0>(__float_as_int(b.hi[a]), __float_as_int(-__builtin_inff()), hi));
+	}
+	return b;
+}
+
+// SAH over a node's bins exactly as the host builder (bvh.cpp
+// Builder2::build), one wave per node: lane 16 a + k of the first 48 holds bin k
+// of axis a (its box and count), prefix and suffix boxes over the 16 bins are
+// DPP scans within a row of 16 lanes, and each lane prices the split after its
+// bin; the first minimum in axis-major, bin-minor order wins.  mine: the lane
+// holds a bin of an axis the centroids extend along.  Minima, maxima and counts
+// are exact in any order.  nPre: references up to the lane's bin.
+__device__ inline Split waveSplit(const Box &own, int cnt, bool mine, float pA, float nodeCost, int &nPre) {
+	const int bin = __lane_id() & 15;
+	auto add	  = [](int x, int y) { return x + y; };
+	const Box pre = rowScanBox<0x110>(own);
+	Box suf		  = rowScanBox<0x100>(own);
+	nPre		  = rowScan<0x110>(cnt, 0, add);
+	int nSuf	  = rowScan<0x100>(cnt, 0, add);
+	// lane k takes the suffix from bin k + 1
+	for (int a = 0; a < 3; a++) {
+		suf.lo[a] = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(suf.lo[a]), 0x101, 0xf, 0xf, true));
+		suf.hi[a] = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(suf.hi[a]), 0x101, 0xf, 0xf, true));
+	}
+	nSuf	   = __builtin_amdgcn_update_dpp(0, nSuf, 0x101, 0xf, 0xf, true);
+	float cost = __builtin_inff();
+	if (mine && bin < NB - 1 && nPre != 0 && nSuf != 0) cost = nodeCost + (pre.area() * nPre + suf.area() * nSuf) / fmaxf(pA, 1e-30f);
+	if (!(cost < __builtin_inff())) cost = __builtin_inff(); // not a number: never the minimum
+	const float best = rowReduce(cost, [](float x, float y) { return fminf(x, y); }, true);
+	if (!(best < __builtin_inff())) return Split{-1, -1, __builtin_inff()};
+	const int w = __ffsll((unsigned long long) __ballot(cost == best)) - 1;
+	return Split{w >> 4, w & 15, best};
 }
 
 // Decision for a node of `count` references: 0 split (binned), 1 leaf,
@@ -210,12 +230,25 @@ struct Level {
 	Bins *bins;
 	int *decision, *axis, *bin; // split per node
 	int *nLeft;					// left references per node
-	const int *blockNode;		// node of each block
-	const int *blockStart;		// first reference of each block
-	int *blockLeft, *blockOff;	// per-block left counts and their exclusive prefix within the node
+	int *blockNode;				// node of each block
+	int *blockStart;			// first reference of each block
+	int *blockLeft;				// per-block left counts
 	const int *blockBegin;		// first block of each node (n + 1 entries)
 };
 
+// One of the two node lists that the levels alternate between.
+struct LevelList {
+	int *first, *count, *node, *blockBegin;
+};
+
+// What the host reads between levels, and the running totals.
+struct LevelCtl {
+	int nodes, blocks;	 // of the next level
+	int small, nextNode; // subtrees handed to k_small, binary nodes numbered so far
+	int bad;			 // a split left a side empty
+};
+
+// Bounds, bins and blocks of each node of the level.
 __global__ void k_level_reset(Level L, int nNodes) {
 	const int t = blockIdx.x;
 	if (t >= nNodes) return;
@@ -225,6 +258,10 @@ __global__ void k_level_reset(Level L, int nNodes) {
 		else L.cbox[6 * t + e - 6] = v;
 	}
 	binsReset(L.bins[t], threadIdx.x, blockDim.x);
+	for (int b = L.blockBegin[t] + (int) threadIdx.x; b < L.blockBegin[t + 1]; b += blockDim.x) {
+		L.blockNode[b]	= t;
+		L.blockStart[b] = L.first[t] + (b - L.blockBegin[t]) * kChunk;
+	}
 }
 
 __device__ inline float waveMin(float v) {
@@ -311,15 +348,33 @@ __global__ void __launch_bounds__(kThreads) k_level_bins(Level L, Prims P, const
 	}
 }
 
-__global__ void k_level_split(Level L, int nNodes, float nodeCost, int maxLeaf) {
-	const int t = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ void __launch_bounds__(64) k_level_split(Level L, int nNodes, float nodeCost, int maxLeaf) {
+	const int t = blockIdx.x, lane = threadIdx.x;
 	if (t >= nNodes) return;
 	const Box bb = loadBox(L.box + 6 * t), cb = loadBox(L.cbox + 6 * t);
-	const Split s = chooseSplit(L.bins[t], cb, bb.area(), nodeCost);
+	const int axis = min(lane >> 4, 2), k = lane & 15;
+	Box own;
+	own.reset();
+	int cnt			= 0;
+	const bool mine = lane < 48 && cb.hi[axis] - cb.lo[axis] > 0;
+	if (mine) {
+		const Bins &b = L.bins[t];
+		cnt			  = b.cnt[axis][k];
+		for (int e = 0; e < 3; e++) {
+			own.lo[e] = unordF(b.lo[axis][k][e]);
+			own.hi[e] = unordF(b.hi[axis][k][e]);
+		}
+	}
+	int nPre;
+	const Split s = waveSplit(own, cnt, mine, bb.area(), nodeCost, nPre);
 	const int d	  = decide(s, L.count[t], maxLeaf);
-	L.decision[t] = d;
-	L.axis[t]	  = s.axis;
-	L.bin[t]	  = s.bin;
+	const int nl  = d == 0 ? __builtin_amdgcn_readlane(nPre, s.axis * 16 + s.bin) : L.count[t] / 2;
+	if (lane == 0) {
+		L.decision[t] = d;
+		L.axis[t]	  = s.axis;
+		L.bin[t]	  = s.bin;
+		L.nLeft[t]	  = nl;
+	}
 }
 
 __device__ inline bool goesLeft(const Level &L, int t, const Box &cb, float scale, int pos, float c) {
@@ -357,24 +412,11 @@ __global__ void __launch_bounds__(kThreads) k_level_count(Level L, Prims P, cons
 	}
 }
 
-// Exclusive prefix of the block counts of each node (blocks of a node are
-// consecutive), and the node's left total.
-__global__ void k_level_scan(Level L, int nNodes) {
-	const int t = blockIdx.x * blockDim.x + threadIdx.x;
-	if (t >= nNodes) return;
-	int s = 0;
-	for (int b = L.blockBegin[t]; b < L.blockBegin[t + 1]; b++) {
-		L.blockOff[b] = s;
-		s += L.blockLeft[b];
-	}
-	L.nLeft[t] = s;
-}
-
 // Stable partition: thread j of the block owns references [8j, 8j + 8) of
 // the block's chunk, in order.
 __global__ void __launch_bounds__(kThreads) k_level_scatter(Level L, Prims P, const int *refs, int *tmp) {
 	constexpr int per = kChunk / kThreads;
-	__shared__ int lefts[kThreads];
+	__shared__ int lefts[kThreads], earlier[kThreads / 64];
 	const int b = blockIdx.x, t = L.blockNode[b];
 	const Box cb	  = loadBox(L.cbox + 6 * t);
 	const float scale = splitScale(L, t, cb);
@@ -396,8 +438,15 @@ __global__ void __launch_bounds__(kThreads) k_level_scatter(Level L, Prims P, co
 			nl += left[k] ? 1 : 0;
 		}
 	}
+	// left references of the node's earlier blocks
+	int before = 0;
+	for (int e = L.blockBegin[t] + (int) threadIdx.x; e < b; e += kThreads) before += L.blockLeft[e];
+	for (int o = 32; o > 0; o >>= 1) before += __shfl_xor(before, o);
+	if (__lane_id() == 0) earlier[threadIdx.x / 64] = before;
 	lefts[threadIdx.x] = nl;
 	__syncthreads();
+	before = 0;
+	for (int w = 0; w < kThreads / 64; w++) before += earlier[w];
 	// exclusive prefix over the threads (Hillis-Steele in LDS)
 	for (int o = 1; o < kThreads; o <<= 1) {
 		const int v = threadIdx.x >= (unsigned) o ? lefts[threadIdx.x - o] : 0;
@@ -407,8 +456,8 @@ __global__ void __launch_bounds__(kThreads) k_level_scatter(Level L, Prims P, co
 	}
 	const int leftBefore  = lefts[threadIdx.x] - nl; // lefts of earlier threads of this block
 	const int blockBefore = i0 - L.blockStart[b];	  // references of earlier threads of this block
-	int lp = first + L.blockOff[b] + leftBefore;
-	int rp = first + L.nLeft[t] + (L.blockStart[b] - first - L.blockOff[b]) + (blockBefore - leftBefore);
+	int lp = first + before + leftBefore;
+	int rp = first + L.nLeft[t] + (L.blockStart[b] - first - before) + (blockBefore - leftBefore);
 	for (int k = 0; k < per; k++) {
 		if (i0 + k >= end) break;
 		if (left[k]) tmp[lp++] = r[k];
@@ -416,26 +465,88 @@ __global__ void __launch_bounds__(kThreads) k_level_scatter(Level L, Prims P, co
 	}
 }
 
-__global__ void __launch_bounds__(kThreads) k_level_copy(Level L, const int *tmp, int *refs) {
-	const int b = blockIdx.x, t = L.blockNode[b];
-	const int end = min(L.blockStart[b] + kChunk, L.first[t] + L.count[t]);
-	for (int i = L.blockStart[b] + (int) threadIdx.x; i < end; i += kThreads) refs[i] = tmp[i];
+struct SmallTask {
+	int node, first, count, nodeBase; // descendants take nodeBase, nodeBase + 1, ...
+	int buf;						  // which of the two reference buffers holds the range
+};
+
+__global__ void k_level_init(LevelList list, SmallTask *small, LevelCtl *ctl, int n) {
+	const bool large = n > kSmall;
+	list.first[0]	 = 0;
+	list.count[0]	 = n;
+	list.node[0]	 = 0;
+	list.blockBegin[0] = 0;
+	list.blockBegin[1] = (n + kChunk - 1) / kChunk;
+	small[0]		 = SmallTask{0, 0, n, 1, 0};
+	*ctl			 = LevelCtl{large ? 1 : 0, (n + kChunk - 1) / kChunk, large ? 0 : 1, large ? 1 : 2 * n - 1, 0};
 }
 
-// Binary nodes of the level: box, and children (childBase[t], +1) or a leaf.
-__global__ void k_level_nodes(Level L, int nNodes, const int *childBase, Nodes2 N) {
-	const int t = blockIdx.x * blockDim.x + threadIdx.x;
-	if (t >= nNodes) return;
-	const Box bb = loadBox(L.box + 6 * t);
-	if (L.decision[t] == 1) writeNode(N, L.node[t], bb, -1, -1, L.first[t], L.count[t]);
-	else writeNode(N, L.node[t], bb, childBase[t], childBase[t] + 1, 0, 0);
+// Binary nodes of the level, the next level's list and the subtrees that are
+// small now (their references are in buffer `buf`), in the nodes' order: one
+// block, 1024 nodes at a time, places by a scan.
+__global__ void __launch_bounds__(1024) k_level_next(Level L, int nNodes, LevelList next, SmallTask *small, int buf, Nodes2 N, LevelCtl *ctl) {
+	__shared__ int4 part[16];
+	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+	const int node0 = ctl->nextNode, small0 = ctl->small;
+	int4 carry		= make_int4(0, 0, 0, 0); // large children, their blocks, small children, their descendants
+	for (int base = 0; base < nNodes; base += 1024) {
+		const int t	 = base + (int) threadIdx.x;
+		const bool v = t < nNodes;
+		int f[2] = {0, 0}, c[2] = {0, 0};
+		int4 own = make_int4(0, 0, 0, 0);
+		if (v) {
+			f[0] = L.first[t];
+			c[0] = L.nLeft[t];
+			f[1] = f[0] + c[0];
+			c[1] = L.count[t] - c[0];
+			if (c[0] <= 0 || c[1] <= 0) ctl->bad = 1;
+			writeNode(N, L.node[t], loadBox(L.box + 6 * t), node0 + 2 * t, node0 + 2 * t + 1, 0, 0);
+			for (int k = 0; k < 2; k++) {
+				if (c[k] > kSmall) own.x++, own.y += (c[k] + kChunk - 1) / kChunk;
+				else own.z++, own.w += 2 * max(c[k], 1) - 2;
+			}
+		}
+		int4 incl = own;
+		for (int o = 1; o < 64; o <<= 1) {
+			const int x = __shfl_up(incl.x, o), y = __shfl_up(incl.y, o), z = __shfl_up(incl.z, o), w = __shfl_up(incl.w, o);
+			if (lane >= o) incl.x += x, incl.y += y, incl.z += z, incl.w += w;
+		}
+		if (lane == 63) part[wave] = incl;
+		__syncthreads();
+		int4 at = carry;
+		for (int w = 0; w < 16; w++) {
+			const int4 p = part[w];
+			if (w < wave) at.x += p.x, at.y += p.y, at.z += p.z, at.w += p.w;
+			carry.x += p.x, carry.y += p.y, carry.z += p.z, carry.w += p.w;
+		}
+		at.x += incl.x - own.x, at.y += incl.y - own.y, at.z += incl.z - own.z, at.w += incl.w - own.w;
+		for (int k = 0; k < 2 && v; k++) {
+			const int node = node0 + 2 * t + k;
+			if (c[k] > kSmall) {
+				next.first[at.x]	  = f[k];
+				next.count[at.x]	  = c[k];
+				next.node[at.x]		  = node;
+				next.blockBegin[at.x] = at.y;
+				at.x++;
+				at.y += (c[k] + kChunk - 1) / kChunk;
+			} else {
+				small[small0 + at.z] = SmallTask{node, f[k], c[k], node0 + 2 * nNodes + at.w, buf};
+				at.z++;
+				at.w += 2 * max(c[k], 1) - 2;
+			}
+		}
+		__syncthreads();
+	}
+	if (threadIdx.x == 0) {
+		next.blockBegin[carry.x] = carry.y;
+		ctl->nodes				 = carry.x;
+		ctl->blocks				 = carry.y;
+		ctl->small				 = small0 + carry.z;
+		ctl->nextNode			 = node0 + 2 * nNodes + carry.w;
+	}
 }
 
 // -------------------------------------------- small subtrees, one per block
-
-struct SmallTask {
-	int node, first, count, nodeBase; // descendants take nodeBase, nodeBase + 1, ...
-};
 
 // One block builds the subtree of one task level by level, each wave taking
 // nodes of the level in turn; references (as local indices), primitive boxes
@@ -455,42 +566,7 @@ struct SmallTask {
 // node).
 constexpr int kSmallThreads = 512;
 
-// v combined over 16 lanes (a DPP row) by f, the result in each of them; over
-// the wave when wide.
-template <class F> __device__ inline float rowReduce(float v, F f, bool wide) {
-	auto dpp = [&](auto ctrl) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), ctrl.value, 0xf, 0xf, true)); };
-	v = f(v, dpp(std::integral_constant<int, 0xB1>{}));	 // lanes xor 1 (quad_perm 1 0 3 2)
-	v = f(v, dpp(std::integral_constant<int, 0x4E>{}));	 // lanes xor 2 (quad_perm 2 3 0 1)
-	v = f(v, dpp(std::integral_constant<int, 0x141>{})); // row_half_mirror
-	v = f(v, dpp(std::integral_constant<int, 0x140>{})); // row_mirror
-	if (wide) {
-		v = f(v, __shfl_xor(v, 16));
-		v = f(v, __shfl_xor(v, 32));
-	}
-	return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
-}
-
-// Inclusive scan over the 16 lanes of a row, from lane 0 up (CTRL0 0x110,
-// row_shr) or from lane 15 down (0x100, row_shl); lanes without a source take
-// the identity.
-template <int CTRL0, class F> __device__ inline int rowScan(int v, int identity, F f) {
-	v = f(v, __builtin_amdgcn_update_dpp(identity, v, CTRL0 + 1, 0xf, 0xf, false));
-	v = f(v, __builtin_amdgcn_update_dpp(identity, v, CTRL0 + 2, 0xf, 0xf, false));
-	v = f(v, __builtin_amdgcn_update_dpp(identity, v, CTRL0 + 4, 0xf, 0xf, false));
-	v = f(v, __builtin_amdgcn_update_dpp(identity, v, CTRL0 + 8, 0xf, 0xf, false));
-	return v;
-}
-template <int CTRL0> __device__ inline Box rowScanBox(Box b) {
-	auto lo = [](int x, int y) { return __float_as_int(fminf(__int_as_float(x), __int_as_float(y))); };
-	auto hi = [](int x, int y) { return __float_as_int(fmaxf(__int_as_float(x), __int_as_float(y))); };
-	for (int a = 0; a < 3; a++) {
-		b.lo[a] = __int_as_float(rowScan<CTRL0>(__float_as_int(b.lo[a]), __float_as_int(__builtin_inff()), lo));
-		b.hi[a] = __int_as_float(rowScan<CTRL0>(__float_as_int(b.hi[a]), __float_as_int(-__builtin_inff()), hi));
-	}
-	return b;
-}
-
-__global__ void __launch_bounds__(kSmallThreads) k_small(const SmallTask *tasks, int nTasks, Prims P, int *refs, Nodes2 N, float nodeCost, int maxLeaf) {
+__global__ void __launch_bounds__(kSmallThreads) k_small(const SmallTask *tasks, int nTasks, Prims P, const int *refs1, int *refs, Nodes2 N, float nodeCost, int maxLeaf) {
 	__shared__ float4 sLo[kSmall], sHi[kSmall]; // boxes of the task's primitives, in the order of the references at the start
 	__shared__ uint16_t sRef[kSmall], sTmp[kSmall];
 	__shared__ int2 sList[2][kSmall / 2]; // nodes of a level with at least two references: {node, first << 11 | count}
@@ -507,7 +583,7 @@ __global__ void __launch_bounds__(kSmallThreads) k_small(const SmallTask *tasks,
 		return b;
 	};
 	for (int i = threadIdx.x; i < tk.count; i += kSmallThreads) {
-		const int r = refs[tk.first + i];
+		const int r = (tk.buf ? refs1 : refs)[tk.first + i];
 		float4 l = P.lo[r];
 		l.w	   = __int_as_float(r); // the reference travels with its box
 		sLo[i] = l;
@@ -521,7 +597,10 @@ __global__ void __launch_bounds__(kSmallThreads) k_small(const SmallTask *tasks,
 	}
 	__syncthreads();
 	if (tk.count < 2) { // a single reference is a leaf, as in the loop below
-		if (threadIdx.x == 0 && tk.count == 1) writeNode(N, tk.node, sBox(0), -1, -1, tk.first, 1);
+		if (threadIdx.x == 0 && tk.count == 1) {
+			writeNode(N, tk.node, sBox(0), -1, -1, tk.first, 1);
+			refs[tk.first] = __float_as_int(sLo[0].w);
+		}
 		return;
 	}
 	const int axis = min(lane >> 4, 2), bin = lane & 15;
@@ -578,29 +657,8 @@ __global__ void __launch_bounds__(kSmallThreads) k_small(const SmallTask *tasks,
 					cnt++;
 				}
 			}
-			// the split after this bin: prefix up to it, suffix from the next one
-			auto add = [](int x, int y) { return x + y; };
-			const Box pre = rowScanBox<0x110>(own);
-			Box suf		  = rowScanBox<0x100>(own);
-			const int nPre = rowScan<0x110>(cnt, 0, add);
-			int nSuf	   = rowScan<0x100>(cnt, 0, add);
-			// lane k takes the suffix from bin k + 1
-			for (int a = 0; a < 3; a++) {
-				suf.lo[a] = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(suf.lo[a]), 0x101, 0xf, 0xf, true));
-				suf.hi[a] = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(suf.hi[a]), 0x101, 0xf, 0xf, true));
-			}
-			nSuf		 = __builtin_amdgcn_update_dpp(0, nSuf, 0x101, 0xf, 0xf, true);
-			float cost	 = __builtin_inff();
-			const bool ok = mine && bin < NB - 1 && nPre != 0 && nSuf != 0;
-			if (ok) cost = nodeCost + (pre.area() * nPre + suf.area() * nSuf) / fmaxf(bb.area(), 1e-30f);
-			if (!(cost < __builtin_inff())) cost = __builtin_inff(); // not a number: never the minimum
-			// the first minimum in axis-major, bin-minor order
-			const float best = rowReduce(cost, mn, true);
-			Split s{-1, -1, __builtin_inff()};
-			if (best < __builtin_inff()) {
-				const int w = __ffsll((unsigned long long) __ballot(cost == best)) - 1;
-				s			= Split{w >> 4, w & 15, best};
-			}
+			int nPre;
+			const Split s = waveSplit(own, cnt, mine, bb.area(), nodeCost, nPre);
 			const int d = decide(s, count, maxLeaf);
 			if (d == 1) {
 				if (lane == 0) writeNode(N, node, bb, -1, -1, tk.first + first, count);
@@ -701,47 +759,47 @@ __device__ int collapseKids(const Nodes2 &N, int b, int kids[4]) {
 	return nk;
 }
 
-__global__ void k_collapse_count(Nodes2 N, const int *level, int n, int *inner) {
-	const int i = blockIdx.x * blockDim.x + threadIdx.x;
-	if (i >= n) return;
-	int kids[4];
-	const int nk = collapseKids(N, level[i], kids);
-	int c		 = 0;
-	for (int k = 0; k < nk; k++) c += N.range[kids[k]].y > 0 ? 0 : 1;
-	inner[i] = c;
-}
-
-// Exclusive prefix sum of `n` ints in one block of 1024 threads (chunked).
-__global__ void __launch_bounds__(1024) k_scan_1block(const int *in, int *out, int n, int *total) {
-	__shared__ int part[1024];
-	const int t		= threadIdx.x;
-	const int per	= (n + 1023) / 1024;
-	const int begin = min(n, t * per), end = min(n, begin + per);
-	int s = 0;
-	for (int i = begin; i < end; i++) s += in[i];
-	part[t] = s;
+// Inner children of each node of the level, summed per block of 256.
+__global__ void __launch_bounds__(256) k_collapse_count(Nodes2 N, const int *level, int n, int *blockSum) {
+	__shared__ int part[4];
+	const int i = blockIdx.x * 256 + threadIdx.x;
+	int c		= 0;
+	if (i < n) {
+		int kids[4];
+		const int nk = collapseKids(N, level[i], kids);
+		for (int k = 0; k < nk; k++) c += N.range[kids[k]].y > 0 ? 0 : 1;
+	}
+	for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o);
+	if (__lane_id() == 0) part[threadIdx.x / 64] = c;
 	__syncthreads();
-	for (int o = 1; o < 1024; o <<= 1) {
-		const int v = t >= o ? part[t - o] : 0;
-		__syncthreads();
-		part[t] += v;
-		__syncthreads();
-	}
-	int run = part[t] - s;
-	for (int i = begin; i < end; i++) {
-		const int v = in[i];
-		out[i]		= run;
-		run += v;
-	}
-	if (t == 1023) *total = part[1023];
+	if (threadIdx.x == 0) blockSum[blockIdx.x] = part[0] + part[1] + part[2] + part[3];
 }
 
-__global__ void k_collapse_emit(Nodes2 N, const int *level, int n, int levelBase, const int *off, int nextBase, int *nextLevel,
-								Bvh4Node *out) {
-	const int i = blockIdx.x * blockDim.x + threadIdx.x;
-	if (i >= n) return;
+// The level's 4-wide nodes; the inner children's places in the next level are
+// the sum of the earlier blocks' counts and a scan within the block.
+__global__ void __launch_bounds__(256) k_collapse_emit(Nodes2 N, const int *level, int n, int levelBase, const int *blockSum, int nextBase,
+													   int *nextLevel, Bvh4Node *out, int *total) {
+	__shared__ int earlier[4], part[4];
+	const int i = blockIdx.x * 256 + threadIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x / 64;
+	int before = 0;
+	for (int e = (int) threadIdx.x; e < (int) blockIdx.x; e += 256) before += blockSum[e];
+	for (int o = 32; o > 0; o >>= 1) before += __shfl_xor(before, o);
 	int kids[4];
-	const int nk = collapseKids(N, level[i], kids);
+	const int nk = i < n ? collapseKids(N, level[i], kids) : 0;
+	int own		 = 0;
+	for (int k = 0; k < nk; k++) own += N.range[kids[k]].y > 0 ? 0 : 1;
+	int incl = own;
+	for (int o = 1; o < 64; o <<= 1) {
+		const int u = __shfl_up(incl, o);
+		if (lane >= o) incl += u;
+	}
+	if (lane == 0) earlier[wave] = before;
+	if (lane == 63) part[wave] = incl;
+	__syncthreads();
+	int off = earlier[0] + earlier[1] + earlier[2] + earlier[3] + incl - own;
+	for (int w = 0; w < wave; w++) off += part[w];
+	if (i == n - 1) *total = off + own;
+	if (i >= n) return;
 	Bvh4Node node;
 	for (int c = 0; c < 4; c++) {
 		node.lox[c] = node.loy[c] = node.loz[c] = __builtin_inff();
@@ -766,7 +824,7 @@ __global__ void k_collapse_emit(Nodes2 N, const int *level, int n, int levelBase
 		const int2 r = N.range[k];
 		if (r.y > 0) node.child[c] = ~(r.x * 8 + (r.y - 1));
 		else {
-			const int slot	= off[i] + j++;
+			const int slot	= off + j++;
 			node.child[c]	= nextBase + slot;
 			nextLevel[slot] = k;
 		}
@@ -814,13 +872,18 @@ struct Buf {
 		}                                                                                                                                  \
 	} while (0)
 
-template <class T> hipError_t upload(Buf &b, const std::vector<T> &v, hipStream_t st) {
-	hipError_t e = b.alloc(v.size() * sizeof(T));
-	if (e != hipSuccess || v.empty()) return e;
-	e = hipMemcpyAsync(b.p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice, st);
-	if (e != hipSuccess) return e;
-	return hipStreamSynchronize(st); // v may go out of scope after the call
-}
+// Every temporary of a build in one allocation: sizes are added up first (null
+// base), then taken again from the block.
+struct Arena {
+	char *base	= nullptr;
+	size_t used = 0;
+	template <class T> T *take(size_t count) {
+		used		= (used + 255) / 256 * 256;
+		T *p		= reinterpret_cast<T *>(base + used);
+		used	   += count * sizeof(T);
+		return p;
+	}
+};
 
 } // namespace bvhdev
 
@@ -843,174 +906,150 @@ int buildBvh4Device(const float *pos, int64_t nVerts, const int32_t *idx, int64_
 		hipStream_t s;
 		~StreamGuard() { (void) hipStreamDestroy(s); }
 	} guard{st};
-	Buf dPos, dIdx, dNull, pLo, pHi, refs, tmp, nLo, nHi, nRange;
-	BVHD_HIP(dPos.alloc((size_t) nVerts * 3 * sizeof(float)));
-	BVHD_HIP(dIdx.alloc((size_t) n * 3 * sizeof(int)));
-	BVHD_HIP(dNull.alloc((size_t) n));
-	BVHD_HIP(hipMemcpyAsync(dPos.p, pos, (size_t) nVerts * 3 * sizeof(float), hipMemcpyHostToDevice, st));
-	BVHD_HIP(hipMemcpyAsync(dIdx.p, idx, (size_t) n * 3 * sizeof(int), hipMemcpyHostToDevice, st));
-	if (nullFlag) BVHD_HIP(hipMemcpyAsync(dNull.p, nullFlag, (size_t) n, hipMemcpyHostToDevice, st));
-	else BVHD_HIP(hipMemsetAsync(dNull.p, 0, (size_t) n, st));
+	// at most one large node per kSmall + 1 references of a level, and a block
+	// per kChunk references or part of them
+	const size_t maxT = (size_t) n / (kSmall + 1) + 1, maxB = (size_t) n / kChunk + maxT + 1, maxNodes2 = 2 * (size_t) n;
+	float *dPos;
+	int *dIdx, *refs[2];
+	unsigned char *dNull;
+	float4 *pLo, *pHi, *nLo, *nHi;
+	int2 *nRange;
+	LevelList list[2];
+	Level L;
+	SmallTask *small;
+	LevelCtl *ctl;
+	int *total;
+	auto layout = [&](Arena &m) {
+		dPos   = m.take<float>((size_t) nVerts * 3);
+		dIdx   = m.take<int>((size_t) n * 3);
+		dNull  = m.take<unsigned char>((size_t) n);
+		pLo	   = m.take<float4>((size_t) n);
+		pHi	   = m.take<float4>((size_t) n);
+		nLo	   = m.take<float4>(maxNodes2);
+		nHi	   = m.take<float4>(maxNodes2);
+		nRange = m.take<int2>(maxNodes2);
+		for (int k = 0; k < 2; k++) {
+			refs[k] = m.take<int>((size_t) n);
+			list[k] = LevelList{m.take<int>(maxT), m.take<int>(maxT), m.take<int>(maxT), m.take<int>(maxT + 1)};
+		}
+		L		   = Level{};
+		L.box	   = m.take<int>(6 * maxT);
+		L.cbox	   = m.take<int>(6 * maxT);
+		L.bins	   = m.take<Bins>(maxT);
+		L.decision = m.take<int>(maxT);
+		L.axis	   = m.take<int>(maxT);
+		L.bin	   = m.take<int>(maxT);
+		L.nLeft	   = m.take<int>(maxT);
+		L.blockNode	 = m.take<int>(maxB);
+		L.blockStart = m.take<int>(maxB);
+		L.blockLeft	 = m.take<int>(maxB);
+		small		 = m.take<SmallTask>((size_t) n);
+		ctl			 = m.take<LevelCtl>(1);
+		total		 = m.take<int>(1);
+	};
+	Arena size, arena;
+	layout(size);
+	Buf block;
+	BVHD_HIP(block.alloc(size.used));
+	arena.base = block.as<char>();
+	layout(arena);
+	BVHD_HIP(hipMemcpyAsync(dPos, pos, (size_t) nVerts * 3 * sizeof(float), hipMemcpyHostToDevice, st));
+	BVHD_HIP(hipMemcpyAsync(dIdx, idx, (size_t) n * 3 * sizeof(int), hipMemcpyHostToDevice, st));
+	if (nullFlag) BVHD_HIP(hipMemcpyAsync(dNull, nullFlag, (size_t) n, hipMemcpyHostToDevice, st));
+	else BVHD_HIP(hipMemsetAsync(dNull, 0, (size_t) n, st));
 	BVHD_HIP(hipStreamSynchronize(st));
 	const auto tUp = std::chrono::steady_clock::now();
-	BVHD_HIP(pLo.alloc((size_t) n * sizeof(float4)));
-	BVHD_HIP(pHi.alloc((size_t) n * sizeof(float4)));
-	BVHD_HIP(refs.alloc((size_t) n * sizeof(int)));
-	BVHD_HIP(tmp.alloc((size_t) n * sizeof(int)));
-	const size_t maxNodes2 = 2 * (size_t) n;
-	BVHD_HIP(nLo.alloc(maxNodes2 * sizeof(float4)));
-	BVHD_HIP(nHi.alloc(maxNodes2 * sizeof(float4)));
-	BVHD_HIP(nRange.alloc(maxNodes2 * sizeof(int2)));
-	const Prims P{pLo.as<float4>(), pHi.as<float4>()};
-	const Nodes2 N{nLo.as<float4>(), nHi.as<float4>(), nRange.as<int2>()};
-	hipLaunchKernelGGL(k_prim_boxes, dim3((n + 255) / 256), dim3(256), 0, st, dPos.as<float>(), dIdx.as<int>(), n, pLo.as<float4>(),
-					   pHi.as<float4>(), refs.as<int>());
+	const Prims P{pLo, pHi};
+	const Nodes2 N{nLo, nHi, nRange};
+	hipLaunchKernelGGL(k_prim_boxes, dim3((n + 255) / 256), dim3(256), 0, st, dPos, dIdx, n, pLo, pHi, refs[0]);
+	hipLaunchKernelGGL(k_level_init, dim3(1), dim3(1), 0, st, list[0], small, ctl, n);
 	BVHD_HIP(hipGetLastError());
 
-	// ---- large nodes, level by level (host keeps the node list)
-	std::vector<int> lFirst{0}, lCount{n}, lNode{0};
-	std::vector<SmallTask> small;
-	int nextNode = 1;
-	Buf bFirst, bCount, bNode, bBox, bCbox, bBins, bDec, bAxis, bBin, bLeft, bBlockNode, bBlockStart, bBlockLeft, bBlockOff, bBlockBegin,
-		bChild;
-	int levels = 0;
-	while (!lCount.empty()) {
-		// nodes of this level that are small go to the per-wave phase
-		std::vector<int> f, c, nd;
-		for (size_t t = 0; t < lCount.size(); t++) {
-			if (lCount[t] <= kSmall) small.push_back(SmallTask{lNode[t], lFirst[t], lCount[t], 0});
-			else {
-				f.push_back(lFirst[t]);
-				c.push_back(lCount[t]);
-				nd.push_back(lNode[t]);
-			}
+	// ---- large nodes, level by level: the lists stay on the device, the host
+	// reads the next level's size (uploading the lists and allocating their
+	// buffers anew per level took 6 of the 8.4 ms of a 328 K-triangle build)
+	LevelCtl c{};
+	BVHD_HIP(hipMemcpyAsync(&c, ctl, sizeof(c), hipMemcpyDeviceToHost, st));
+	BVHD_HIP(hipStreamSynchronize(st));
+	int levels = 0, cur = 0;
+	while (c.nodes > 0) {
+		const int T = c.nodes, B = c.blocks;
+		// guards against a malformed level; a split always leaves fewer references a node
+		if ((size_t) T > maxT || (size_t) B > maxB || levels > n) {
+			err = "device BVH build: malformed level";
+			return -1;
 		}
-		if (f.empty()) break;
-		levels++;
-		const int T = (int) f.size();
-		std::vector<int> blockNode, blockStart, blockBegin(T + 1);
-		for (int t = 0; t < T; t++) {
-			blockBegin[t] = (int) blockNode.size();
-			for (int s = f[t]; s < f[t] + c[t]; s += kChunk) {
-				blockNode.push_back(t);
-				blockStart.push_back(s);
-			}
-		}
-		blockBegin[T] = (int) blockNode.size();
-		const int B	  = (int) blockNode.size();
-		BVHD_HIP(upload(bFirst, f, st));
-		BVHD_HIP(upload(bCount, c, st));
-		BVHD_HIP(upload(bNode, nd, st));
-		BVHD_HIP(upload(bBlockNode, blockNode, st));
-		BVHD_HIP(upload(bBlockStart, blockStart, st));
-		BVHD_HIP(upload(bBlockBegin, blockBegin, st));
-		BVHD_HIP(bBox.alloc((size_t) T * 6 * sizeof(int)));
-		BVHD_HIP(bCbox.alloc((size_t) T * 6 * sizeof(int)));
-		BVHD_HIP(bBins.alloc((size_t) T * sizeof(Bins)));
-		BVHD_HIP(bDec.alloc((size_t) T * sizeof(int)));
-		BVHD_HIP(bAxis.alloc((size_t) T * sizeof(int)));
-		BVHD_HIP(bBin.alloc((size_t) T * sizeof(int)));
-		BVHD_HIP(bLeft.alloc((size_t) T * sizeof(int)));
-		BVHD_HIP(bBlockLeft.alloc((size_t) B * sizeof(int)));
-		BVHD_HIP(bBlockOff.alloc((size_t) B * sizeof(int)));
-		Level L{bFirst.as<int>(),	 bCount.as<int>(),	  bNode.as<int>(),		bBox.as<int>(),		   bCbox.as<int>(),
-				bBins.as<Bins>(),	 bDec.as<int>(),	  bAxis.as<int>(),		bBin.as<int>(),		   bLeft.as<int>(),
-				bBlockNode.as<int>(), bBlockStart.as<int>(), bBlockLeft.as<int>(), bBlockOff.as<int>(), bBlockBegin.as<int>()};
+		L.first		 = list[cur].first;
+		L.count		 = list[cur].count;
+		L.node		 = list[cur].node;
+		L.blockBegin = list[cur].blockBegin;
+		const int *in = refs[levels & 1];
+		int *to		  = refs[(levels & 1) ^ 1];
 		hipLaunchKernelGGL(k_level_reset, dim3(T), dim3(256), 0, st, L, T);
-		hipLaunchKernelGGL(k_level_bounds, dim3(B), dim3(kThreads), 0, st, L, P, (const int *) refs.as<int>());
-		hipLaunchKernelGGL(k_level_bins, dim3(B), dim3(kThreads), 0, st, L, P, (const int *) refs.as<int>());
-		hipLaunchKernelGGL(k_level_split, dim3((T + 63) / 64), dim3(64), 0, st, L, T, cost, maxLeaf);
-		hipLaunchKernelGGL(k_level_count, dim3(B), dim3(kThreads), 0, st, L, P, (const int *) refs.as<int>());
-		hipLaunchKernelGGL(k_level_scan, dim3((T + 63) / 64), dim3(64), 0, st, L, T);
-		hipLaunchKernelGGL(k_level_scatter, dim3(B), dim3(kThreads), 0, st, L, P, (const int *) refs.as<int>(), tmp.as<int>());
-		hipLaunchKernelGGL(k_level_copy, dim3(B), dim3(kThreads), 0, st, L, (const int *) tmp.as<int>(), refs.as<int>());
+		hipLaunchKernelGGL(k_level_bounds, dim3(B), dim3(kThreads), 0, st, L, P, in);
+		hipLaunchKernelGGL(k_level_bins, dim3(B), dim3(kThreads), 0, st, L, P, in);
+		hipLaunchKernelGGL(k_level_split, dim3(T), dim3(64), 0, st, L, T, cost, maxLeaf);
+		hipLaunchKernelGGL(k_level_count, dim3(B), dim3(kThreads), 0, st, L, P, in);
+		hipLaunchKernelGGL(k_level_scatter, dim3(B), dim3(kThreads), 0, st, L, P, in, to);
+		hipLaunchKernelGGL(k_level_next, dim3(1), dim3(1024), 0, st, L, T, list[cur ^ 1], small, (levels & 1) ^ 1, N, ctl);
 		BVHD_HIP(hipGetLastError());
-		std::vector<int> dec(T), left(T);
-		BVHD_HIP(hipMemcpyAsync(dec.data(), bDec.p, T * sizeof(int), hipMemcpyDeviceToHost, st));
-		BVHD_HIP(hipMemcpyAsync(left.data(), bLeft.p, T * sizeof(int), hipMemcpyDeviceToHost, st));
+		BVHD_HIP(hipMemcpyAsync(&c, ctl, sizeof(c), hipMemcpyDeviceToHost, st));
 		BVHD_HIP(hipStreamSynchronize(st));
-		std::vector<int> childBase(T, -1), nf, nc, nn;
-		for (int t = 0; t < T; t++) {
-			if (dec[t] == 1) continue; // not reached for nodes above kSmall (> 8 references)
-			int nl = dec[t] == 2 ? c[t] / 2 : left[t];
-			if (nl <= 0 || nl >= c[t]) {
-				err = "device BVH build: empty side in a large-node split";
-				return -1;
-			}
-			childBase[t] = nextNode;
-			nextNode += 2;
-			nf.push_back(f[t]);
-			nc.push_back(nl);
-			nn.push_back(childBase[t]);
-			nf.push_back(f[t] + nl);
-			nc.push_back(c[t] - nl);
-			nn.push_back(childBase[t] + 1);
+		if (c.bad) {
+			err = "device BVH build: empty side in a large-node split";
+			return -1;
 		}
-		BVHD_HIP(upload(bChild, childBase, st));
-		hipLaunchKernelGGL(k_level_nodes, dim3((T + 63) / 64), dim3(64), 0, st, L, T, (const int *) bChild.as<int>(), N);
-		BVHD_HIP(hipGetLastError());
-		BVHD_HIP(hipStreamSynchronize(st)); // the level buffers are reallocated next round
-		lFirst.swap(nf);
-		lCount.swap(nc);
-		lNode.swap(nn);
+		cur ^= 1;
+		levels++;
 	}
 	const auto tLarge = std::chrono::steady_clock::now();
-	// ---- small subtrees, one wave each; descendants numbered per subtree
-	for (SmallTask &t : small) {
-		t.nodeBase = nextNode;
-		nextNode += 2 * t.count - 2;
-	}
-	if ((size_t) nextNode > maxNodes2) {
+	// ---- small subtrees, one block each; descendants numbered per subtree
+	if ((size_t) c.nextNode > maxNodes2 || c.small > n) {
 		err = "device BVH build: node count overflow";
 		return -1;
 	}
-	if (!small.empty()) {
-		Buf bSmall;
-		BVHD_HIP(upload(bSmall, small, st));
-		hipLaunchKernelGGL(k_small, dim3((unsigned) small.size()), dim3(kSmallThreads), 0, st, (const SmallTask *) bSmall.as<SmallTask>(),
-						   (int) small.size(), P, refs.as<int>(), N, cost, maxLeaf);
+	if (c.small > 0) {
+		hipLaunchKernelGGL(k_small, dim3((unsigned) c.small), dim3(kSmallThreads), 0, st, small, c.small, P, refs[1], refs[0], N, cost, maxLeaf);
 		BVHD_HIP(hipGetLastError());
 		BVHD_HIP(hipStreamSynchronize(st));
 	}
 	const auto tSmall = std::chrono::steady_clock::now();
-	// ---- collapse to 4-wide nodes, level by level
-	Buf lvl[2], inner, off, total, nodes4, tris;
-	BVHD_HIP(lvl[0].alloc(maxNodes2 * sizeof(int)));
-	BVHD_HIP(lvl[1].alloc(maxNodes2 * sizeof(int)));
-	BVHD_HIP(inner.alloc(maxNodes2 * sizeof(int)));
-	BVHD_HIP(off.alloc(maxNodes2 * sizeof(int)));
-	BVHD_HIP(total.alloc(sizeof(int)));
+	// ---- collapse to 4-wide nodes, level by level; the level lists and block
+	// sums take the place of the primitive boxes and the second references
+	Buf nodes4, tris;
+	int *lvl[2]	  = {reinterpret_cast<int *>(pLo), reinterpret_cast<int *>(pHi)};
+	int *blockSum = refs[1];
 	// at most one 4-wide node per inner binary node, plus the root
-	const size_t cap4 = (size_t) nextNode / 2 + 1;
+	const size_t cap4 = (size_t) c.nextNode / 2 + 1;
 	BVHD_HIP(nodes4.alloc(cap4 * sizeof(Bvh4Node)));
 	const int zero = 0;
-	BVHD_HIP(hipMemcpyAsync(lvl[0].p, &zero, sizeof(int), hipMemcpyHostToDevice, st));
-	int levelN = 1, levelBase = 0, depth = 0, cur = 0;
+	BVHD_HIP(hipMemcpyAsync(lvl[0], &zero, sizeof(int), hipMemcpyHostToDevice, st));
+	int levelN = 1, levelBase = 0, depth = 0;
+	cur = 0;
 	while (levelN > 0) {
 		depth++;
 		// a well-formed tree never trips these; they keep a malformed one from
 		// writing past the node array or looping
-		if (depth > 64 || (size_t) levelBase + (size_t) levelN > cap4 || (size_t) levelN > maxNodes2) {
+		if (depth > 64 || (size_t) levelBase + (size_t) levelN > cap4 || levelN > n) {
 			err = "device BVH build: malformed tree in the 4-wide collapse";
 			return -1;
 		}
-		const unsigned g = (unsigned) ((levelN + 255) / 256);
-		hipLaunchKernelGGL(k_collapse_count, dim3(g), dim3(256), 0, st, N, (const int *) lvl[cur].as<int>(), levelN, inner.as<int>());
-		hipLaunchKernelGGL(k_scan_1block, dim3(1), dim3(1024), 0, st, (const int *) inner.as<int>(), off.as<int>(), levelN, total.as<int>());
+		const unsigned g   = (unsigned) ((levelN + 255) / 256);
 		const int nextBase = levelBase + levelN;
-		hipLaunchKernelGGL(k_collapse_emit, dim3(g), dim3(256), 0, st, N, (const int *) lvl[cur].as<int>(), levelN, levelBase,
-						   (const int *) off.as<int>(), nextBase, lvl[cur ^ 1].as<int>(), nodes4.as<Bvh4Node>());
+		hipLaunchKernelGGL(k_collapse_count, dim3(g), dim3(256), 0, st, N, (const int *) lvl[cur], levelN, blockSum);
+		hipLaunchKernelGGL(k_collapse_emit, dim3(g), dim3(256), 0, st, N, (const int *) lvl[cur], levelN, levelBase, (const int *) blockSum, nextBase,
+						   lvl[cur ^ 1], nodes4.as<Bvh4Node>(), total);
 		BVHD_HIP(hipGetLastError());
 		int nextN = 0;
-		BVHD_HIP(hipMemcpyAsync(&nextN, total.p, sizeof(int), hipMemcpyDeviceToHost, st));
+		BVHD_HIP(hipMemcpyAsync(&nextN, total, sizeof(int), hipMemcpyDeviceToHost, st));
 		BVHD_HIP(hipStreamSynchronize(st));
 		levelBase = nextBase;
 		levelN	  = nextN;
 		cur ^= 1;
 	}
 	BVHD_HIP(tris.alloc((size_t) n * sizeof(LeafTri)));
-	hipLaunchKernelGGL(k_leaf_tris, dim3((n + 255) / 256), dim3(256), 0, st, (const float *) dPos.as<float>(), (const int *) dIdx.as<int>(),
-					   (const unsigned char *) dNull.as<unsigned char>(), (const int *) refs.as<int>(), n, tris.as<LeafTri>());
+	hipLaunchKernelGGL(k_leaf_tris, dim3((n + 255) / 256), dim3(256), 0, st, (const float *) dPos, (const int *) dIdx, (const unsigned char *) dNull,
+					   (const int *) refs[0], n, tris.as<LeafTri>());
 	BVHD_HIP(hipGetLastError());
 	BVHD_HIP(hipStreamSynchronize(st));
 	out.nodes	   = nodes4.p;
@@ -1019,10 +1058,10 @@ int buildBvh4Device(const float *pos, int64_t nVerts, const int32_t *idx, int64_
 	tris.p		   = nullptr;
 	out.nNodes	   = levelBase;
 	out.nTris	   = n;
-	out.nBinary	   = nextNode;
+	out.nBinary	   = c.nextNode;
 	out.maxDepth   = depth;
 	out.largeLevels = levels;
-	out.smallTrees = (int64_t) small.size();
+	out.smallTrees = c.small;
 	const auto t1  = std::chrono::steady_clock::now();
 	out.seconds	   = std::chrono::duration<double>(t1 - t0).count();
 	out.buildSeconds = std::chrono::duration<double>(t1 - tUp).count();

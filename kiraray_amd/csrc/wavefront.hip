@@ -1547,7 +1547,12 @@ __global__ void k_quantize_nodes(const Bvh4Node *in, int64_t n, Bvh4QNode *out) 
 
 namespace {
 
+// The 64-byte copy of the nodes, for traversals that read it.
 int quantizeAccel(AccelData &a) {
+	if (!a.quantized) {
+		a.qnodes.release();
+		return KRR_OK;
+	}
 	KRR_HIP(a.qnodes.alloc((size_t) std::max<int64_t>(a.nNodes, 1) * sizeof(Bvh4QNode)));
 	if (a.nNodes > 0) {
 		hipLaunchKernelGGL(k_quantize_nodes, dim3((unsigned) ((a.nNodes + 255) / 256)), dim3(256), 0, 0, a.nodes.as<Bvh4Node>(), a.nNodes,
@@ -2133,8 +2138,8 @@ int uploadScene(krr_wf *wf, const krr_scene_desc *s) {
 	else wf->tan.release();
 	if (!texs.empty()) KRR_HIP(wf->textures.upload(texs.data(), texs.size() * sizeof(DevTexture)));
 	else wf->textures.release();
-	int rc = buildAccel(s, wf->accel, wf->leafSize, wf->sahNodeCost, wf->deviceBuilder);
 	wf->accel.quantized = wf->quantizedNodes;
+	int rc = buildAccel(s, wf->accel, wf->leafSize, wf->sahNodeCost, wf->deviceBuilder);
 	if (rc) return rc;
 	DevScene &ds	= wf->ds;
 	ds.pos			= wf->pos.as<float>();
@@ -2315,10 +2320,10 @@ int krr_accel_build(const krr_scene_desc *scene, const char *json_opts, krr_acce
 	for (int m = 0; m < scene->n_meshes; m++)
 		if (scene->meshes[m].material >= scene->n_materials) return krr::fail(KRR_ERR_INVALID_ARG, "mesh %d material out of range", m);
 	auto a = std::make_unique<krr_accel>();
-	int rc = buildAccel(scene, a->a, leafSize, nodeCost, deviceBuilder);
-	if (rc) return rc;
-	a->a.stackLds  = stackLdsEntries;
 	a->a.quantized = quantized;
+	int rc		   = buildAccel(scene, a->a, leafSize, nodeCost, deviceBuilder);
+	if (rc) return rc;
+	a->a.stackLds = stackLdsEntries;
 	KRR_HIP(a->counters.alloc(sizeof(Counters)));
 	KRR_HIP(hipMemset(a->counters.p, 0, sizeof(Counters)));
 	*out = a.release();
