@@ -58,7 +58,11 @@ KRR_HD f3 vabs(const f3 &v) { return {fabsf(v.x), fabsf(v.y), fabsf(v.z)}; }
 KRR_HD f3 vmaxs(const f3 &v, float s) { return {v.x > s ? v.x : s, v.y > s ? v.y : s, v.z > s ? v.z : s}; }
 KRR_HD f3 vmins(const f3 &v, float s) { return {v.x < s ? v.x : s, v.y < s ? v.y : s, v.z < s ? v.z : s}; }
 KRR_HD f3 vsqrt(const f3 &v) { return {sqrtf(v.x), sqrtf(v.y), sqrtf(v.z)}; }
-KRR_HD f3 vexp(const f3 &v) { return {detmath::expf(v.x), detmath::expf(v.y), detmath::expf(v.z)}; }
+// Equal components (a grey medium's optical depth) share one exponential.
+KRR_HD f3 vexp(const f3 &v) {
+	const float e = detmath::expf(v.x);
+	return {e, v.y == v.x ? e : detmath::expf(v.y), v.z == v.x ? e : detmath::expf(v.z)};
+}
 KRR_HD float clampf(float v, float lo, float hi) { return v < lo ? lo : (v > hi ? hi : v); }
 KRR_HD float pow2(float x) { return x * x; }
 KRR_HD float maxf(float a, float b) { return a > b ? a : b; }

@@ -284,6 +284,7 @@ KRR_DEV f3 sampleTmaj(const DevScene &sc, int medium, f3 o, f3 d, float tMax, Pc
 	MajorantSeg seg;
 	while (true) {
 		if (!it.next(seg)) return T_maj;
+		if (!seg.sigma_maj.any()) continue; // empty cell: T_maj times exp(0)
 		if (seg.sigma_maj[channel] == 0.f) {
 			float dt = seg.tMax - seg.tMin;
 			if (__builtin_isinf(dt)) dt = kFloatMax;

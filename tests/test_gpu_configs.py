@@ -138,3 +138,23 @@ def test_nrc_on_1080p_field(krr, gpu):
     _, plain = gpu_render(krr, gpu, s, 1920, 1080, base, frame_index=8)
     print("plain rays", plain["closest_rays"], plain["shadow_rays"], flush=True)
     assert st["closest_rays"] < 0.9 * plain["closest_rays"]
+
+
+@pytest.mark.parametrize("res,sigma_t", [([1, 1, 1], [3.0, 3.0, 3.0]), ([2, 3, 2], [4.0, 4.0, 4.0]), ([5, 4, 6], [1.0, 4.0, 2.5]), ([5, 4, 6], [2.0, 2.0, 5.0])])
+def test_small_grid_media_match_checker(krr, oracle, gpu, res, sigma_t):
+    """Grids whose lookups are all, partly or never on the border, with empty
+    voxels, grey media (one exponential for the three channels) and coloured
+    ones."""
+    print(f"case: dense grid {res} sigma_t {sigma_t}, 48x40", flush=True)
+    rng = np.random.default_rng(sum(res))
+    density = rng.random(res[0] * res[1] * res[2])
+    density[rng.random(len(density)) < 0.4] = 0.0
+    cfg = icosphere_scene(count=16, level=1, res=(48, 40))
+    cfg["media"] = [{"type": "dense_grid", "res": res, "density": density.tolist(), "sigma_t": sigma_t, "albedo": [0.8, 0.7, 0.6], "g": 0.2}]
+    cfg["camera"]["medium"] = 0
+    s = krr.Scene(cfg)
+    params = dict(spp=2, max_depth=10, rr=0.8, rr_min_depth=3)
+    g, gs = gpu_render(krr, gpu, s, 48, 40, params)
+    o, os_ = oracle.render(s.desc, s.camera(0), 48, 40, 1, **params)
+    assert gs["closest_rays"] == os_["closest_rays"] and gs["shadow_rays"] == os_["shadow_rays"]
+    assert_images_match(g, o)
