@@ -208,3 +208,31 @@ def test_node_formats_on_hard_rays(krr, oracle, gpu, node_format):
     _assert_same_hits(g, o)
     assert np.array_equal(vis, oracle.trace_any(s.desc, rays))
     assert (o["prim"] >= 0).mean() > 0.2
+
+
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 1000, 4097, 30001])
+@pytest.mark.parametrize("count,level", [(1, 1), (200, 2)])
+def test_ray_counts_and_refill(krr, oracle, gpu, n, count, level):
+    """Ray arrays from one ray to several per lane, on a tree below and one
+    above the small-tree line: few rays go to many waves with few lanes each,
+    waves take new rays as old ones end.  Closest (both entry points) and any
+    hits equal the checker's."""
+    print(f"case: {n} rays, {count} icospheres of level {level}", flush=True)
+    s = krr.Scene(icosphere_scene(count=count, level=level, res=(8, 8)))
+    pos, idx, _ = s.arrays()
+    rng = np.random.default_rng(n)
+    rays = _rays_towards_triangles(pos, idx, n, rng, np.array([-0.5, 0.0, -0.5]), np.array([1.5, 1.7, 1.5]), jitter=0.05)
+    rays[::5, 3] = 0.5
+    rays[::7, 4] = 0.0
+    g, vis, _ = _gpu_closest(krr, gpu, s, rays)
+    o = oracle.trace_closest(s.desc, rays)
+    _assert_same_hits(g, o)
+    assert np.array_equal(vis, oracle.trace_any(s.desc, rays))
+    acc = krr.Accel(s.desc)
+    r, hits = gpu.DeviceBuffer.from_numpy(rays), gpu.DeviceBuffer(n * 16)
+    acc.trace_closest_noalloc(r.ptr, n, hits.ptr, 0)
+    gpu.synchronize()
+    h = hits.to_numpy(np.float32, (n, 4))
+    assert np.array_equal(h[:, 0], g["t"]) and np.array_equal(h[:, 1].view(np.int32), g["prim"])
+    assert np.array_equal(h[:, 2], g["b1"]) and np.array_equal(h[:, 3], g["b2"])
+    acc.close()
