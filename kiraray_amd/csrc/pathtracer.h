@@ -19,7 +19,10 @@ struct PtArgs {
 	float4 *film;		  // W x H, row H-1-y
 	int *ovf;			  // traversal stack overflow: (stack size - LDS entries) * grid * tb ints
 	unsigned long long *rays; // [0] closest rays, [1] shadow rays (added to)
-	int tilesX, nTiles;		  // 8 x 8-pixel tiles, one per wave at a time
+	int *work;				  // next place to take up: pixel i % 64 of tile i / 64
+	int fetchLanes;			  // lanes of a wave that take up pixels
+	int refillLanes;		  // a traversal round ends below this many traversing lanes of 64 (0: rays run to their end)
+	int tilesX, nTiles;		  // 8 x 8-pixel tiles
 	bool textured;			  // textures, image-lit infinite lights or alpha tests: the kernel with those lookups
 };
 

@@ -3268,7 +3268,7 @@ struct krr_mk {
 	bool haveCamera	 = false;
 	uint64_t frameIndex = 0;
 	DevBuf rays, ovf;
-	int grid		 = 0;
+	PathGrid grid;
 	uint64_t gridKey = ~0ull;
 	hipStream_t lastStream = nullptr;
 	hipEvent_t ev[2]	   = {nullptr, nullptr};
@@ -3397,7 +3397,6 @@ int krr_mk_render(krr_mk *mk, float *film_dev, void *hip_stream) {
 	const size_t lds   = stackLds(wf->accel, tb);
 	const int tilesX = (mk->W + 7) / 8, tilesY = (mk->H + 7) / 8;
 	const int nTiles = tilesX * tilesY;
-	const int needed = (nTiles + tb / 64 - 1) / (tb / 64);
 	const uint64_t key = ((uint64_t) nTiles << 20) ^ ((uint64_t) tb << 8) ^ ((uint64_t) wf->accel.stackSize << 44) ^
 						 ((uint64_t) wf->stackLdsEntries << 36) ^ ((uint64_t) (mk->occupancy * 1024.f) << 52) ^ (wf->sceneTextured ? 1ull : 0ull);
 	if (key != mk->gridKey) {
@@ -3405,9 +3404,9 @@ int krr_mk_render(krr_mk *mk, float *film_dev, void *hip_stream) {
 		KRR_HIP(hipGetDevice(&dev));
 		KRR_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
 		const int resident = scaledGrid(pathTracerBlocksPerCU(tb, lds, wf->sceneTextured) * std::max(cus, 1), mk->occupancy);
-		mk->grid		   = std::max(1, std::min(needed, resident));
-		if (int rc = reserveOverflow(mk->ovf, wf->accel, (size_t) mk->grid * tb)) return rc;
-		if (!mk->rays.p) KRR_HIP(mk->rays.alloc(2 * sizeof(unsigned long long)));
+		mk->grid		   = pathGrid(resident, tb, (int64_t) nTiles * 64, smallTree(wf->accel));
+		if (int rc = reserveOverflow(mk->ovf, wf->accel, (size_t) mk->grid.blocks * tb)) return rc;
+		if (!mk->rays.p) KRR_HIP(mk->rays.alloc(256)); // the two counts, and the work counter on a line of its own
 		mk->gridKey = key;
 	}
 	if ((size_t) (bvh.stackLds + kStackPad) * tb * sizeof(int) != lds) return krr::fail(KRR_ERR_INVALID_ARG, "krr_mk_render: stack layout mismatch");
@@ -3425,6 +3424,9 @@ int krr_mk_render(krr_mk *mk, float *film_dev, void *hip_stream) {
 	a.film		  = (float4 *) film_dev;
 	a.ovf		  = mk->ovf.as<int>();
 	a.rays		  = mk->rays.as<unsigned long long>();
+	a.work		  = mk->rays.as<int>() + 32;
+	a.fetchLanes  = mk->grid.lanes;
+	a.refillLanes = refillLanesOf(wf);
 	a.tilesX	  = tilesX;
 	a.nTiles	  = nTiles;
 	a.textured	  = wf->sceneTextured;
@@ -3434,7 +3436,7 @@ int krr_mk_render(krr_mk *mk, float *film_dev, void *hip_stream) {
 			if (!e) KRR_HIP(hipEventCreate(&e));
 		KRR_HIP(hipEventRecord(mk->ev[0], st));
 	}
-	KRR_HIP(launchPathTracer(a, mk->grid, tb, lds, st));
+	KRR_HIP(launchPathTracer(a, mk->grid.blocks, tb, lds, st));
 	if (mk->timed) KRR_HIP(hipEventRecord(mk->ev[1], st));
 	mk->paths = (uint64_t) mk->W * mk->H * mk->spp;
 	return KRR_OK;

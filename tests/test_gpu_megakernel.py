@@ -77,3 +77,18 @@ def test_uneven_film_and_repeat(krr, oracle, gpu):
     o, os_ = oracle.render_megakernel(s.desc, s.camera(0), 61, 37, 7, spp=2)
     assert sa["closest_rays"] == os_["closest_rays"]
     assert_images_match(a, o)
+
+
+@pytest.mark.parametrize("w,h,spp,field,more", [(1, 1, 3, False, {}), (7, 3, 2, True, {}), (9, 17, 3, False, {}), (65, 33, 2, True, {}),
+                                                (130, 90, 2, True, {"occupancy": 0.01}), (61, 50, 2, False, {"occupancy": 0.01, "block_size": 64})])
+def test_pixels_taken_up_by_lanes(krr, oracle, gpu, w, h, spp, field, more):
+    """Images that do not fill their 8 x 8 tiles, a lane's samples one after
+    the other, and launches held to few blocks, whose lanes take up pixel
+    after pixel; rays run to their end on the small tree and are refilled on
+    the large one."""
+    print(f"case: megakernel {w}x{h} {spp} spp field={field} {more}", flush=True)
+    s = krr.Scene(icosphere_scene(count=200, level=2, res=(w, h)) if field else CORNELL)
+    g, gs = mk_render(krr, gpu, s, w, h, dict({"max_depth": 6, "spp": spp}, **more), frame_index=2)
+    o, os_ = oracle.render_megakernel(s.desc, s.camera(0), w, h, 2, spp=spp, max_depth=6)
+    assert gs["closest_rays"] == os_["closest_rays"] and gs["shadow_rays"] == os_["shadow_rays"]
+    assert_images_match(g, o)
