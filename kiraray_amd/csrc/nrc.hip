@@ -225,46 +225,81 @@ __global__ void __launch_bounds__(256) k_encode(const float *vertices, int64_t n
 	out[i] = encodeSlot(vertices + row * 16, g, 4 * s + j);
 }
 
-// Inference: each wave evaluates tiles of 32 samples.
-__global__ void __launch_bounds__(256) k_infer(const uint16_t *wtAll, const float *vertices, int64_t n, float *radiance) {
+// Vertex record i as 16 floats, zeros past the end.
+__device__ __forceinline__ void loadVertex(const float *vertices, int64_t i, int64_t n, float v[16]) {
+	if (i < n) {
+		const float4 *p = reinterpret_cast<const float4 *>(vertices + i * 16);
+#pragma unroll
+		for (int q = 0; q < 4; q++) {
+			const float4 f = p[q];
+			v[4 * q]	   = f.x;
+			v[4 * q + 1]   = f.y;
+			v[4 * q + 2]   = f.z;
+			v[4 * q + 3]   = f.w;
+		}
+	} else {
+#pragma unroll
+		for (int q = 0; q < 16; q++) v[q] = 0.f;
+	}
+}
+
+// Inference: each wave evaluates T tiles of 32 samples at a time.  Reading a
+// layer's weights from LDS takes as long as the matrix cores take for one tile
+// (47 KB at 128 bytes a cycle, 370 cycles each), so with two tiles per wave the
+// reads halve; 118 registers leave 4 waves per SIMD, in two blocks of 8 waves
+// that share a copy of the weights each and stay resident.  1 M samples 51
+// against 58 us, 4 M 197 against 228 us on one card; on another 53 against 61
+// (one tile, 5 waves: 57; two tiles with the next ones prefetched, 3 waves: 55;
+// four tiles: 59).  A wave's own vector work (encoding, rounding) is the larger
+// part now.
+template <int T, int THREADS, int WAVES>
+__global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WAVES, 8))) k_infer(const uint16_t *wtAll, const float *vertices, int64_t n, float *radiance) {
 	extern __shared__ uint16_t ldsW[];
 	loadWeights(ldsW, wtAll);
 	__syncthreads();
 	const int lane = threadIdx.x & 63, g = lane >> 5, m = lane & 31;
-	const int wavesPerBlock = blockDim.x >> 6;
-	const int64_t tiles		= (n + 31) / 32;
-	for (int64_t t = (int64_t) blockIdx.x * wavesPerBlock + (threadIdx.x >> 6); t < tiles; t += (int64_t) gridDim.x * wavesPerBlock) {
-		const int64_t i = t * 32 + m;
-		float v[16];
-		if (i < n) {
-			const float4 *p = reinterpret_cast<const float4 *>(vertices + i * 16);
+	const int64_t tiles = (n + 32 * T - 1) / (32 * T), stride = (int64_t) gridDim.x * (THREADS / 64);
+	int64_t t = (int64_t) blockIdx.x * (THREADS / 64) + (threadIdx.x >> 6);
+	for (; t < tiles; t += stride) {
+		float v[T][16];
+		short4v x[T][8];
 #pragma unroll
-			for (int q = 0; q < 4; q++) {
-				const float4 f = p[q];
-				v[4 * q]	   = f.x;
-				v[4 * q + 1]   = f.y;
-				v[4 * q + 2]   = f.z;
-				v[4 * q + 3]   = f.w;
-			}
-		} else {
+		for (int k = 0; k < T; k++) loadVertex(vertices, (t * T + k) * 32 + m, n, v[k]);
 #pragma unroll
-			for (int q = 0; q < 16; q++) v[q] = 0.f;
-		}
-		short4v x[8], y[8];
-		encodeB(v, g, x);
-		float16v a0, a1;
+		for (int k = 0; k < T; k++) encodeB(v[k], g, x[k]);
 		// not unrolled: an unrolled loop hoists every layer's weight loads
 #pragma unroll 1
 		for (int l = 0; l < kHidden; l++) {
-			hiddenForward(ldsW + l * 64 * kRowH, lane, g, x, y, a0, a1);
+			const uint16_t *wt = ldsW + l * 64 * kRowH;
+			float16v a0[T], a1[T];
 #pragma unroll
-			for (int s = 0; s < 8; s++) x[s] = y[s];
+			for (int k = 0; k < T; k++) a0[k] = a1[k] = zero16();
+#pragma unroll
+			for (int s = 0; s < 8; s += 2) {
+				const short4v w00 = ldsA(wt, m, s, g), w01 = ldsA(wt, m, s + 1, g), w10 = ldsA(wt, 32 + m, s, g), w11 = ldsA(wt, 32 + m, s + 1, g);
+#pragma unroll
+				for (int k = 0; k < T; k++) {
+					a0[k] = mfma2(w00, w01, x[k][s], x[k][s + 1], a0[k]);
+					a1[k] = mfma2(w10, w11, x[k][s], x[k][s + 1], a1[k]);
+				}
+			}
+#pragma unroll
+			for (int k = 0; k < T; k++)
+#pragma unroll
+				for (int s = 0; s < 4; s++) {
+					x[k][s]		= pack4(fmaxf(a0[k][4 * s], 0.f), fmaxf(a0[k][4 * s + 1], 0.f), fmaxf(a0[k][4 * s + 2], 0.f), fmaxf(a0[k][4 * s + 3], 0.f));
+					x[k][4 + s] = pack4(fmaxf(a1[k][4 * s], 0.f), fmaxf(a1[k][4 * s + 1], 0.f), fmaxf(a1[k][4 * s + 2], 0.f), fmaxf(a1[k][4 * s + 3], 0.f));
+				}
 		}
-		const float16v o = outputForward(ldsW + kHidden * 64 * kRowH, lane, g, x);
-		if (g == 0 && i < n) {
-			radiance[3 * i]		= o[0];
-			radiance[3 * i + 1] = o[1];
-			radiance[3 * i + 2] = o[2];
+#pragma unroll
+		for (int k = 0; k < T; k++) {
+			const float16v o = outputForward(ldsW + kHidden * 64 * kRowH, lane, g, x[k]);
+			const int64_t i	 = (t * T + k) * 32 + m;
+			if (g == 0 && i < n) {
+				radiance[3 * i]		= o[0];
+				radiance[3 * i + 1] = o[1];
+				radiance[3 * i + 2] = o[2];
+			}
 		}
 	}
 }
@@ -682,6 +717,7 @@ struct Buf {
 		if (e_ != hipSuccess) return krr::fail(KRR_ERR_HIP, "%s: %s", #expr, hipGetErrorString(e_));                  \
 	} while (0)
 
+constexpr int64_t kInferSmall = 1 << 17;
 constexpr int kChunk	= 1024; // batch granularity of the training buffers
 constexpr int kWChunk = 256;	// samples per split-K chunk of the weight gradient
 static_assert(kWChunk % 64 == 0, "k_weight_grad loads eight 8-sample k-steps at a time");
@@ -693,6 +729,7 @@ struct krr_nrc {
 	uint64_t seed	= 1;
 	int64_t maxBatch = 65536, ld = 0;
 	bool bwdLds		 = false; // the device's blocks hold both padded weight copies in LDS
+	int cus			 = 256;
 	int inferBlocks	 = 1024;  // k_infer_queue blocks resident at once on the device (each loads the weights once)
 	Buf w, m, v, grad, wt, wb, xT, dzT, partial, tileLoss, loss, step;
 };
@@ -817,6 +854,7 @@ int krr_nrc_create(const char *json, krr_nrc **out) {
 		int cus = 0, perCu = 0;
 		NRC_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
 		NRC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCu, k_infer_queue, kInferBlock, kFwdLdsElems * sizeof(uint16_t)));
+		h->cus		   = std::max(cus, 1);
 		h->inferBlocks = std::max(1, cus * std::max(perCu, 1));
 	}
 	NRC_HIP(h->wt.alloc(sizeof(uint16_t) * kFwdElems));
@@ -873,10 +911,13 @@ int krr_nrc_infer(krr_nrc *nrc, const krr_nrc_vertex *vertices_dev, int64_t n, f
 	krr::clearError();
 	if (!nrc || !validN(n) || (n > 0 && (!vertices_dev || !radiance_dev))) return krr::fail(KRR_ERR_INVALID_ARG, "krr_nrc_infer: bad argument");
 	if (n == 0) return KRR_OK;
-	const int64_t tiles = (n + 31) / 32;
-	const int blocks	= (int) std::min<int64_t>(2048, (tiles + 3) / 4);
-	hipLaunchKernelGGL(k_infer, dim3(blocks), dim3(256), kFwdLdsElems * (int) sizeof(uint16_t), (hipStream_t) hip_stream, nrc->wt.as<uint16_t>(),
-					   (const float *) vertices_dev, n, radiance_dev);
+	// up to kInferSmall samples, one tile per wave in small blocks: the chip is
+	// not full and the launch is most of the time (60 K samples 6.8 us)
+	const bool small  = n <= kInferSmall;
+	const int threads = small ? 256 : 512, perBlock = 32 * (small ? 1 : 2) * (threads / 64);
+	const int blocks  = (int) std::min<int64_t>(small ? 2048 : 2 * nrc->cus, (n + perBlock - 1) / perBlock);
+	hipLaunchKernelGGL((small ? k_infer<1, 256, 3> : k_infer<2, 512, 4>), dim3(blocks), dim3(threads), kFwdLdsElems * (int) sizeof(uint16_t), (hipStream_t) hip_stream,
+					   nrc->wt.as<uint16_t>(), (const float *) vertices_dev, n, radiance_dev);
 	NRC_HIP(hipGetLastError());
 	return KRR_OK;
 }

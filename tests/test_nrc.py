@@ -137,6 +137,28 @@ def test_gpu_inference_matches_reference(krr, gpu, rng, n):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n", [131072, 131073, 131072 + 63, 200001, 524288 + 33])
+def test_gpu_inference_of_many_samples(krr, gpu, rng, n):
+    """Above 2^17 samples a wave evaluates two tiles of 32 at a time: the same
+    products in the same order per sample, so each sample's radiance equals
+    that of a small call bit for bit."""
+    from kiraray_amd.nrc import NeuralRadianceCache
+    print(f"case: nrc infer n={n} against calls of 1000", flush=True)
+    nrc = NeuralRadianceCache({"seed": 5})
+    v = ref.random_vertices(n, rng)
+    vb, out, part = _dev(gpu, v), gpu.DeviceBuffer(n * 12), gpu.DeviceBuffer(1000 * 12)
+    nrc.infer(vb.ptr, n, out.ptr)
+    gpu.synchronize()
+    y = out.to_numpy(np.float32, (n, 3))
+    assert np.isfinite(y).all()
+    for first in (0, 4321, n // 2, n - 1000):  # slices of 1000 inside the n samples
+        nrc.infer(vb.ptr + first * 64, 1000, part.ptr)
+        gpu.synchronize()
+        assert np.array_equal(y[first:first + 1000], part.to_numpy(np.float32, (1000, 3)))
+    nrc.close()
+
+
+@pytest.mark.gpu
 def test_gpu_gradient_matches_reference(krr, gpu, rng):
     """Weight gradient and loss of the fused forward/backward + split-K
     kernels against the CPU FP64 backprop, per layer."""
