@@ -63,13 +63,13 @@ KRR_DEV void pathVertex(const PtArgs &A, const TravState &h, const f3 &d, Pcg &r
 		return;
 	}
 	SurfaceInteraction intr;
-	prepareSurfaceInteraction<TEX>(sc, h.prim, h.b1, h.b2, d, -1, intr);
+	surfaceAt<TEX>(sc, h.prim, h.b1, h.b2, d, -1, intr);
 	if (intr.light >= 0) { // handleHit (device.cu:52-65)
 		const DevLight Lr = sc.lights[intr.light];
 		const f3 Le		  = areaLightL<TEX>(Lr, intr.n, intr.wo, intr.u, intr.v);
 		float w			  = 1.f;
 		if (A.nee && p.depth > 0) {
-			const float lightPdf = lightPdfLi(sc, Lr, intr.p, intr.n, p.ctxP) * selPdf;
+			const float lightPdf = lightPdfLi(sc, intr.light, intr.p, intr.n, p.ctxP) * selPdf;
 			if (!(p.bsdfType & BSDF_SPECULAR)) w = misPower(p.pdf, lightPdf);
 			if (!finiteWeight(w)) w = 1.f;
 		}
@@ -85,7 +85,7 @@ KRR_DEV void pathVertex(const PtArgs &A, const TravState &h, const f3 &d, Pcg &r
 		const float ul		 = rng.get1D();
 		const int li		 = min((int) (uint32_t) (ul * (float) nL), nL - 1);
 		const float u0		 = rng.get1D(), u1 = rng.get1D();
-		const LightSample ls = sampleLi<TEX>(sc, sc.lights[li], u0, u1, intr.p);
+		const LightSample ls = sampleLi<TEX>(sc, li, u0, u1, intr.p);
 		const f3 wiL		 = intr.toLocal(normalize(ls.p - intr.p));
 		const float lightPdf = selPdf * ls.pdf;
 		if (lightPdf != 0.f) {

@@ -80,6 +80,48 @@ __global__ void k_begin_frame(WfParams P, PixelStateDev px) {
 	px.rng[i]			= s.state;
 }
 
+// The records of every triangle and light (kTriRec, kLightRec).
+__global__ void k_tri_records(DevScene sc, int64_t n, float4 *out) {
+	const int64_t i = blockIdx.x * (int64_t) blockDim.x + threadIdx.x;
+	if (i >= n) return;
+	const DevMesh m = sc.meshes[sc.triMesh[i]];
+	f3 p[3], nr[3];
+	for (int k = 0; k < 3; k++) {
+		const int v = sc.idx[3 * i + k];
+		p[k]		= loadV(sc.pos, v);
+		if (m.hasNormals) nr[k] = loadV(sc.nrm, v);
+	}
+	float4 *r	  = out + i * kTriRec;
+	const int light = m.lightBase >= 0 ? m.lightBase + ((int) i - m.firstTri) : -1;
+	r[0] = make_float4(p[0].x, p[0].y, p[0].z, __int_as_float(m.material));
+	r[1] = make_float4(p[1].x, p[1].y, p[1].z, __int_as_float(light));
+	r[2] = make_float4(p[2].x, p[2].y, p[2].z, __int_as_float(m.hasNormals));
+	r[3] = make_float4(nr[0].x, nr[0].y, nr[0].z, __int_as_float(m.mediumIn));
+	r[4] = make_float4(nr[1].x, nr[1].y, nr[1].z, __int_as_float(m.mediumOut));
+	r[5] = make_float4(nr[2].x, nr[2].y, nr[2].z, 0.f);
+}
+
+__global__ void k_light_records(DevScene sc, float4 *out) {
+	const int i = blockIdx.x * blockDim.x + threadIdx.x;
+	if (i >= sc.nLights || sc.lights[i].type != 0) return;
+	const int prim = sc.lights[i].prim;
+	f3 p[3], nr[3];
+	for (int k = 0; k < 3; k++) {
+		const int v = sc.idx[3 * prim + k];
+		p[k]		= loadV(sc.pos, v);
+		nr[k]		= loadV(sc.nrm, v); // emissive meshes have normals
+	}
+	const f3 ng = normalize(cross(p[1] - p[0], p[2] - p[0])), nn = normalize(ng);
+	float4 *r	= out + (size_t) i * kLightRec;
+	r[0] = make_float4(p[0].x, p[0].y, p[0].z, 1.f / triArea(sc, prim));
+	r[1] = make_float4(p[1].x, p[1].y, p[1].z, ng.x);
+	r[2] = make_float4(p[2].x, p[2].y, p[2].z, ng.y);
+	r[3] = make_float4(nr[0].x, nr[0].y, nr[0].z, ng.z);
+	r[4] = make_float4(nr[1].x, nr[1].y, nr[1].z, 0.f);
+	r[5] = make_float4(nr[2].x, nr[2].y, nr[2].z, 0.f);
+	r[6] = make_float4(nn.x, nn.y, nn.z, 0.f);
+}
+
 // generateCameraRays (integrator.cpp:166-179).  Camera rays go to slot =
 // pixelId, so the first trace sees image-coherent rays.
 __global__ void k_camera(WfParams P, CameraDev cam, PixelStateDev px, RayQueueDev q, Counters *cnt) {
@@ -386,7 +428,10 @@ KRR_DEV void shadeCore(const WfParams &P, const DevScene &sc, const RayItem &r, 
 	Pcg rng{pr.rng, P.inc};
 	const int channel = MEDIA ? pr.channel : 0;
 	f3 L			  = pr.L;
-	f3 thp = r.thp, pu = r.pu, pl = r.pl;
+	// Without media the path's unidirectional density stays 1 and its light
+	// density is the same in every channel: one value, not six, is carried
+	// from vertex to vertex.
+	f3 thp = r.thp, pu = MEDIA ? r.pu : f3(1.f), pl = MEDIA ? r.pl : f3(r.pl.x);
 	bool hasHL = false, hasScatter = false, hasMiss = false, hasMS = false, hasMSc = false;
 	SurfaceInteraction intr;
 	float msTmax   = __builtin_inff();
@@ -394,7 +439,7 @@ KRR_DEV void shadeCore(const WfParams &P, const DevScene &sc, const RayItem &r, 
 	f3 mscP, mscThp, mscPu, mscWo;
 	float mscG = 0.f;
 	if (prim >= 0) {
-		prepareSurfaceInteraction<!PLAIN>(sc, prim, h.z, h.w, r.d, r.medium, intr);
+		surfaceAt<!PLAIN>(sc, prim, h.z, h.w, r.d, r.medium, intr);
 		if (MEDIA && P.enableMedium && r.medium >= 0) {
 			hasMS	  = true;
 			msTmax	  = h.x;
@@ -483,7 +528,7 @@ KRR_DEV void shadeCore(const WfParams &P, const DevScene &sc, const RayItem &r, 
 		const DevLight Lr = sc.lights[intr.light];
 		f3 Le			  = areaLightL<!PLAIN>(Lr, intr.n, intr.wo, intr.u, intr.v) * thp;
 		if (P.nee && r.depth && !(r.bsdfType & BSDF_DELTA)) {
-			const float lightPdf = lightPdfLi(sc, Lr, intr.p, intr.n, r.cp) * lightSelectPdf;
+			const float lightPdf = lightPdfLi(sc, intr.light, intr.p, intr.n, r.cp) * lightSelectPdf;
 			Le					 = Le / (pl * lightPdf + pu).mean();
 		} else Le = Le / pu.mean();
 		L = L + Le;
@@ -541,7 +586,7 @@ KRR_DEV void shadeCore(const WfParams &P, const DevScene &sc, const RayItem &r, 
 				const float ul	 = rng.get1D();
 				const int li	 = min((int) (uint32_t) (ul * (float) sc.nLights), sc.nLights - 1);
 				const float u0	 = rng.get1D(), u1 = rng.get1D();
-				const LightSample ls = sampleLi<!PLAIN>(sc, sc.lights[li], u0, u1, mscP);
+				const LightSample ls = sampleLi<!PLAIN>(sc, li, u0, u1, mscP);
 				const f3 to		 = offsetRayOrigin(ls.p, ls.n, mscP - ls.p);
 				const f3 p_o	 = offsetRayOrigin(mscP, f3(), to - mscP);
 				const f3 sdir	 = to - p_o;
@@ -601,7 +646,7 @@ KRR_DEV void shadeCore(const WfParams &P, const DevScene &sc, const RayItem &r, 
 					const float ul		 = rng.get1D();
 					const int li		 = min((int) (uint32_t) (ul * (float) sc.nLights), sc.nLights - 1);
 					const float u0		 = rng.get1D(), u1 = rng.get1D();
-					const LightSample ls = sampleLi<!PLAIN>(sc, sc.lights[li], u0, u1, intr.p);
+					const LightSample ls = sampleLi<!PLAIN>(sc, li, u0, u1, intr.p);
 					const f3 to			 = offsetRayOrigin(ls.p, ls.n, intr.p - ls.p);
 					const f3 p_o		 = offsetRayOrigin(intr.p, intr.n, to - intr.p);
 					const f3 sdir		 = to - p_o;
@@ -724,7 +769,7 @@ KRR_DEV void transmittanceItem(const WfParams &P, const DevScene &sc, const Trac
 		const TraceResult h = traverse<false, COUNT, ALPHA>(bvh, o, d, tMax, stack, nv, nt);
 		const bool visible	= h.prim < 0;
 		// only a null-material surface lets the ray on, and it has no normal map
-		if (!visible) prepareSurfaceInteraction<false>(sc, h.prim, h.b1, h.b2, d, origMedium, intr);
+		if (!visible) prepareSurfaceRecord(sc, h.prim, h.b1, h.b2, d, origMedium, intr);
 		if (!visible && intr.material >= 0) {
 			T_ray = f3();
 			break;
@@ -1791,7 +1836,7 @@ struct krr_wf {
 	AccelData accel;
 	DevBuf pos, nrm, idx, triMesh, meshes, materials, lights, media;
 	std::vector<std::unique_ptr<DevBuf>> mediumBufs, imageBufs, textureBufs;
-	DevBuf uv, tan, textures;
+	DevBuf uv, tan, textures, triRec, lightRec;
 	DevScene ds{};
 	bool sceneHasMedia = false;
 	bool sceneTextured = false; // textures or image-lit infinite lights: the kernels with texture lookups
@@ -2168,6 +2213,15 @@ int uploadScene(krr_wf *wf, const krr_scene_desc *s) {
 		ds.bmin[a] = lo[a];
 		ds.binv[a] = hi[a] > lo[a] ? 1.f / (hi[a] - lo[a]) : 1.f;
 	}
+	KRR_HIP(wf->triRec.alloc((size_t) s->n_triangles * kTriRec * sizeof(float4)));
+	KRR_HIP(wf->lightRec.alloc(lights.size() * kLightRec * sizeof(float4)));
+	if (s->n_triangles > 0)
+		hipLaunchKernelGGL(k_tri_records, dim3((unsigned) ((s->n_triangles + 255) / 256)), dim3(256), 0, nullptr, ds, s->n_triangles, wf->triRec.as<float4>());
+	if (!lights.empty()) hipLaunchKernelGGL(k_light_records, dim3((unsigned) ((lights.size() + 63) / 64)), dim3(64), 0, nullptr, ds, wf->lightRec.as<float4>());
+	KRR_HIP(hipGetLastError());
+	KRR_HIP(hipDeviceSynchronize());
+	ds.tri		= wf->triRec.as<float4>();
+	ds.lightTri = wf->lightRec.as<float4>();
 	wf->sceneHasMedia = s->n_media > 0;
 	wf->sceneTextured = s->n_textures > 0 || wf->accel.alphaTri.p != nullptr;
 	for (int i = 0; i < s->n_meshes; i++) wf->sceneTextured |= s->meshes[i].has_tangents != 0;
