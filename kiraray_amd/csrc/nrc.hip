@@ -13,9 +13,10 @@
 // the next layer, so activations never leave the registers between layers.
 // Pairs of k-steps run as one v_mfma_f32_32x32x16_bf16.  Backward uses the
 // same layout with A = W (dX^T = W dZ^T).  Weight gradients
-// dW_l = X_l dZ_l^T are a split-K GEMM over the batch on X^T and dZ^T stored
-// feature-major in HBM, reduced in a fixed order (deterministic), then Adam
-// updates the FP32 master weights and rewrites both BF16 copies.
+// dW_l = X_l dZ_l^T are summed over the batch in the same launch, on operands
+// transposed through LDS; the blocks' sums are reduced in a fixed order
+// (deterministic), then Adam updates the FP32 master weights and rewrites both
+// BF16 copies.
 //
 // Encoding (64 features, lane half g = 0/1 computes slots q = 4s + j of
 // feature 8s + 4g + j):
@@ -52,13 +53,13 @@ namespace nrc {
 __device__ __forceinline__ uint16_t toBf16(float f) { return __builtin_bit_cast(uint16_t, (__bf16) f); }
 __device__ __forceinline__ float fromBf16(uint16_t h) { return __uint_as_float((uint32_t) h << 16); }
 
+// Two values with one conversion (left to itself the compiler converts them one
+// by one and joins the halves).
+typedef float float2v __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2v __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t pack2(float a, float b) { return __builtin_bit_cast(uint32_t, __builtin_convertvector((float2v){a, b}, bf16x2v)); }
 __device__ __forceinline__ short4v pack4(float a, float b, float c, float d) {
-	short4v v;
-	v[0] = (short) toBf16(a);
-	v[1] = (short) toBf16(b);
-	v[2] = (short) toBf16(c);
-	v[3] = (short) toBf16(d);
-	return v;
+	return __builtin_bit_cast(short4v, (uint64_t) pack2(c, d) << 32 | pack2(a, b));
 }
 
 // The encoding uses the hardware exp2 / sine / cosine (a learned input needs
@@ -133,85 +134,61 @@ __device__ __forceinline__ float16v zero16() {
 // FP32 order of the additions inside the instruction differs.  Half the
 // instructions of the 32x32x8 form, each at the same rate.
 typedef __bf16 bf16x8v __attribute__((ext_vector_type(8)));
-typedef short short8v __attribute__((ext_vector_type(8)));
-__device__ __forceinline__ float16v mfma2(short4v a0, short4v a1, short4v b0, short4v b1, float16v c) {
-	const short8v a = __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7);
-	const short8v b = __builtin_shufflevector(b0, b1, 0, 1, 2, 3, 4, 5, 6, 7);
+__device__ __forceinline__ short8v join(short4v a, short4v b) { return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7); }
+__device__ __forceinline__ float16v mfma2(short8v a, short4v b0, short4v b1, float16v c) {
+	const short8v b = join(b0, b1);
 	return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8v, a), __builtin_bit_cast(bf16x8v, b), c, 0, 0, 0);
 }
 
-// A operand: 4 consecutive bf16 at row `row` (rows `stride` bf16 apart), column 8s + 4g.
-__device__ __forceinline__ short4v ldsA(const uint16_t *m, int row, int s, int g, int stride = kRowH) {
-	return *reinterpret_cast<const short4v *>(m + row * stride + 8 * s + 4 * g);
+// A lane's operand pair `pair` of a weight copy (in LDS or in memory).
+__device__ __forceinline__ short8v weightPair(const uint16_t *w, int pair, int lane) {
+	return *reinterpret_cast<const short8v *>(w + pair * 512 + lane * 8);
+}
+
+// ReLU of both row halves' accumulators, rounded to bf16 (B layout).
+__device__ __forceinline__ void reluPack(const float16v &a0, const float16v &a1, short4v out[8]) {
+#pragma unroll
+	for (int s = 0; s < 4; s++) {
+		out[s]	   = pack4(fmaxf(a0[4 * s], 0.f), fmaxf(a0[4 * s + 1], 0.f), fmaxf(a0[4 * s + 2], 0.f), fmaxf(a0[4 * s + 3], 0.f));
+		out[4 + s] = pack4(fmaxf(a1[4 * s], 0.f), fmaxf(a1[4 * s + 1], 0.f), fmaxf(a1[4 * s + 2], 0.f), fmaxf(a1[4 * s + 3], 0.f));
+	}
 }
 
 // One hidden layer, forward: out (B layout, relu, bf16) = W^T x.
-__device__ __forceinline__ void hiddenForward(const uint16_t *wt, int lane, int g, const short4v x[8], short4v out[8], float16v &acc0,
-											  float16v &acc1) {
-	acc0 = zero16();
-	acc1 = zero16();
-	const int r0 = lane & 31;
-#pragma unroll
-	for (int s = 0; s < 8; s += 2) {
-		acc0 = mfma2(ldsA(wt, r0, s, g), ldsA(wt, r0, s + 1, g), x[s], x[s + 1], acc0);
-		acc1 = mfma2(ldsA(wt, 32 + r0, s, g), ldsA(wt, 32 + r0, s + 1, g), x[s], x[s + 1], acc1);
-	}
+__device__ __forceinline__ void hiddenForward(const uint16_t *wt, int lane, const short4v x[8], short4v out[8]) {
+	float16v acc0 = zero16(), acc1 = zero16();
 #pragma unroll
 	for (int s = 0; s < 4; s++) {
-		out[s]	   = pack4(fmaxf(acc0[4 * s], 0.f), fmaxf(acc0[4 * s + 1], 0.f), fmaxf(acc0[4 * s + 2], 0.f), fmaxf(acc0[4 * s + 3], 0.f));
-		out[4 + s] = pack4(fmaxf(acc1[4 * s], 0.f), fmaxf(acc1[4 * s + 1], 0.f), fmaxf(acc1[4 * s + 2], 0.f), fmaxf(acc1[4 * s + 3], 0.f));
+		acc0 = mfma2(weightPair(wt, s, lane), x[2 * s], x[2 * s + 1], acc0);
+		acc1 = mfma2(weightPair(wt, 4 + s, lane), x[2 * s], x[2 * s + 1], acc1);
 	}
+	reluPack(acc0, acc1, out);
 }
 
 // Output layer forward: y_c (c < 3) lands in acc[c] of lanes with g == 0.
-__device__ __forceinline__ float16v outputForward(const uint16_t *wt5, int lane, int g, const short4v x[8]) {
+__device__ __forceinline__ float16v outputForward(const uint16_t *wt5, int lane, const short4v x[8]) {
 	float16v acc = zero16();
-	const int r0 = lane & 31;
 #pragma unroll
-	for (int s = 0; s < 8; s += 2) acc = mfma2(ldsA(wt5, r0, s, g), ldsA(wt5, r0, s + 1, g), x[s], x[s + 1], acc);
+	for (int s = 0; s < 4; s++) acc = mfma2(weightPair(wt5, s, lane), x[2 * s], x[2 * s + 1], acc);
 	return acc;
 }
 
-// Copies `rows` dense rows of rowLen bf16 into LDS rows of rowLen + kPad.
-// Each thread issues up to twelve 16-byte loads before it stores them (two
-// 8-byte LDS writes each: padded rows are 8-byte aligned), so a block of 256
-// threads fetches one copy of all layers' weights (~48 KB) in one round trip.  One
-// load per store would put a memory round trip between consecutive loads,
-// and the training kernel runs one wave per SIMD with nothing to hide it.
-__device__ void loadRows(uint16_t *lds, const uint16_t *src, int rows, int rowLen) {
-	constexpr int kBatch = 12;
-	const int per = rowLen / 8; // 16-byte pieces per row
-	const int total = rows * per, stride = (int) blockDim.x;
-	for (int base = (int) threadIdx.x; base < total; base += kBatch * stride) {
-		uint4 v[kBatch];
+// Forward weights into LDS as they are.  Each thread issues up to twelve
+// 16-byte loads before it stores them, so a block of 256 threads fetches all
+// layers' weights (44 KB) in one round trip; one load per store would put a
+// memory round trip between consecutive loads.
+__device__ void loadWeights(uint16_t *lds, const uint16_t *wtAll) {
+	constexpr int batch = 12, total = kFwdElems / 8;
+	const uint4 *src = reinterpret_cast<const uint4 *>(wtAll);
+	const int stride = (int) blockDim.x;
+	for (int base = (int) threadIdx.x; base < total; base += batch * stride) {
+		uint4 v[batch];
 #pragma unroll
-		for (int k = 0; k < kBatch; k++) {
-			const int i = base + k * stride;
-			if (i < total) {
-				const int r = i / per, c = i - r * per;
-				v[k]		= *reinterpret_cast<const uint4 *>(src + r * rowLen + 8 * c);
-			}
-		}
+		for (int k = 0; k < batch; k++) v[k] = src[min(base + k * stride, total - 1)];
 #pragma unroll
-		for (int k = 0; k < kBatch; k++) {
-			const int i = base + k * stride;
-			if (i < total) {
-				const int r = i / per, c = i - r * per;
-				uint2 *d = reinterpret_cast<uint2 *>(lds + r * (rowLen + kPad) + 8 * c);
-				d[0]	 = make_uint2(v[k].x, v[k].y);
-				d[1]	 = make_uint2(v[k].z, v[k].w);
-			}
-		}
+		for (int k = 0; k < batch; k++)
+			if (base + k * stride < total) reinterpret_cast<uint4 *>(lds)[base + k * stride] = v[k];
 	}
-}
-
-// Forward weights (W^T of every layer, output rows padded to 32) into LDS.
-__device__ void loadWeights(uint16_t *lds, const uint16_t *wtAll) { loadRows(lds, wtAll, kHidden * 64 + 32, 64); }
-
-// Backward weights (W of every layer, output columns padded to 32) into LDS.
-__device__ void loadWeightsBwd(uint16_t *lds, const uint16_t *wbAll) {
-	loadRows(lds, wbAll, kHidden * 64, 64);
-	loadRows(lds + kHidden * 64 * kRowH, wbAll + kHidden * 4096, 64, 32);
 }
 
 // ----------------------------------------------------------------- kernels
@@ -270,30 +247,25 @@ __global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WA
 		// not unrolled: an unrolled loop hoists every layer's weight loads
 #pragma unroll 1
 		for (int l = 0; l < kHidden; l++) {
-			const uint16_t *wt = ldsW + l * 64 * kRowH;
+			const uint16_t *wt = ldsW + l * 4096;
 			float16v a0[T], a1[T];
 #pragma unroll
 			for (int k = 0; k < T; k++) a0[k] = a1[k] = zero16();
 #pragma unroll
-			for (int s = 0; s < 8; s += 2) {
-				const short4v w00 = ldsA(wt, m, s, g), w01 = ldsA(wt, m, s + 1, g), w10 = ldsA(wt, 32 + m, s, g), w11 = ldsA(wt, 32 + m, s + 1, g);
+			for (int s = 0; s < 4; s++) {
+				const short8v w0 = weightPair(wt, s, lane), w1 = weightPair(wt, 4 + s, lane);
 #pragma unroll
 				for (int k = 0; k < T; k++) {
-					a0[k] = mfma2(w00, w01, x[k][s], x[k][s + 1], a0[k]);
-					a1[k] = mfma2(w10, w11, x[k][s], x[k][s + 1], a1[k]);
+					a0[k] = mfma2(w0, x[k][2 * s], x[k][2 * s + 1], a0[k]);
+					a1[k] = mfma2(w1, x[k][2 * s], x[k][2 * s + 1], a1[k]);
 				}
 			}
 #pragma unroll
-			for (int k = 0; k < T; k++)
-#pragma unroll
-				for (int s = 0; s < 4; s++) {
-					x[k][s]		= pack4(fmaxf(a0[k][4 * s], 0.f), fmaxf(a0[k][4 * s + 1], 0.f), fmaxf(a0[k][4 * s + 2], 0.f), fmaxf(a0[k][4 * s + 3], 0.f));
-					x[k][4 + s] = pack4(fmaxf(a1[k][4 * s], 0.f), fmaxf(a1[k][4 * s + 1], 0.f), fmaxf(a1[k][4 * s + 2], 0.f), fmaxf(a1[k][4 * s + 3], 0.f));
-				}
+			for (int k = 0; k < T; k++) reluPack(a0[k], a1[k], x[k]);
 		}
 #pragma unroll
 		for (int k = 0; k < T; k++) {
-			const float16v o = outputForward(ldsW + kHidden * 64 * kRowH, lane, g, x[k]);
+			const float16v o = outputForward(ldsW + kHidden * 4096, lane, x[k]);
 			const int64_t i	 = (t * T + k) * 32 + m;
 			if (g == 0 && i < n) {
 				radiance[3 * i]		= o[0];
@@ -305,7 +277,7 @@ __global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WA
 }
 
 // Threads per k_infer_queue block: the block's waves share one LDS copy of
-// the weights (52 KB), which limits a CU to 3 copies; blocks of 8 waves,
+// the weights (44 KB), which limits a CU to 3 copies; blocks of 8 waves,
 // compiled for 5 waves per SIMD (96 VGPRs, 20 B of spills), run 5 waves per SIMD
 // where blocks of 4 ran 3.  On the 1080p field (0.36 M queries per launch):
 // 27.8 us per launch against 32.4 us; 6 waves per SIMD (80 VGPRs, 84 B of
@@ -362,15 +334,14 @@ __global__ void __launch_bounds__(kInferBlock) __attribute__((amdgpu_waves_per_e
 		short4v x[8], y[8];
 		encodeB(v, g, x);
 		loadQuery(queries, stride, (t + tStride) * 32 + m, n, v, pay); // the next tile's queries
-		float16v a0, a1;
 		// not unrolled: an unrolled loop hoists every layer's weight loads
 #pragma unroll 1
 		for (int l = 0; l < kHidden; l++) {
-			hiddenForward(ldsW + l * 64 * kRowH, lane, g, x, y, a0, a1);
+			hiddenForward(ldsW + l * 4096, lane, x, y);
 #pragma unroll
 			for (int s = 0; s < 8; s++) x[s] = y[s];
 		}
-		const float16v o = outputForward(ldsW + kHidden * 64 * kRowH, lane, g, x);
+		const float16v o = outputForward(ldsW + kHidden * 4096, lane, x);
 		if (mine) {
 			acc.x += thp.x * fmaxf(o[0], 0.f);
 			acc.y += thp.y * fmaxf(o[1], 0.f);
@@ -380,111 +351,193 @@ __global__ void __launch_bounds__(kInferBlock) __attribute__((amdgpu_waves_per_e
 	}
 }
 
-// Writes the B-layout bf16 operand (features 8s + 4g + j of sample m) to a
-// feature-major [feature][ld] array at column `col` (`dst` is a layer's
-// 64 x ld block).  Buffer stores: the lane's column offset is computed once
-// and the feature row's offset, (8s + j) ld, is wave-uniform (soffset), so a
-// store takes no per-lane address arithmetic; stores past the block are
-// dropped by the buffer's range check.  The rows of features >= `features`
-// (s >= features / 8, for every g) are not written.
-__device__ __forceinline__ void storeFeatureMajor(uint16_t *dst, int64_t ld, int64_t col, int g, const short4v x[8], int features = 64) {
-	// ld <= 2^24 (max_batch): the largest row offset, 63 ld bf16, stays below
-	// 2^31 bytes; the range, 64 ld bf16 <= 2^31 bytes, is read as unsigned
-	const int ld32 = (int) ld;
-	const uint32_t range = 64u * (uint32_t) ld32 * (uint32_t) sizeof(uint16_t);
-	const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(dst, (short) 0, (int) range, 0x00020000);
-	const int voff = (4 * g * ld32 + (int) col) * (int) sizeof(uint16_t);
+// Training works on groups of 128 samples: a block of four waves, one tile of
+// 32 samples each.
+constexpr int kTrainBlock = 256;
+constexpr int kGroup	  = 128;
+constexpr int kTileElems  = 32 * 64; // a tile's layer input or output gradient in LDS, sample-major
+
+// A mini-batch: `n` samples, or with a device count, the step-th of `steps`
+// equal slices of the first min(*nDev, capTotal) samples (at most n).
+struct Batch {
+	int64_t n;
+	const int *nDev;
+	int64_t capTotal;
+	int step, steps;
+	__device__ int64_t range(int64_t &off) const {
+		off = 0;
+		if (!nDev) return n;
+		const int64_t cnt = min((int64_t) max(*nDev, 0), capTotal);
+		off				  = (int64_t) step * cnt / steps;
+		return min((int64_t) (step + 1) * cnt / steps - off, n);
+	}
+};
+
+// A tile in LDS: row m = sample, sixteen 8-byte chunks of 4 features.  Rows
+// are 128 bytes, so chunks are permuted by the row: the 64 lanes that write
+// one chunk pair of 32 rows, and the 64 lanes that read 8 rows of 8 chunks, each
+// spread evenly over the banks.
+__device__ __forceinline__ int tileChunk(int m, int c) { return m * 64 + 4 * (c ^ ((((m >> 1) & 1) << 3) | (m >> 2))); }
+
+// The tile transposed, as an operand whose rows are features f0 + (lane & 31)
+// and whose K-step s holds samples 8s + 4g + j: of each 16 lanes, lane i reads
+// the chunk of 4 features i % 4 of row i / 4 and receives feature i of the 4 rows.
+__device__ __forceinline__ int tileRead(int lane, int f0, int s) {
+	return tileChunk(8 * s + 4 * (lane >> 5) + ((lane & 15) >> 2), f0 / 4 + 4 * ((lane >> 4) & 1) + (lane & 3));
+}
+typedef __attribute__((address_space(3))) short4v *LdsShort4;
+__device__ __forceinline__ short4v tileT(const uint16_t *p) { return __builtin_amdgcn_ds_read_tr16_b64_v4i16((LdsShort4) p); }
+
+// The A operands of a layer's two 32-row halves (`pairs` pairs of K-steps
+// each), read ahead of the products that use them.
+struct Rows {
+	short8v w[8];
+	__device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t copy, int first, int pairs, int lane) {
 #pragma unroll
-	for (int s = 0; s < 8; s++)
+		for (int k = 0; k < 2 * pairs; k++)
+			w[k] = __builtin_bit_cast(short8v, __builtin_amdgcn_raw_buffer_load_b128(copy, lane * 16, (first + k * 512) * (int) sizeof(uint16_t), 0));
+	}
+	__device__ __forceinline__ void multiply(const short4v x[8], int pairs, float16v &a0, float16v &a1) const {
+		a0 = zero16();
+		a1 = zero16();
 #pragma unroll
-		for (int j = 0; j < 4; j++)
-			if (8 * s < features) __builtin_amdgcn_raw_buffer_store_b16((unsigned short) x[s][j], rsrc, voff, (8 * s + j) * ld32 * (int) sizeof(uint16_t), 0);
+		for (int s = 0; s < pairs; s++) {
+			a0 = mfma2(w[s], x[2 * s], x[2 * s + 1], a0);
+			a1 = mfma2(w[pairs + s], x[2 * s], x[2 * s + 1], a1);
+		}
+	}
+};
+
+// The transposed X and dZ operands of one tile.
+struct TileRead {
+	short4v x[4], z[4];
+	__device__ __forceinline__ void load(const uint16_t *const getX[4], const uint16_t *const getZ[4], int offset) {
+#pragma unroll
+		for (int s = 0; s < 4; s++) {
+			x[s] = tileT(getX[s] + offset);
+			z[s] = tileT(getZ[s] + offset);
+		}
+	}
+	__device__ __forceinline__ void multiply(float16v &acc) const {
+#pragma unroll
+		for (int s = 0; s < 4; s += 2) acc = mfma2(join(x[s], x[s + 1]), z[s], z[s + 1], acc);
+	}
+};
+
+// (a, b, c, d) where x > 0, else 0, as the next B operand's four features; x is
+// a ReLU's output (zero of either sign, or positive), so a 16-bit half of it
+// is zero but for the sign exactly where adding 0x7fff leaves the top bit clear.
+__device__ __forceinline__ uint32_t positiveMask(uint32_t x) {
+	const uint32_t top = ((x & 0x7fff7fffu) + 0x7fff7fffu) & 0x80008000u;
+	return (top - (top >> 15)) | top;
+}
+__device__ __forceinline__ short4v maskedPack(const short4v x, float a, float b, float c, float d) {
+	const uint64_t bits = __builtin_bit_cast(uint64_t, x);
+	const uint32_t lo = pack2(a, b) & positiveMask((uint32_t) bits), hi = pack2(c, d) & positiveMask((uint32_t) (bits >> 32));
+	return __builtin_bit_cast(short4v, (uint64_t) hi << 32 | lo);
 }
 
-// Forward + backward of one tile of 32 samples per wave.  Writes X_l^T and
-// dZ_l^T (bf16, feature-major, leading dimension ld = padded batch) and the
-// tile's loss sum.  Samples i >= n contribute nothing.
-template <bool BWD_LDS>
-__global__ void __launch_bounds__(256) k_train_tile(const uint16_t *wtAll, const uint16_t *wAll, const float *vertices, const float *targets,
-													int64_t nHost, const int *nDev, int64_t capTotal, int step, int steps, int64_t nTiles,
-													int64_t ld, float lossEps, uint16_t *xT, uint16_t *dzT, float *tileLoss, int *adamStep) {
+// A lane's LDS offset the compiler takes as it is: the offsets of layers and
+// tiles then stay immediates of the accesses (below 64 KB from this base),
+// where folding the base in would take a register for each of them.
+__device__ __forceinline__ int laneOffset(int elems) {
+	asm("" : "+v"(elems));
+	return elems;
+}
+
+// Forward, backward and weight gradients of one mini-batch; block b takes the
+// groups b, b + gridDim.x, ... and writes its sum of every weight's gradient
+// to partial[layer][b] (read by k_reduce; blocks without a group write
+// nothing).  Samples i >= n contribute nothing.
+//
+// Bound by latency: a mini-batch of 16384 samples is half a block per CU, one
+// wave per SIMD, a chain of 12 products and 6 barriers with vector work in
+// between (about 720 cycles per layer forward and 1900 backward, of which the
+// matrix cores are busy 512 and 768).  So every layer's input stays in
+// registers, a layer's weight gradient is taken while its X and dZ are here
+// (their transposed operands come from LDS by the transposing read), nothing
+// but the partial sums goes to memory, and operands are read ahead of the
+// products that use them.  16384 samples 16.3 us and k_reduce 6.1 us, where
+// X^T and dZ^T stored for a split-K product in a launch of its own took
+// 23 + 18 + 7 us; four training steps with weights set and read back 192
+// against 350 us.  Weights through LDS: 18 us; without the reads ahead 22 us.
+__global__ void __launch_bounds__(kTrainBlock) __attribute__((amdgpu_waves_per_eu(1, 1)))
+k_train(const uint16_t *wtAll, const uint16_t *wAll, const float *vertices, const float *targets, Batch batch, float lossEps, float *partialAll,
+		float *tileLoss, int *adamStep) {
 	// a training step (not a bare gradient) counts Adam's step here: the
-	// kernels after this one in the stream read the new count
+	// kernel after this one in the stream reads the new count
 	if (adamStep && blockIdx.x == 0 && threadIdx.x == 0) *adamStep += 1;
-	// samples: nHost, or with a device count, the step-th of `steps` equal
-	// slices of the first min(*nDev, capTotal) samples
-	int64_t n = nHost;
-	if (nDev) {
-		const int64_t cnt = min((int64_t) max(*nDev, 0), capTotal);
-		const int64_t off = (int64_t) step * cnt / steps;
-		n				  = min((int64_t) (step + 1) * cnt / steps - off, nHost);
-		vertices += off * 16;
-		targets += off * 3;
+	int64_t off;
+	const int64_t n = batch.range(off), groups = (n + kGroup - 1) / kGroup;
+	if (blockIdx.x >= groups) return;
+	vertices += off * 16;
+	targets += off * 3;
+	__shared__ __attribute__((aligned(16))) uint16_t lds[2 * 8 * kTileElems];
+	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 5, m = lane & 31;
+	const int kt = 32 * (wave >> 1), nt = 32 * (wave & 1); // this wave's 32x32 tile of each weight gradient
+	const float invCount = 1.0f / (3.0f * (float) n);
+
+	float v[16], tg[3];
+	auto fetch = [&](int64_t group) {
+		const int64_t i = group * kGroup + 32 * wave + m;
+		loadVertex(vertices, i, n, v);
+#pragma unroll
+		for (int c = 0; c < 3; c++) tg[c] = g == 0 && i < n ? targets[3 * i + c] : 0.f;
+	};
+	fetch(blockIdx.x);
+	// A layer's weights come straight from memory (the copies are in operand
+	// order: each read is one kilobyte, and the block's waves share the lines)
+	// two layers ahead of the products; LDS, which the transposition keeps busy,
+	// would have to carry them twice more.
+	// (Buffer loads: one register of address for all of them.)
+	const __amdgpu_buffer_rsrc_t fwd = __builtin_amdgcn_make_buffer_rsrc((void *) wtAll, (short) 0, kFwdElems * (int) sizeof(uint16_t), 0x00020000);
+	const __amdgpu_buffer_rsrc_t bwd = __builtin_amdgcn_make_buffer_rsrc((void *) wAll, (short) 0, kBwdElems * (int) sizeof(uint16_t), 0x00020000);
+	Rows w[3];
+	w[0].load(fwd, 0, 4, lane);
+	w[1].load(fwd, 4096, 4, lane);
+
+	// this lane's chunks of its wave's tile, its reads of the transposed tiles
+	constexpr int buffer = 8 * kTileElems; // four X tiles, then four dZ tiles
+	uint16_t *put[8];
+	const uint16_t *getX[4], *getZ[4];
+#pragma unroll
+	for (int s = 0; s < 8; s++) put[s] = lds + laneOffset(wave * kTileElems + tileChunk(m, 2 * s + g));
+#pragma unroll
+	for (int s = 0; s < 4; s++) {
+		getX[s] = lds + laneOffset(tileRead(lane, kt, s));
+		getZ[s] = lds + laneOffset(4 * kTileElems + tileRead(lane, nt, s));
 	}
-	// A operands from LDS; with BWD_LDS false (a device whose blocks cannot
-	// hold both copies) the backward ones come straight from global memory
-	// (45 KB, cache resident), unpadded
-	extern __shared__ uint16_t lds[];
-	uint16_t *ldsWt = lds;
-	loadWeights(ldsWt, wtAll);
-	const uint16_t *ldsW = wAll;
-	constexpr int sH = BWD_LDS ? kRowH : 64, sO = BWD_LDS ? kRowO : 32;
-	if (BWD_LDS) {
-		loadWeightsBwd(lds + kFwdLdsElems, wAll);
-		ldsW = lds + kFwdLdsElems;
-	}
-	__syncthreads();
-	const int lane = threadIdx.x & 63, g = lane >> 5, m = lane & 31;
-	const int wavesPerBlock = blockDim.x >> 6;
-	const float invCount	= n > 0 ? 1.0f / (3.0f * (float) n) : 0.f;
-	for (int64_t t = (int64_t) blockIdx.x * wavesPerBlock + (threadIdx.x >> 6); t < nTiles; t += (int64_t) gridDim.x * wavesPerBlock) {
-		const int64_t i	  = t * 32 + m;
+
+	float16v dW[kHidden + 1];
+#pragma unroll
+	for (int l = 0; l <= kHidden; l++) dW[l] = zero16();
+	for (int64_t group = blockIdx.x; group < groups; group += gridDim.x) {
+		const int64_t i	 = group * kGroup + 32 * wave + m;
 		const bool valid = i < n;
-		float v[16];
-		float tg[3] = {0.f, 0.f, 0.f}; // loaded with the inputs: the loss needs them after the forward pass
-		if (valid && g == 0) {
-#pragma unroll
-			for (int c = 0; c < 3; c++) tg[c] = targets[3 * i + c];
-		}
-		if (valid) {
-			const float4 *p = reinterpret_cast<const float4 *>(vertices + i * 16);
-#pragma unroll
-			for (int q = 0; q < 4; q++) {
-				const float4 f = p[q];
-				v[4 * q]	   = f.x;
-				v[4 * q + 1]   = f.y;
-				v[4 * q + 2]   = f.z;
-				v[4 * q + 3]   = f.w;
-			}
-		} else {
-#pragma unroll
-			for (int q = 0; q < 16; q++) v[q] = 0.f;
-		}
-		// forward: each layer input goes to X^T as it is produced; the
-		// backward pass needs only its ReLU mask, one bit per held feature
-		// (bit 4s + j of mask[l] <=> feature 8s + 4g + j of x_l is > 0)
-		short4v x[8], y[8];
-		uint32_t mask[kHidden + 1];
-		encodeB(v, g, x);
+		short4v x[kHidden + 1][8];
+		encodeB(v, g, x[0]);
+		// (the barriers keep the scheduler from moving reads back to their use)
 		float16v a0, a1;
-#pragma unroll 1
+#pragma unroll
 		for (int l = 0; l < kHidden; l++) {
-			storeFeatureMajor(xT + (int64_t) l * 64 * ld, ld, i, g, x);
-			hiddenForward(ldsWt + l * 64 * kRowH, lane, g, x, y, a0, a1);
-			uint32_t mk = 0;
-#pragma unroll
-			for (int s = 0; s < 8; s++) {
-				x[s] = y[s];
-#pragma unroll
-				for (int j = 0; j < 4; j++) mk |= (fromBf16((uint16_t) y[s][j]) > 0.f ? 1u : 0u) << (4 * s + j);
-			}
-			mask[l + 1] = mk;
+			if (l + 2 < kHidden) w[(l + 2) % 3].load(fwd, (l + 2) * 4096, 4, lane);
+			if (l + 2 == kHidden) w[(l + 2) % 3].load(fwd, (l + 2) * 4096, 2, lane); // four pairs of one half
+			if (l + 2 == kHidden + 1) w[(l + 2) % 3].load(bwd, kHidden * 4096, 2, lane);
+			__builtin_amdgcn_sched_barrier(0);
+			w[l % 3].multiply(x[l], 4, a0, a1);
+			reluPack(a0, a1, x[l + 1]);
+			__builtin_amdgcn_sched_barrier(0);
 		}
-		storeFeatureMajor(xT + (int64_t) kHidden * 64 * ld, ld, i, g, x);
-		const float16v o = outputForward(ldsWt + kHidden * 64 * kRowH, lane, g, x);
+		// from here layer l's backward weights are in w[(2 kHidden + 1 - l) % 3]
+		w[(kHidden + 2) % 3].load(bwd, (kHidden - 1) * 4096, 4, lane);
+		__builtin_amdgcn_sched_barrier(0);
+		// output c < 3 lands in o[c] of lanes with g == 0
+		float16v o = zero16();
+#pragma unroll
+		for (int s = 0; s < 4; s++) o = mfma2(w[kHidden % 3].w[s], x[kHidden][2 * s], x[kHidden][2 * s + 1], o);
 		// relative L2 loss and its gradient (lanes g == 0 hold the 3 outputs)
-		float d[3]	 = {0.f, 0.f, 0.f};
-		float lsum	 = 0.f;
+		float d[3] = {0.f, 0.f, 0.f};
+		float lsum = 0.f;
 		if (g == 0 && valid) {
 #pragma unroll
 			for (int c = 0; c < 3; c++) {
@@ -494,110 +547,64 @@ __global__ void __launch_bounds__(256) k_train_tile(const uint16_t *wtAll, const
 				d[c] = 2.0f * r / den * invCount;
 			}
 		}
-		// wave sum of the loss
-		for (int off = 32; off > 0; off >>= 1) lsum += __shfl_xor(lsum, off);
-		if (lane == 0) tileLoss[t] = lsum * invCount;
-		// dZ_5 as a B operand: outputs n = 8s + 4g + j, only n < 3 nonzero
+		if (group + gridDim.x < groups) fetch(group + gridDim.x);
+		// dZ of the output layer as a B operand: outputs 8s + 4g + j, only the
+		// first 3 nonzero, of 32 padded ones
 		short4v dz[8];
 #pragma unroll
-		for (int s = 0; s < 8; s++) dz[s] = pack4(0.f, 0.f, 0.f, 0.f);
+		for (int s = 0; s < 4; s++) dz[s] = pack4(0.f, 0.f, 0.f, 0.f);
 		if (g == 0) dz[0] = pack4(d[0], d[1], d[2], 0.f);
-		storeFeatureMajor(dzT + (int64_t) kHidden * 64 * ld, ld, i, g, dz, 32); // 32 padded output rows
-		// backward through the output layer: dX_5^T = W_5 dZ_5^T (K = 32 padded outputs)
-		const int r0 = lane & 31;
-		{
-			const uint16_t *w5 = ldsW + kHidden * 64 * sH;
-			a0 = zero16();
-			a1 = zero16();
 #pragma unroll
-			for (int s = 0; s < 4; s += 2) {
-				a0 = mfma2(ldsA(w5, r0, s, g, sO), ldsA(w5, r0, s + 1, g, sO), dz[s], dz[s + 1], a0);
-				a1 = mfma2(ldsA(w5, 32 + r0, s, g, sO), ldsA(w5, 32 + r0, s + 1, g, sO), dz[s], dz[s + 1], a1);
+		for (int l = kHidden; l >= 0; l--) {
+			// the other buffer was last read before the barrier of layer l + 1
+			const int buf = (l & 1) * buffer;
+#pragma unroll
+			for (int s = 0; s < 8; s++) {
+				*reinterpret_cast<short4v *>(put[s] + buf) = x[l][s];
+				if (s < 4 || l < kHidden) *reinterpret_cast<short4v *>(put[s] + buf + 4 * kTileElems) = dz[s];
 			}
-		}
-#pragma unroll 1
-		for (int l = kHidden - 1; l >= 0; l--) {
-			// dZ_l = dX_{l+1} * (x_{l+1} > 0), as the next B operand
-			const uint32_t mk = mask[l + 1];
-#pragma unroll
-			for (int s = 0; s < 4; s++)
-#pragma unroll
-				for (int j = 0; j < 4; j++) {
-					dz[s][j]	 = (short) toBf16((mk >> (4 * s + j)) & 1u ? a0[4 * s + j] : 0.f);
-					dz[4 + s][j] = (short) toBf16((mk >> (16 + 4 * s + j)) & 1u ? a1[4 * s + j] : 0.f);
-				}
-			storeFeatureMajor(dzT + (int64_t) l * 64 * ld, ld, i, g, dz);
+			__syncthreads();
+			// dX_l^T = W_l dZ_l^T, and dW_l = X_l^T dZ_l over the block's 128 samples
+			// (a 32x32 tile per wave; of the output layer only 3 columns are kept)
+			TileRead t[4];
+			t[0].load(getX, getZ, buf);
+			t[1].load(getX, getZ, buf + kTileElems);
+			__builtin_amdgcn_sched_barrier(0);
+			if (l > 0) w[(2 * kHidden + 1 - l) % 3].multiply(dz, l == kHidden ? 2 : 4, a0, a1);
+			t[2].load(getX, getZ, buf + 2 * kTileElems);
+			t[3].load(getX, getZ, buf + 3 * kTileElems);
+			__builtin_amdgcn_sched_barrier(0);
+			t[0].multiply(dW[l]);
+			t[1].multiply(dW[l]);
+			if (l > 2) w[(2 * kHidden + 3 - l) % 3].load(bwd, (l - 2) * 4096, 4, lane);
+			if (l < 2) w[1 - l].load(fwd, (1 - l) * 4096, 4, lane); // the next group's first layers
+			__builtin_amdgcn_sched_barrier(0);
+			t[2].multiply(dW[l]);
+			t[3].multiply(dW[l]);
+			if (l == 0) { // the wave's sum of the loss, here where nothing waits for it
+				for (int k = 32; k > 0; k >>= 1) lsum += __shfl_xor(lsum, k);
+				if (lane == 0) tileLoss[group * (kGroup / 32) + wave] = lsum * invCount;
+			}
+			// masked by x_l > 0, the next dZ
 			if (l > 0) {
-				const uint16_t *w = ldsW + l * 64 * sH;
-				a0				  = zero16();
-				a1				  = zero16();
 #pragma unroll
-				for (int s = 0; s < 8; s += 2) {
-					a0 = mfma2(ldsA(w, r0, s, g, sH), ldsA(w, r0, s + 1, g, sH), dz[s], dz[s + 1], a0);
-					a1 = mfma2(ldsA(w, 32 + r0, s, g, sH), ldsA(w, 32 + r0, s + 1, g, sH), dz[s], dz[s + 1], a1);
+				for (int s = 0; s < 4; s++) {
+					dz[s]	  = maskedPack(x[l][s], a0[4 * s], a0[4 * s + 1], a0[4 * s + 2], a0[4 * s + 3]);
+					dz[4 + s] = maskedPack(x[l][4 + s], a1[4 * s], a1[4 * s + 1], a1[4 * s + 2], a1[4 * s + 3]);
 				}
 			}
+			__builtin_amdgcn_sched_barrier(0);
 		}
 	}
-}
-
-// Split-K weight gradients of all layers in one launch: blockIdx.z = layer,
-// blockIdx.y = chunk of `chunk` samples; partial[layer][chunk][k][nOut] =
-// sum over the chunk of X_l^T[k][m] dZ_l^T[n][m].  One wave per 32x32
-// output tile (4 for hidden layers, 2 for the 64x3 output layer).
-__global__ void __launch_bounds__(256) k_weight_grad(const uint16_t *xTAll, const uint16_t *dzTAll, int64_t ld, int chunk, int chunks,
-													 float *partialAll) {
-	const int layer = blockIdx.z;
-	const int nOut = layer < kHidden ? 64 : 3, nOutTiles = layer < kHidden ? 2 : 1;
-	const int lane = threadIdx.x & 63, g = lane >> 5, r0 = lane & 31;
-	const int tile = threadIdx.x >> 6;
-	if (tile >= 2 * nOutTiles) return;
-	const int kt = tile / nOutTiles, nt = tile % nOutTiles;
-	const int64_t m0	 = (int64_t) blockIdx.y * chunk;
-	const uint16_t *xT	 = xTAll + (int64_t) layer * 64 * ld;
-	const uint16_t *dzT	 = dzTAll + (int64_t) layer * 64 * ld;
-	float16v acc		 = zero16();
-	const uint16_t *arow = xT + (int64_t) (32 * kt + r0) * ld + m0;
-	const uint16_t *brow = dzT + (int64_t) (32 * nt + r0) * ld + m0;
-	// eight k-steps of loads in flight before their MFMAs (same order of
-	// accumulation); chunk is a multiple of 64 (checked by the caller)
-	constexpr int kU = 8;
-	for (int s0 = 0; s0 < chunk / 8; s0 += kU) {
-		short4v a[kU], b[kU];
+	// D[i = k][j = n]: lane holds column n = nt + m, rows k = kt + 8(r/4) + 4g + r%4
 #pragma unroll
-		for (int u = 0; u < kU; u++) {
-			a[u] = *reinterpret_cast<const short4v *>(arow + 8 * (s0 + u) + 4 * g);
-			b[u] = *reinterpret_cast<const short4v *>(brow + 8 * (s0 + u) + 4 * g);
-		}
+	for (int l = 0; l <= kHidden; l++) {
+		const int nOut = l < kHidden ? 64 : 3;
+		float *dst	   = partialAll + ((int64_t) l * gridDim.x) * 4096 + (int64_t) blockIdx.x * 64 * nOut;
+		if (nt + m < nOut)
 #pragma unroll
-		for (int u = 0; u < kU; u += 2) acc = mfma2(a[u], a[u + 1], b[u], b[u + 1], acc);
+			for (int r = 0; r < 16; r++) dst[(kt + 8 * (r / 4) + 4 * g + (r % 4)) * nOut + nt + m] = dW[l][r];
 	}
-	// D[i = k][j = n]: lane holds column n = r0, rows k = 8(r/4) + 4g + r%4
-	float *dst = partialAll + (int64_t) layer * chunks * 4096 + (int64_t) blockIdx.y * 64 * nOut;
-#pragma unroll
-	for (int r = 0; r < 16; r++) {
-		const int k = 32 * kt + 8 * (r / 4) + 4 * g + (r % 4);
-		const int n = 32 * nt + r0;
-		if (n < nOut) dst[k * nOut + n] = acc[r];
-	}
-}
-
-// Sum over chunks (fixed order) of the layer's partials of weight p
-// (layer-major like the master weights).
-__device__ __forceinline__ float chunkSum(const float *partialAll, int chunks, int p) {
-	const int layer = min(p / 4096, kHidden);
-	const int q		= p - layer * 4096;
-	const int count = layer < kHidden ? 4096 : 64 * 3;
-	const float *src = partialAll + (int64_t) layer * chunks * 4096 + q;
-	float s			 = 0.f;
-	for (int c = 0; c < chunks; c++) s += src[(int64_t) c * count];
-	return s;
-}
-
-__global__ void k_reduce_chunks(const float *partialAll, int chunks, float *grad) {
-	const int p = blockIdx.x * blockDim.x + threadIdx.x;
-	if (p >= KRR_NRC_PARAMS) return;
-	grad[p] = chunkSum(partialAll, chunks, p);
 }
 
 // Deterministic loss total over tiles (one block of 256 threads).
@@ -614,75 +621,102 @@ __device__ void reduceLoss(const float *tileLoss, int64_t nTiles, float *out) {
 	if (threadIdx.x == 0) *out = part[0];
 }
 
-__global__ void k_reduce_loss(const float *tileLoss, int64_t nTiles, float *out) { reduceLoss(tileLoss, nTiles, out); }
-
 // Rewrites both bf16 copies from the fp32 master weights.
 __device__ void writeCopies(const float *w, uint16_t *wt, uint16_t *wb, int p) {
 	// p indexes the master array: layer l < 5 at 4096 l + 64 k + n; layer 5 at 20480 + 3 k + n.
-	if (p < kHidden * 4096) {
-		const int l = p / 4096, k = (p / 64) % 64, n = p % 64;
-		wt[l * 4096 + n * 64 + k] = toBf16(w[p]);
-		wb[l * 4096 + k * 64 + n] = toBf16(w[p]);
-	} else {
-		const int q = p - kHidden * 4096, k = q / 3, n = q % 3;
-		wt[kHidden * 4096 + n * 64 + k] = toBf16(w[p]);
-		wb[kHidden * 4096 + k * 32 + n] = toBf16(w[p]);
-	}
+	const int l = min(p / 4096, kHidden), q = p - l * 4096;
+	const int k = l < kHidden ? q / 64 : q / 3, n = l < kHidden ? q % 64 : q % 3;
+	const uint16_t b = toBf16(w[p]);
+	wt[l * 4096 + operandIndex(n, k, 64)]					   = b;
+	wb[l * 4096 + operandIndex(k, n, l < kHidden ? 64 : 32)] = b;
 }
 
-__global__ void k_write_copies(const float *w, uint16_t *wt, uint16_t *wb) {
+// New master weights: both copies, no moments, no steps.
+__global__ void k_set_weights(const float *w, float *mo, float *ve, uint16_t *wt, uint16_t *wb, int *step) {
 	const int p = blockIdx.x * blockDim.x + threadIdx.x;
-	if (p < KRR_NRC_PARAMS) writeCopies(w, wt, wb, p);
+	if (p == 0) *step = 0;
+	if (p >= KRR_NRC_PARAMS) return;
+	mo[p] = ve[p] = 0.f;
+	writeCopies(w, wt, wb, p);
 }
 
 // Adam (Kingma & Ba 2015) with bias corrections c1 = 1 - beta1^t, c2 = 1 - beta2^t.
 // Adam's step count lives in device memory, so that training steps recorded
 // in a graph count up on every replay.
-__device__ __forceinline__ void adamUpdate(float *w, float *mo, float *ve, float gr, float lr, float b1, float b2, float eps, float t,
+struct AdamState {
+	float w, m, v, c1, c2;
+};
+__device__ __forceinline__ void adamUpdate(float *w, float *mo, float *ve, const AdamState &a, float gr, float lr, float b1, float b2, float eps,
 										   uint16_t *wt, uint16_t *wb, int p) {
-	const float c1 = 1.f - powf(b1, t), c2 = 1.f - powf(b2, t); // bias corrections
-	const float m  = b1 * mo[p] + (1.f - b1) * gr;
-	const float v  = b2 * ve[p] + (1.f - b2) * gr * gr;
-	mo[p]		   = m;
-	ve[p]		   = v;
-	w[p] -= lr * (m / c1) / (sqrtf(v / c2) + eps);
+	const float m = b1 * a.m + (1.f - b1) * gr;
+	const float v = b2 * a.v + (1.f - b2) * gr * gr;
+	mo[p]		  = m;
+	ve[p]		  = v;
+	w[p]		  = a.w - lr * (m / a.c1) / (sqrtf(v / a.c2) + eps);
 	writeCopies(w, wt, wb, p);
 }
 
-// One training step's tail in one launch: per weight the fixed-order chunk
-// sum (the gradient, also stored), the Adam update and the bf16 copies; the
-// last block also totals the loss.  The step count was raised by
-// k_train_tile.
+// The tail of a gradient or training step in one launch: per weight the
+// fixed-order sum over the blocks of k_train that had samples, stored to `grad`
+// or, with Adam, applied (the step count was raised by k_train) and copied to
+// bf16; the last block also totals the loss.
 //
 // A block of 256 threads takes 32 weights: thread (group q, weight j) sums
-// the chunks of its eighth of the chunk range in order, and the eight group
-// sums are added in group order (a fixed order: deterministic).  One thread
-// per weight would leave most of the chip idle on a few hundred
-// latency-bound sequential loads.
+// its eighth of the partials in order, and the eight group sums are added in
+// group order (a fixed order: deterministic).  One thread per weight would
+// leave most of the chip idle on a few hundred latency-bound sequential loads;
+// with sixteen partials and Adam's state in flight at once 6.1 us for 128
+// partials, 8.7 us with the loads as the compiler orders them.
 constexpr int kReduceWeights = 32, kReduceGroups = 8;
-__global__ void __launch_bounds__(256) k_reduce_adam(const float *partialAll, int chunks, float *grad, float *w, float *mo, float *ve,
-													 float lr, float b1, float b2, float eps, const int *tDev, uint16_t *wt, uint16_t *wb,
-													 const float *tileLoss, int64_t nTiles, float *loss) {
+constexpr int kReduceBatch = 16; // partials in flight per thread
+struct Adam {
+	float *w, *m, *v;
+	uint16_t *wt, *wb;
+	const int *step;
+	float lr, b1, b2, eps;
+};
+template <bool ADAM>
+__global__ void __launch_bounds__(256) k_reduce(const float *partialAll, int blocks, Batch batch, float *grad, Adam adam, const float *tileLoss,
+												float *loss) {
 	__shared__ float part[kReduceGroups][kReduceWeights];
+	int64_t off;
+	const int64_t groups = (batch.range(off) + kGroup - 1) / kGroup;
+	const int chunks	 = (int) min((int64_t) blocks, groups);
 	const int j = threadIdx.x % kReduceWeights, q = threadIdx.x / kReduceWeights;
 	const int p = blockIdx.x * kReduceWeights + j;
 	float s		= 0.f;
+	AdamState a;
+	if (ADAM && q == 0 && p < KRR_NRC_PARAMS) { // on their way while the partials are
+		a.w	 = adam.w[p];
+		a.m	 = adam.m[p];
+		a.v	 = adam.v[p];
+		a.c1 = 1.f - powf(adam.b1, (float) *adam.step); // bias corrections
+		a.c2 = 1.f - powf(adam.b2, (float) *adam.step);
+	}
 	if (p < KRR_NRC_PARAMS) {
 		const int layer	 = min(p / 4096, kHidden);
 		const int count	 = layer < kHidden ? 4096 : 64 * 3;
-		const float *src = partialAll + (int64_t) layer * chunks * 4096 + (p - layer * 4096);
+		const float *src = partialAll + (int64_t) layer * blocks * 4096 + (p - layer * 4096);
 		const int c0 = q * chunks / kReduceGroups, c1 = (q + 1) * chunks / kReduceGroups;
-		for (int c = c0; c < c1; c++) s += src[(int64_t) c * count];
+		for (int c = c0; c < c1; c += kReduceBatch) {
+			float r[kReduceBatch];
+#pragma unroll
+			for (int k = 0; k < kReduceBatch; k++) r[k] = c + k < c1 ? src[(int64_t) (c + k) * count] : 0.f;
+#pragma unroll
+			for (int k = 0; k < kReduceBatch; k++) s += r[k];
+		}
 	}
 	part[q][j] = s;
 	__syncthreads();
 	if (q == 0 && p < KRR_NRC_PARAMS) {
 		float gr = part[0][j];
 		for (int k = 1; k < kReduceGroups; k++) gr += part[k][j];
-		grad[p] = gr;
-		adamUpdate(w, mo, ve, gr, lr, b1, b2, eps, (float) *tDev, wt, wb, p);
+		if (ADAM)
+			adamUpdate(adam.w, adam.m, adam.v, a, gr, adam.lr, adam.b1, adam.b2, adam.eps, adam.wt, adam.wb, p);
+		else
+			grad[p] = gr;
 	}
-	if (blockIdx.x == gridDim.x - 1) reduceLoss(tileLoss, nTiles, loss);
+	if (blockIdx.x == gridDim.x - 1) reduceLoss(tileLoss, groups * (kGroup / 32), loss);
 }
 
 } // namespace nrc
@@ -711,6 +745,21 @@ struct Buf {
 	template <class T> T *as() const { return reinterpret_cast<T *>(p); }
 };
 
+// A float that kernels write into host memory: it is read after the stream's
+// synchronisation without a copy in between.
+struct HostFloat {
+	float *p = nullptr, *dev = nullptr;
+	~HostFloat() {
+		if (p) (void) hipHostFree(p);
+	}
+	hipError_t alloc() {
+		if (hipError_t e = hipHostMalloc((void **) &p, sizeof(float), hipHostMallocMapped)) return e;
+		*p = 0.f;
+		return hipHostGetDevicePointer((void **) &dev, p, 0);
+	}
+	float read() const { return *(const volatile float *) p; }
+};
+
 #define NRC_HIP(expr)                                                                                                  \
 	do {                                                                                                               \
 		hipError_t e_ = (expr);                                                                                        \
@@ -718,35 +767,25 @@ struct Buf {
 	} while (0)
 
 constexpr int64_t kInferSmall = 1 << 17;
-constexpr int kChunk	= 1024; // batch granularity of the training buffers
-constexpr int kWChunk = 256;	// samples per split-K chunk of the weight gradient
-static_assert(kWChunk % 64 == 0, "k_weight_grad loads eight 8-sample k-steps at a time");
-
 } // namespace
 
 struct krr_nrc {
 	float lr = 1e-3f, beta1 = 0.9f, beta2 = 0.99f, eps = 1e-8f, lossEps = 0.01f;
 	uint64_t seed	= 1;
-	int64_t maxBatch = 65536, ld = 0;
-	bool bwdLds		 = false; // the device's blocks hold both padded weight copies in LDS
+	int64_t maxBatch = 65536;
 	int cus			 = 256;
 	int inferBlocks	 = 1024;  // k_infer_queue blocks resident at once on the device (each loads the weights once)
-	Buf w, m, v, grad, wt, wb, xT, dzT, partial, tileLoss, loss, step;
+	Buf w, m, v, wt, wb, partial, tileLoss, step;
+	HostFloat loss;
 };
 
 namespace {
 
 int uploadWeights(krr_nrc *h, const std::vector<float> &host) {
 	NRC_HIP(hipMemcpy(h->w.p, host.data(), sizeof(float) * KRR_NRC_PARAMS, hipMemcpyHostToDevice));
-	NRC_HIP(hipMemset(h->m.p, 0, sizeof(float) * KRR_NRC_PARAMS));
-	NRC_HIP(hipMemset(h->v.p, 0, sizeof(float) * KRR_NRC_PARAMS));
-	NRC_HIP(hipMemset(h->wt.p, 0, h->wt.sz));
-	NRC_HIP(hipMemset(h->wb.p, 0, h->wb.sz));
-	hipLaunchKernelGGL(k_write_copies, dim3((KRR_NRC_PARAMS + 255) / 256), dim3(256), 0, 0, h->w.as<float>(), h->wt.as<uint16_t>(),
-					   h->wb.as<uint16_t>());
+	hipLaunchKernelGGL(k_set_weights, dim3((KRR_NRC_PARAMS + 255) / 256), dim3(256), 0, 0, h->w.as<float>(), h->m.as<float>(), h->v.as<float>(),
+					   h->wt.as<uint16_t>(), h->wb.as<uint16_t>(), h->step.as<int>());
 	NRC_HIP(hipGetLastError());
-	NRC_HIP(hipDeviceSynchronize());
-	NRC_HIP(hipMemset(h->step.p, 0, sizeof(int)));
 	NRC_HIP(hipDeviceSynchronize());
 	return KRR_OK;
 }
@@ -776,37 +815,20 @@ std::vector<float> initialWeights(uint64_t seed) {
 
 bool validN(int64_t n) { return n >= 0 && n <= ((int64_t) 1 << 31); }
 
-// Gradient of one batch; with adam, also the Adam step (3 launches: tiles,
-// split-K weight gradients, reduction + update).
-int gradientImpl(krr_nrc *h, const krr_nrc_vertex *vert, const float *targets, int64_t n, hipStream_t st, bool adam, const int *nDev = nullptr,
+// Gradient of one batch, stored to `grad`, or without `grad` the Adam step.
+// One block per CU at most: each holds a CU's LDS and its share of the
+// batch's groups, and leaves one partial sum however large the batch is.
+int gradientImpl(krr_nrc *h, const krr_nrc_vertex *vert, const float *targets, int64_t n, hipStream_t st, float *grad, const int *nDev = nullptr,
 				 int64_t capTotal = 0, int step = 0, int steps = 1) {
-	const int64_t chunks = (n + kChunk - 1) / kChunk;
-	const int64_t nTiles = chunks * (kChunk / 32);
-	const bool bwdLds	 = h->bwdLds;
-	const int lds		 = (kFwdLdsElems + (bwdLds ? kBwdLdsElems : 0)) * (int) sizeof(uint16_t);
-	const int blocks	 = (int) std::min<int64_t>(1024, (nTiles + 3) / 4);
-	hipLaunchKernelGGL(bwdLds ? k_train_tile<true> : k_train_tile<false>, dim3(blocks), dim3(256), lds, st, h->wt.as<uint16_t>(),
-					   h->wb.as<uint16_t>(), (const float *) vert,
-					   targets, n, nDev, capTotal, step, steps, nTiles, h->ld, h->lossEps, h->xT.as<uint16_t>(), h->dzT.as<uint16_t>(),
-					   h->tileLoss.as<float>(), adam ? h->step.as<int>() : nullptr);
+	const int blocks = (int) std::min<int64_t>(h->cus, (n + kGroup - 1) / kGroup);
+	const Batch batch{n, nDev, capTotal, step, steps};
+	hipLaunchKernelGGL(k_train, dim3(blocks), dim3(kTrainBlock), 0, st, h->wt.as<uint16_t>(), h->wb.as<uint16_t>(), (const float *) vert,
+					   targets, batch, h->lossEps, h->partial.as<float>(), h->tileLoss.as<float>(), grad ? nullptr : h->step.as<int>());
 	NRC_HIP(hipGetLastError());
-	const int wchunks = (int) ((nTiles * 32 + kWChunk - 1) / kWChunk);
-	hipLaunchKernelGGL(k_weight_grad, dim3(1, (unsigned) wchunks, kHidden + 1), dim3(256), 0, st, h->xT.as<uint16_t>(), h->dzT.as<uint16_t>(),
-					   h->ld, kWChunk, wchunks, h->partial.as<float>());
-	NRC_HIP(hipGetLastError());
-	if (adam) {
-		hipLaunchKernelGGL(k_reduce_adam, dim3((KRR_NRC_PARAMS + kReduceWeights - 1) / kReduceWeights), dim3(kReduceWeights * kReduceGroups), 0,
-						   st, h->partial.as<float>(), wchunks,
-						   h->grad.as<float>(), h->w.as<float>(), h->m.as<float>(), h->v.as<float>(), h->lr, h->beta1, h->beta2, h->eps,
-						   (const int *) h->step.as<int>(), h->wt.as<uint16_t>(), h->wb.as<uint16_t>(), h->tileLoss.as<float>(), nTiles,
-						   h->loss.as<float>());
-		NRC_HIP(hipGetLastError());
-		return KRR_OK;
-	}
-	hipLaunchKernelGGL(k_reduce_chunks, dim3((KRR_NRC_PARAMS + 255) / 256), dim3(256), 0, st, h->partial.as<float>(), wchunks,
-					   h->grad.as<float>());
-	NRC_HIP(hipGetLastError());
-	hipLaunchKernelGGL(k_reduce_loss, dim3(1), dim3(256), 0, st, h->tileLoss.as<float>(), nTiles, h->loss.as<float>());
+	const Adam adam{h->w.as<float>(), h->m.as<float>(), h->v.as<float>(), h->wt.as<uint16_t>(), h->wb.as<uint16_t>(), h->step.as<int>(), h->lr, h->beta1, h->beta2, h->eps};
+	hipLaunchKernelGGL(grad ? k_reduce<false> : k_reduce<true>, dim3((KRR_NRC_PARAMS + kReduceWeights - 1) / kReduceWeights),
+					   dim3(kReduceWeights * kReduceGroups), 0, st, h->partial.as<float>(), blocks, batch, grad, adam, h->tileLoss.as<float>(),
+					   h->loss.dev);
 	NRC_HIP(hipGetLastError());
 	return KRR_OK;
 }
@@ -840,35 +862,28 @@ int krr_nrc_create(const char *json, krr_nrc **out) {
 	if (h->maxBatch < 32 || h->maxBatch > (1 << 24)) return krr::fail(KRR_ERR_BAD_CONFIG, "nrc config: max_batch must be in [32, 2^24]");
 	int nDev = 0;
 	if (hipGetDeviceCount(&nDev) != hipSuccess || nDev < 1) return krr::fail(KRR_ERR_NO_DEVICE, "krr_nrc_create: no HIP device");
-	h->ld = ((h->maxBatch + kChunk - 1) / kChunk) * kChunk;
-	const int64_t chunks = h->ld / kChunk;
 	NRC_HIP(h->w.alloc(sizeof(float) * KRR_NRC_PARAMS));
 	NRC_HIP(h->m.alloc(sizeof(float) * KRR_NRC_PARAMS));
 	NRC_HIP(h->v.alloc(sizeof(float) * KRR_NRC_PARAMS));
-	NRC_HIP(h->grad.alloc(sizeof(float) * KRR_NRC_PARAMS));
 	{
-		int dev = 0, maxLds = 0;
+		int dev = 0;
 		NRC_HIP(hipGetDevice(&dev));
-		NRC_HIP(hipDeviceGetAttribute(&maxLds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
-		h->bwdLds = maxLds >= (kFwdLdsElems + kBwdLdsElems) * (int) sizeof(uint16_t);
 		int cus = 0, perCu = 0;
 		NRC_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-		NRC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCu, k_infer_queue, kInferBlock, kFwdLdsElems * sizeof(uint16_t)));
+		NRC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCu, k_infer_queue, kInferBlock, kFwdElems * sizeof(uint16_t)));
 		h->cus		   = std::max(cus, 1);
 		h->inferBlocks = std::max(1, cus * std::max(perCu, 1));
 	}
 	NRC_HIP(h->wt.alloc(sizeof(uint16_t) * kFwdElems));
 	NRC_HIP(h->wb.alloc(sizeof(uint16_t) * kBwdElems));
-	NRC_HIP(h->xT.alloc(sizeof(uint16_t) * 64 * (kHidden + 1) * h->ld));
-	NRC_HIP(h->dzT.alloc(sizeof(uint16_t) * 64 * (kHidden + 1) * h->ld));
-	NRC_HIP(h->partial.alloc(sizeof(float) * 4096 * (kHidden + 1) * (h->ld / kWChunk)));
-	NRC_HIP(h->tileLoss.alloc(sizeof(float) * (h->ld / 32)));
-	NRC_HIP(h->loss.alloc(sizeof(float)));
+	const int64_t groups = (h->maxBatch + kGroup - 1) / kGroup;
+	NRC_HIP(h->partial.alloc(sizeof(float) * 4096 * (kHidden + 1) * std::min<int64_t>(groups, h->cus)));
+	NRC_HIP(h->tileLoss.alloc(sizeof(float) * groups * (kGroup / 32)));
+	NRC_HIP(h->loss.alloc());
 	NRC_HIP(h->step.alloc(sizeof(int)));
-	// padded rows of dZ_5^T (outputs 3..31) and of X^T are written per tile;
-	// clear once so that unused feature rows are finite
-	NRC_HIP(hipMemset(h->xT.p, 0, h->xT.sz));
-	NRC_HIP(hipMemset(h->dzT.p, 0, h->dzT.sz));
+	// the padded rows and columns of the bf16 copies are never written
+	NRC_HIP(hipMemset(h->wt.p, 0, h->wt.sz));
+	NRC_HIP(hipMemset(h->wb.p, 0, h->wb.sz));
 	if (int rc = uploadWeights(h.get(), initialWeights(h->seed))) return rc;
 	*out = h.release();
 	return KRR_OK;
@@ -916,7 +931,7 @@ int krr_nrc_infer(krr_nrc *nrc, const krr_nrc_vertex *vertices_dev, int64_t n, f
 	const bool small  = n <= kInferSmall;
 	const int threads = small ? 256 : 512, perBlock = 32 * (small ? 1 : 2) * (threads / 64);
 	const int blocks  = (int) std::min<int64_t>(small ? 2048 : 2 * nrc->cus, (n + perBlock - 1) / perBlock);
-	hipLaunchKernelGGL((small ? k_infer<1, 256, 3> : k_infer<2, 512, 4>), dim3(blocks), dim3(threads), kFwdLdsElems * (int) sizeof(uint16_t), (hipStream_t) hip_stream,
+	hipLaunchKernelGGL((small ? k_infer<1, 256, 3> : k_infer<2, 512, 4>), dim3(blocks), dim3(threads), kFwdElems * (int) sizeof(uint16_t), (hipStream_t) hip_stream,
 					   nrc->wt.as<uint16_t>(), (const float *) vertices_dev, n, radiance_dev);
 	NRC_HIP(hipGetLastError());
 	return KRR_OK;
@@ -928,11 +943,10 @@ int krr_nrc_gradient(krr_nrc *nrc, const krr_nrc_vertex *vertices_dev, const flo
 	if (!nrc || n < 1 || !vertices_dev || !targets_dev || !grad_dev) return krr::fail(KRR_ERR_INVALID_ARG, "krr_nrc_gradient: bad argument");
 	if (n > nrc->maxBatch) return krr::fail(KRR_ERR_CAPACITY, "krr_nrc_gradient: batch %lld exceeds max_batch %lld", (long long) n, (long long) nrc->maxBatch);
 	hipStream_t st = (hipStream_t) hip_stream;
-	if (int rc = gradientImpl(nrc, vertices_dev, targets_dev, n, st, false)) return rc;
-	NRC_HIP(hipMemcpyAsync(grad_dev, nrc->grad.p, sizeof(float) * KRR_NRC_PARAMS, hipMemcpyDeviceToDevice, st));
+	if (int rc = gradientImpl(nrc, vertices_dev, targets_dev, n, st, grad_dev)) return rc;
 	if (loss_out) {
-		NRC_HIP(hipMemcpyAsync(loss_out, nrc->loss.p, sizeof(float), hipMemcpyDeviceToHost, st));
 		NRC_HIP(hipStreamSynchronize(st));
+		*loss_out = nrc->loss.read();
 	}
 	return KRR_OK;
 }
@@ -945,7 +959,7 @@ int nrcInferAccumulate(krr_nrc *nrc, const float4 *queries, int strideF4, const 
 	// and then takes query tiles until the queue is done
 	const int tilesPerPass = kInferBlock / 64; // one 32-query tile per wave
 	const int blocks	   = std::max(1, std::min(nrc->inferBlocks, (capacity + 32 * tilesPerPass - 1) / (32 * tilesPerPass)));
-	hipLaunchKernelGGL(k_infer_queue, dim3(blocks), dim3(kInferBlock), kFwdLdsElems * (int) sizeof(uint16_t), st, nrc->wt.as<uint16_t>(), queries, strideF4,
+	hipLaunchKernelGGL(k_infer_queue, dim3(blocks), dim3(kInferBlock), kFwdElems * (int) sizeof(uint16_t), st, nrc->wt.as<uint16_t>(), queries, strideF4,
 					   count, capacity, L);
 	NRC_HIP(hipGetLastError());
 	return KRR_OK;
@@ -956,15 +970,13 @@ int nrcTrainDevice(krr_nrc *nrc, const float *vertices, const float *targets, co
 	if (cap <= 0 || steps <= 0) return KRR_OK;
 	const int64_t m = (cap + steps - 1) / steps; // largest mini-batch
 	for (int b = 0; b < steps; b++)
-		if (int rc = gradientImpl(nrc, (const krr_nrc_vertex *) vertices, targets, m, st, true, count, cap, b, steps)) return rc;
+		if (int rc = gradientImpl(nrc, (const krr_nrc_vertex *) vertices, targets, m, st, nullptr, count, cap, b, steps)) return rc;
 	return KRR_OK;
 }
 
 float nrcLastLoss(krr_nrc *nrc, hipStream_t st) {
-	float l = 0.f;
-	if (hipMemcpyAsync(&l, nrc->loss.p, sizeof(float), hipMemcpyDeviceToHost, st) != hipSuccess) return -1.f;
 	if (hipStreamSynchronize(st) != hipSuccess) return -1.f;
-	return l;
+	return nrc->loss.read();
 }
 
 extern "C" {
@@ -975,10 +987,10 @@ int krr_nrc_train_step(krr_nrc *nrc, const krr_nrc_vertex *vertices_dev, const f
 	if (!nrc || n < 1 || !vertices_dev || !targets_dev) return krr::fail(KRR_ERR_INVALID_ARG, "krr_nrc_train_step: bad argument");
 	if (n > nrc->maxBatch) return krr::fail(KRR_ERR_CAPACITY, "krr_nrc_train_step: batch %lld exceeds max_batch %lld", (long long) n, (long long) nrc->maxBatch);
 	hipStream_t st = (hipStream_t) hip_stream;
-	if (int rc = gradientImpl(nrc, vertices_dev, targets_dev, n, st, true)) return rc;
+	if (int rc = gradientImpl(nrc, vertices_dev, targets_dev, n, st, nullptr)) return rc;
 	if (loss_out) {
-		NRC_HIP(hipMemcpyAsync(loss_out, nrc->loss.p, sizeof(float), hipMemcpyDeviceToHost, st));
 		NRC_HIP(hipStreamSynchronize(st));
+		*loss_out = nrc->loss.read();
 	}
 	return KRR_OK;
 }

@@ -12,20 +12,20 @@ namespace nrc {
 constexpr int kHidden = KRR_NRC_HIDDEN_LAYERS; // hidden layers of width 64 (= matrices before the output one)
 // bf16 weight copies: forward A operands W^T [out][in] (output layer padded
 // to 32 rows) and backward A operands W [in][out] (output layer padded to 32
-// columns)
+// columns), each layer in the order in which the matrix cores' lanes take it:
+// half of 32 rows, pair of 8-column K-steps, lane, 8 bf16.  A wave reads a pair
+// as 64 consecutive 16-byte pieces, from LDS without bank conflicts or
+// padding, from memory without partial lines.
 constexpr int kFwdElems = kHidden * 64 * 64 + 32 * 64;
 constexpr int kBwdElems = kHidden * 64 * 64 + 64 * 32;
-// The copies in LDS pad every row by 4 bf16 (8 bytes): the 32 lanes that read
-// an A operand read 32 consecutive rows, and unpadded 128-byte rows would put
-// all of them on one bank.  With the padding consecutive rows start 2 banks
-// apart, so a wave's 8-byte reads spread over every bank.
-constexpr int kPad			= 4;
-constexpr int kRowH			= 64 + kPad; // LDS row of a 64-wide matrix
-constexpr int kRowO			= 32 + kPad; // LDS row of the backward output matrix (32 padded columns)
-constexpr int kFwdLdsElems = (kHidden * 64 + 32) * kRowH;
-constexpr int kBwdLdsElems = kHidden * 64 * kRowH + 64 * kRowO;
+// Place of element (row, col) of a layer with `cols` columns: lane half g of
+// row r holds columns 8s + 4g + j of K-steps s and s + 1.
+__host__ __device__ constexpr int operandIndex(int row, int col, int cols) {
+	return ((row / 32 * (cols / 16) + col / 16) * 64 + (col / 4 % 2) * 32 + row % 32) * 8 + col / 8 % 2 * 4 + col % 4;
+}
 
 typedef short short4v __attribute__((ext_vector_type(4)));	// 4 x bf16 (bit patterns)
+typedef short short8v __attribute__((ext_vector_type(8)));	// two of them: a pair of K-steps
 typedef float float16v __attribute__((ext_vector_type(16))); // 32x32 accumulator slice of one lane
 
 } // namespace nrc

@@ -196,6 +196,39 @@ def test_gpu_gradient_matches_reference(krr, gpu, rng):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 31, 33, 127, 128, 129, 1000, 32768 + 1, 65536])
+def test_gpu_gradient_at_the_edges_of_tiles_and_groups(krr, gpu, rng, n):
+    """One sample to several 128-sample groups per block: the gradient is the
+    bf16-emulated reference's.  Where an activation or output gradient rounds
+    to the other bf16 neighbour (accumulation order) the sample's gradient
+    moves by 2^-8; a mean over n samples by at most that, so a single sample is
+    held to 2^-7 and 1000 or more to the 1e-3 of the test above.  The loss is
+    read after the call, and nothing is kept between calls."""
+    from kiraray_amd.nrc import NeuralRadianceCache
+    print("case: nrc gradient n", n, flush=True)
+    nrc = NeuralRadianceCache({"seed": 11})
+    w = nrc.get_weights().astype(np.float64)
+    v = ref.random_vertices(n, rng)
+    t = (rng.random((n, 3)) * 1.5).astype(np.float32)
+    grad, enc = gpu.DeviceBuffer(ref.PARAMS * 4), gpu.DeviceBuffer(n * 64 * 4)
+    vb, tb = _dev(gpu, v), _dev(gpu, t)
+    nrc.encode(vb.ptr, n, enc.ptr)
+    loss = nrc.gradient(vb.ptr, tb.ptr, n, grad.ptr)
+    gpu.synchronize()
+    g = grad.to_numpy(np.float32, (ref.PARAMS,))
+    le, ge = ref.loss_and_grad(w, enc.to_numpy(np.float32, (n, 64)).astype(np.float64), t, emulate_bf16=True)
+    tol = 1e-3 if n >= 1000 else 2.0 ** -7
+    assert abs(loss - le) <= tol * le
+    for l in range(ref.HIDDEN + 1):
+        sl = slice(l * 4096, (l + 1) * 4096) if l < ref.HIDDEN else slice(ref.HIDDEN * 4096, None)
+        assert np.linalg.norm(g[sl] - ge[sl]) <= tol * np.linalg.norm(ge[sl]) + 1e-12, l
+    again = nrc.gradient(vb.ptr, tb.ptr, n, grad.ptr)
+    gpu.synchronize()
+    assert again == loss and np.array_equal(grad.to_numpy(np.float32, (ref.PARAMS,)), g)
+    nrc.close()
+
+
+@pytest.mark.gpu
 def test_gpu_adam_step(krr, gpu, rng):
     """One training step = the GPU gradient followed by the Adam update of
     the reference, on the FP32 master weights."""
