@@ -1190,15 +1190,14 @@ __global__ void k_megakernel(WfParams P0, DevScene sc, TraceBvh bvh, RayQueueDev
 // next depth in this order, and each ray takes the same traversal steps, so
 // the radiance additions, RNG draws and hits are those of k_megakernel.  Once
 // no path is left to take, the rounds run every traversal to its end.
-// Waves per SIMD the refill launch is compiled for: 3 (168 VGPRs, no
-// scratch) for the single-view launch, where it runs as fast as 4 waves with
-// 120 bytes per lane of spills (3.80 against 3.79-3.83 ms per frame on the
-// 1.31 M-triangle 1080p field); 4 for the multi-view launch, which 3 waves
-// slow by 7 % (259 against 243 ms for 256 views).
-constexpr int refillWaves(bool views) { return views ? 4 : 3; }
-
-template <bool COUNT, bool NRC = false, bool VIEWS = false, bool PLAIN = false>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(refillWaves(VIEWS), refillWaves(VIEWS))))
+// DENSE compiles it for 4 waves per SIMD (128 registers, 40-110 bytes of
+// scratch), else 3 (168 registers, no scratch).  Half of a wave's cycles wait
+// for memory, so the fourth wave pays where there are paths for it and the
+// tree does not sit in the caches: every multi-view launch (32 views 7.6 against
+// 8.6 ms), and frames by denseRefill below.  Textures (1.55 against 1.61 ms)
+// and the radiance cache's queries (1.72 against 1.85 ms) spill too much.
+template <bool COUNT, bool NRC, bool VIEWS, bool PLAIN, bool DENSE>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DENSE ? 4 : 3, DENSE ? 4 : 3)))
 k_megakernel_refill(WfParams P0, DevScene sc, TraceBvh bvh, RayQueueDev q, const int *countPtr, int startDepth,
 									PixelStateDev px, int *ovf, Counters *cnt, NrcDev nrc = NrcDev{}, ViewsDev V = ViewsDev{},
 									CameraDev cam = CameraDev{}, int camFetch = 0) {
@@ -1739,18 +1738,18 @@ int reserveOverflow(DevBuf &buf, const AccelData &a, size_t threads) {
 }
 
 // The persistent kernel variants of every frame kind.
-// REFILL: k_megakernel_refill (scenes without media).
+// REFILL: k_megakernel_refill (scenes without media), DENSE its 4-wave form.
 // nodeBytes: the refill launch's LDS copy of the top tree nodes, behind the stack.
-template <bool MEDIA, bool COUNT, bool NRC, bool VIEWS, bool PLAIN, bool REFILL = false> struct Mega {
+template <bool MEDIA, bool COUNT, bool NRC, bool VIEWS, bool PLAIN, bool REFILL = false, bool DENSE = VIEWS> struct Mega {
 	static int grid(int tb, size_t lds, int maxBlocks, size_t nodeBytes = 0) {
-		if constexpr (REFILL) return persistentGrid(k_megakernel_refill<COUNT, NRC, VIEWS, PLAIN>, tb, lds + nodeBytes, maxBlocks);
+		if constexpr (REFILL) return persistentGrid(k_megakernel_refill<COUNT, NRC, VIEWS, PLAIN, DENSE>, tb, lds + nodeBytes, maxBlocks);
 		else return persistentGrid(k_megakernel<MEDIA, COUNT, NRC, VIEWS, PLAIN>, tb, lds, maxBlocks);
 	}
 	static void launch(unsigned g, int tb, size_t lds, hipStream_t st, const WfParams &P, const DevScene &ds, const TraceBvh &bvh,
 					   const RayQueueDev &q, const int *countPtr, const PixelStateDev &px, int *ovf, Counters *cnt, const NrcDev &nrc,
 					   const ViewsDev &V, int startDepth = 0, const CameraDev &cam = CameraDev{}, int camFetch = 0) {
 		if constexpr (REFILL)
-			hipLaunchKernelGGL((k_megakernel_refill<COUNT, NRC, VIEWS, PLAIN>), dim3(g), dim3(tb), lds + (size_t) P.ldsNodes * sizeof(Bvh4Node), st, P,
+			hipLaunchKernelGGL((k_megakernel_refill<COUNT, NRC, VIEWS, PLAIN, DENSE>), dim3(g), dim3(tb), lds + (size_t) P.ldsNodes * sizeof(Bvh4Node), st, P,
 							   ds, bvh, q, countPtr, startDepth, px, ovf, cnt, nrc, V, cam, camFetch);
 		else
 			hipLaunchKernelGGL((k_megakernel<MEDIA, COUNT, NRC, VIEWS, PLAIN>), dim3(g), dim3(tb), lds, st, P, ds, bvh, q, countPtr, startDepth, px, ovf,
@@ -1766,9 +1765,20 @@ template <bool VIEWS, bool REFILL, class F> auto withMegaR(bool media, bool coun
 	return count ? f(Mega<false, true, false, VIEWS, false, REFILL>{}) : f(Mega<false, false, false, VIEWS, false, REFILL>{});
 }
 
+// Single-view frames that take the refill launch's 4-wave form: at least three
+// times the paths it has lanes, so that lanes are refilled for most of the
+// launch, and nodes of 2 MB, half an L2.  ms with 3 / 4 waves: 1.31 M triangles
+// 640x360 1.40 / 1.48, 960x540 1.64 / 1.79, 1100x700 1.87 / 1.87, 1280x720
+// 1.99 / 1.94, 1920x1080 3.58 / 3.39 and with two samples 6.22 / 5.69; 82 K
+// triangles 1280x720 1.10 / 1.10, 1920x1080 1.88 / 1.84; 20 K triangles 1920x1080
+// 1.44 / 1.47.
+bool denseRefill(const AccelData &a, int64_t paths) { return paths >= 3 << 18 && a.nNodes >= 1 << 14; }
+
 // The persistent kernel for these flags; the refill launch for scenes
 // without media when refill_lanes > 0.
-template <bool VIEWS, class F> auto withMega(bool media, bool count, bool nrc, bool plain, bool refill, F &&f) {
+template <bool VIEWS, class F> auto withMega(bool media, bool count, bool nrc, bool plain, bool refill, bool dense, F &&f) {
+	if constexpr (!VIEWS)
+		if (dense && refill && !media && !nrc && plain) return count ? f(Mega<false, true, false, false, true, true, true>{}) : f(Mega<false, false, false, false, true, true, true>{});
 	if (refill && !media) return withMegaR<VIEWS, true>(media, count, nrc, plain, f);
 	return withMegaR<VIEWS, false>(media, count, nrc, plain, f);
 }
@@ -1849,6 +1859,7 @@ struct krr_wf {
 	krr_camera cam{};
 	uint64_t frameIndex = 0;
 	uint64_t gridKey	= ~0ull;
+	bool gridDense = false; // which form of the refill launch the grids were sized for
 	int gClosest = 1, gShadow = 1, gShade = 1;
 	PathGrid gMega;
 	bool beginPending	= false;
@@ -2657,11 +2668,12 @@ int krr_wf_render(krr_wf *wf, float *film_dev, void *hip_stream) {
 	const bool media   = wf->enableMedium && wf->sceneHasMedia;
 	const bool plain   = !wf->sceneTextured;
 	const bool refill  = refillLanesOf(wf) > 0;
+	const bool dense   = denseRefill(wf->accel, N);
 	// persistent grid sizes (resident blocks), computed once per shape
 	const uint64_t shapeKey = ((uint64_t) N << 24) ^ ((uint64_t) tb << 12) ^ ((uint64_t) bs << 2) ^ ((uint64_t) wf->accel.stackSize << 50) ^ ((uint64_t) wf->stackLdsEntries << 43) ^
 							  (count ? 2 : 0) ^ (media ? 1 : 0) ^ (wf->nrcOn ? 4 : 0) ^ (plain ? 8 : 0) ^ (refill ? 16 : 0) ^
 							  ((uint64_t) ldsNodeCount(wf) << 5) ^ ((uint64_t) (wf->occupancy * 1024.f) << 32);
-	if (shapeKey != wf->gridKey) {
+	if (shapeKey != wf->gridKey || dense != wf->gridDense) {
 		// Counting variants use more registers: size each grid for the variant launched.
 		wf->gClosest = count ? persistentGrid(k_trace_closest_queue<true>, tb, lds, gTmax) : persistentGrid(k_trace_closest_queue<false>, tb, lds, gTmax);
 		if (media) wf->gShadow = count ? persistentGrid(k_shadow_tr<true>, tb, lds, gTmax) : persistentGrid(k_shadow_tr<false>, tb, lds, gTmax);
@@ -2669,14 +2681,15 @@ int krr_wf_render(krr_wf *wf, float *film_dev, void *hip_stream) {
 		wf->gShade = media ? persistentGrid(k_shade<true>, bs, 0, (int) gN) : persistentGrid(k_shade<false>, bs, 0, (int) gN);
 		const size_t nodeBytes = (size_t) ldsNodeCount(wf) * sizeof(Bvh4Node);
 		auto mega = [&](bool nrc) {
-			const int resident = withMega<false>(media, count, nrc, plain, refill, [&](auto k) { return decltype(k)::grid(tb, lds, 1 << 20, nodeBytes); });
+			const int resident = withMega<false>(media, count, nrc, plain, refill, dense, [&](auto k) { return decltype(k)::grid(tb, lds, 1 << 20, nodeBytes); });
 			return pathGrid(scaledGrid(resident, wf->occupancy), tb, N, !media && !refill);
 		};
 		wf->gMega = mega(false);
 		if (wf->nrcOn) wf->gMegaNrc = mega(true);
 		const int gMax = std::max(std::max(std::max(wf->gClosest, wf->gShadow), wf->gMega.blocks), wf->nrcOn ? wf->gMegaNrc.blocks : 0);
 		if (int rc = reserveOverflow(wf->ovf, wf->accel, (size_t) gMax * tb)) return rc;
-		wf->gridKey = shapeKey;
+		wf->gridKey	  = shapeKey;
+		wf->gridDense = dense;
 	}
 	int *ovf = wf->ovf.as<int>();
 	const unsigned gTc = (unsigned) wf->gClosest, gTs = (unsigned) wf->gShadow, gS = (unsigned) wf->gShade;
@@ -2747,7 +2760,7 @@ int krr_wf_render(krr_wf *wf, float *film_dev, void *hip_stream) {
 				timed(4, [&] {
 					const int camFetch = depth == 0 ? 1 : 0; // k_camera skipped: the kernel makes the camera rays
 					const int *cp	 = (const int *) &cnt->rayCount[cur];
-					withMega<false>(media, count, wf->nrcOn, plain, refill, [&](auto k) {
+					withMega<false>(media, count, wf->nrcOn, plain, refill, dense, [&](auto k) {
 						decltype(k)::launch((unsigned) pg.blocks, tb, lds, st, P, wf->ds, bvh, cq, cp, px, ovf, cnt,
 											wf->nrcOn ? nrc : NrcDev{}, ViewsDev{}, depth, cam, camFetch);
 						return 0;
@@ -2846,7 +2859,7 @@ int viewsLaunch(krr_wf *wf, int N, bool nrc, ViewsLaunch &L) {
 						 (refillLanesOf(wf) > 0 ? 16 : 0) ^ ((uint64_t) ldsNodeCount(wf) << 5) ^ ((uint64_t) (wf->occupancy * 1024.f) << 32);
 	if (key != wf->viewsGridKey) {
 		const size_t nodeBytes = (size_t) ldsNodeCount(wf) * sizeof(Bvh4Node);
-		const int resident = withMega<true>(L.media, L.count, nrc, !wf->sceneTextured, refillLanesOf(wf) > 0,
+		const int resident = withMega<true>(L.media, L.count, nrc, !wf->sceneTextured, refillLanesOf(wf) > 0, false,
 											[&](auto k) { return decltype(k)::grid(tb, L.lds, 1 << 20, nodeBytes); });
 		wf->gMegaViews = pathGrid(scaledGrid(resident, wf->occupancy), tb, N, !L.media && refillLanesOf(wf) == 0);
 		if (int rc = reserveOverflow(wf->ovf, wf->accel, (size_t) wf->gMegaViews.blocks * tb)) return rc;
@@ -2911,7 +2924,7 @@ int enqueueViews(krr_wf *wf, WfParams P, const ViewsLaunch &L, hipStream_t st, b
 			hipLaunchKernelGGL(k_tile_pixels_views, dim3(nT), dim3(64), 0, st, sorted, off, V, wf->vOrder.as<int>());
 		}
 		timed(4, [&] {
-			withMega<true>(L.media, L.count, L.nrc, !wf->sceneTextured, refillLanesOf(wf) > 0, [&](auto k) {
+			withMega<true>(L.media, L.count, L.nrc, !wf->sceneTextured, refillLanesOf(wf) > 0, false, [&](auto k) {
 				decltype(k)::launch((unsigned) L.grid.blocks, tb, L.lds, st, P, wf->ds, L.bvh, RayQueueDev{}, nullptr, px, ovf, cnt, nrc, V);
 				return 0;
 			});
@@ -3118,7 +3131,7 @@ int krr_wf_autotune(krr_wf *wf, int64_t trial_paths, char *report, int32_t cap, 
 				hipLaunchKernelGGL(k_begin_views, dim3((unsigned) ((N + 255) / 256)), dim3(256), 0, st, P, viewsDev(wf), tpx);
 				hipLaunchKernelGGL(k_mega_begin, dim3(1), dim3(1), 0, st, wf->counters.as<Counters>());
 				KRR_HIP(hipEventRecord(e0, st));
-				withMega<true>(L.media, false, false, !wf->sceneTextured, refillLanesOf(wf) > 0, [&](auto k) {
+				withMega<true>(L.media, false, false, !wf->sceneTextured, refillLanesOf(wf) > 0, false, [&](auto k) {
 					decltype(k)::launch((unsigned) L.grid.blocks, wf->traceBlockSize, L.lds, st, P, wf->ds, L.bvh, RayQueueDev{}, nullptr, tpx,
 										wf->ovf.as<int>(), wf->counters.as<Counters>(), NrcDev{}, viewsDev(wf));
 					return 0;
@@ -3130,7 +3143,7 @@ int krr_wf_autotune(krr_wf *wf, int64_t trial_paths, char *report, int32_t cap, 
 				const size_t lds   = stackLds(wf->accel, t.tb);
 				const int maxBlocks = std::max(1, (N + t.tb - 1) / t.tb);
 				const size_t nodeBytes = (size_t) ldsNodeCount(wf) * sizeof(Bvh4Node);
-				int g = withMega<false>(media, false, false, !wf->sceneTextured, refillLanesOf(wf) > 0,
+				int g = withMega<false>(media, false, false, !wf->sceneTextured, refillLanesOf(wf) > 0, denseRefill(wf->accel, N),
 										[&](auto k) { return decltype(k)::grid(t.tb, lds, maxBlocks, nodeBytes); });
 				g	  = scaledGrid(g, t.occ);
 				if (int e = reserveOverflow(wf->ovf, wf->accel, (size_t) g * t.tb)) return e;
@@ -3143,7 +3156,7 @@ int krr_wf_autotune(krr_wf *wf, int64_t trial_paths, char *report, int32_t cap, 
 				hipLaunchKernelGGL(k_camera, dim3(gN), dim3(256), 0, st, P, cameraDev(wf->cam), px, rayQueue(wf, 0), cnt);
 				hipLaunchKernelGGL(k_mega_begin, dim3(1), dim3(1), 0, st, cnt);
 				KRR_HIP(hipEventRecord(e0, st));
-				withMega<false>(media, false, false, !wf->sceneTextured, refillLanesOf(wf) > 0, [&](auto k) {
+				withMega<false>(media, false, false, !wf->sceneTextured, refillLanesOf(wf) > 0, denseRefill(wf->accel, N), [&](auto k) {
 					decltype(k)::launch((unsigned) g, t.tb, lds, st, P, wf->ds, bvh, rayQueue(wf, 0), (const int *) &cnt->rayCount[0], px,
 										wf->ovf.as<int>(), cnt, NrcDev{}, ViewsDev{});
 					return 0;

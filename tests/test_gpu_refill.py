@@ -154,3 +154,27 @@ def test_refill_by_scene_size(krr, gpu):
     wf.set_scene(krr.Scene(CORNELL))
     assert wf.to_json()["refill_lanes_in_force"] == 16
     wf.close()
+
+
+@pytest.mark.parametrize("width,count", [(1023, 256), (1024, 256), (1025, 256), (1024, 64)])
+def test_refill_large_frames_equal_plain_launch(krr, gpu, width, count):
+    """Around 1024x768 paths and the tree size from which the refill launch
+    takes its 4-wave form: the frame and the ray counts are those of the launch
+    without refill, also when the frame shrinks below the line and grows back
+    in one tracer."""
+    print(f"case: {width}x768 over {count} spheres", flush=True)
+    s = krr.Scene(icosphere_scene(count=count, level=2, res=(width, 768)))
+    params = {"spp": 1, "max_depth": 4, "rr": 0.8}
+    a, sa = gpu_render(krr, gpu, s, width, 768, params)
+    b, sb = gpu_render(krr, gpu, s, width, 768, {**params, "refill_lanes": 0})
+    assert np.array_equal(a, b) and sa["closest_rays"] == sb["closest_rays"] and sa["shadow_rays"] == sb["shadow_rays"]
+    wf = krr.WavefrontPathTracer(params)
+    wf.set_scene(s)
+    for w, h in ((width, 768), (64, 48), (width, 768)):
+        wf.resize(w, h)
+        film = gpu.DeviceBuffer(w * h * 16)
+        wf.begin_frame(s.camera(0), 1)
+        wf.render(film.ptr, 0)
+        wf.end_frame()
+    assert np.array_equal(film.to_numpy(np.float32, (768, width, 4)), a)
+    wf.close()
