@@ -222,7 +222,7 @@ __device__ __forceinline__ void loadVertex(const float *vertices, int64_t i, int
 
 // Inference: each wave evaluates T tiles of 32 samples at a time.  Reading a
 // layer's weights from LDS takes as long as the matrix cores take for one tile
-// (47 KB at 128 bytes a cycle, 370 cycles each), so with two tiles per wave the
+// (44 KB at 128 bytes a cycle, 350 cycles each), so with two tiles per wave the
 // reads halve; 118 registers leave 4 waves per SIMD, in two blocks of 8 waves
 // that share a copy of the weights each and stay resident.  1 M samples 51
 // against 58 us, 4 M 197 against 228 us on one card; on another 53 against 61
