@@ -15,8 +15,12 @@
 //  * large nodes (> kSmall references) are processed level by level, all
 //    nodes of a level together: bounds, bins (LDS per block, merged with
 //    integer atomics on order-preserving float encodings), split choice, a
-//    stable partition between two reference buffers (per-block counts, a
-//    scatter), and the next level's list made on the device;
+//    stable partition between two reference buffers (places from the blocks'
+//    bin counts) that also takes the children's bounds, and the next level's list
+//    made on the device.  Two passes over the references per level, bound by
+//    the latency of gathered boxes and by atomics on few addresses: 13 levels of a
+//    328 K-triangle build 0.94 ms, 1.30 ms with bounds and counts in two more
+//    passes and blocks of 2,048 references;
 //  * every node of at most kSmall references roots a subtree that one block
 //    builds alone in LDS, level by level, a node per wave;
 //  * the binary tree is collapsed into 4-wide nodes level by level (open the
@@ -43,8 +47,12 @@ namespace bvhdev {
 
 constexpr int NB	   = 16;   // SAH bins per axis (the host builder's default)
 constexpr int kSmall   = 1024; // nodes of at most this many references are built by one block
-constexpr int kChunk   = 2048; // references per block in the level-synchronous phase
-constexpr int kThreads = 256;
+// References and threads per block in the level-synchronous phase: its passes
+// wait for gathered boxes, and a level of 328 K references in blocks of 2,048 and
+// 256 threads is less than one wave per SIMD.  2,048 with 1,024 threads, a
+// build and two traces 4.48 against 4.43 ms.
+constexpr int kChunk   = 1024;
+constexpr int kThreads = 512;
 
 // Order-preserving float <-> int map: a < b (floats) <=> ordF(a) < ordF(b).
 __host__ __device__ inline int ordF(float f) {
@@ -232,13 +240,14 @@ struct Level {
 	int *nLeft;					// left references per node
 	int *blockNode;				// node of each block
 	int *blockStart;			// first reference of each block
-	int *blockLeft;				// per-block left counts
+	int *blockCnt;				// the axes' bin counts of each block's references
+	int *childBox;				// per node 24 ints: bounds and centroid bounds of the left child, then the right
 	const int *blockBegin;		// first block of each node (n + 1 entries)
 };
 
 // One of the two node lists that the levels alternate between.
 struct LevelList {
-	int *first, *count, *node, *blockBegin;
+	int *first, *count, *node, *blockBegin, *box, *cbox;
 };
 
 // What the host reads between levels, and the running totals.
@@ -248,15 +257,14 @@ struct LevelCtl {
 	int bad;			 // a split left a side empty
 };
 
-// Bounds, bins and blocks of each node of the level.
+// Empty bounds, as ordered ints: entry e of a box is one of lo xyz, hi xyz.
+__device__ inline int emptyBound(int e) { return e % 6 < 3 ? ordF(__builtin_inff()) : ordF(-__builtin_inff()); }
+
+// Bins, child bounds and blocks of each node of the level.
 __global__ void k_level_reset(Level L, int nNodes) {
 	const int t = blockIdx.x;
 	if (t >= nNodes) return;
-	for (int e = threadIdx.x; e < 12; e += blockDim.x) {
-		const int v = (e % 6) < 3 ? ordF(__builtin_inff()) : ordF(-__builtin_inff());
-		if (e < 6) L.box[6 * t + e] = v;
-		else L.cbox[6 * t + e - 6] = v;
-	}
+	for (int e = threadIdx.x; e < 24; e += blockDim.x) L.childBox[24 * t + e] = emptyBound(e);
 	binsReset(L.bins[t], threadIdx.x, blockDim.x);
 	for (int b = L.blockBegin[t] + (int) threadIdx.x; b < L.blockBegin[t + 1]; b += blockDim.x) {
 		L.blockNode[b]	= t;
@@ -273,30 +281,51 @@ __device__ inline float waveMax(float v) {
 	return v;
 }
 
-__global__ void __launch_bounds__(kThreads) k_level_bounds(Level L, Prims P, const int *refs) {
-	const int b = blockIdx.x, t = L.blockNode[b];
-	const int end = min(L.blockStart[b] + kChunk, L.first[t] + L.count[t]);
+// A wave's bounds and centroid bounds into twelve ordered ints.
+__device__ inline void mergeBounds(int *to, const Box &box, const Box &cen) {
+#pragma unroll
+	for (int a = 0; a < 3; a++) {
+		const float v[4] = {waveMin(box.lo[a]), waveMax(box.hi[a]), waveMin(cen.lo[a]), waveMax(cen.hi[a])};
+		if (__lane_id() == 0) {
+			atomicMin(&to[a], ordF(v[0]));
+			atomicMax(&to[3 + a], ordF(v[1]));
+			atomicMin(&to[6 + a], ordF(v[2]));
+			atomicMax(&to[9 + a], ordF(v[3]));
+		}
+	}
+}
+
+__device__ inline void growCentroid(Box &cen, const float c[3]) {
+	for (int a = 0; a < 3; a++) {
+		cen.lo[a] = fminf(cen.lo[a], c[a]);
+		cen.hi[a] = fmaxf(cen.hi[a], c[a]);
+	}
+}
+
+// Bounds of the root (a child's come from the scatter of its parent), by few
+// blocks: their atomics meet at twelve addresses.
+constexpr int kRootBlocks = 128;
+__global__ void __launch_bounds__(kThreads) k_root_bounds(Prims P, int n, int *box, int *cbox) {
+	__shared__ int bounds[12];
+	if (threadIdx.x < 12) bounds[threadIdx.x] = emptyBound(threadIdx.x);
+	__syncthreads();
 	Box bb, cb;
 	bb.reset();
 	cb.reset();
-	for (int i = L.blockStart[b] + (int) threadIdx.x; i < end; i += kThreads) {
+	for (int i = blockIdx.x * kThreads + (int) threadIdx.x; i < n; i += gridDim.x * kThreads) {
 		Box pb;
 		float c[3];
-		primBox(P, refs[i], pb, c);
+		primBox(P, i, pb, c);
 		bb.grow(pb);
-		for (int a = 0; a < 3; a++) {
-			cb.lo[a] = fminf(cb.lo[a], c[a]);
-			cb.hi[a] = fmaxf(cb.hi[a], c[a]);
-		}
+		growCentroid(cb, c);
 	}
-	for (int a = 0; a < 3; a++) {
-		const float v[4] = {waveMin(bb.lo[a]), waveMax(bb.hi[a]), waveMin(cb.lo[a]), waveMax(cb.hi[a])};
-		if (__lane_id() == 0) {
-			atomicMin(&L.box[6 * t + a], ordF(v[0]));
-			atomicMax(&L.box[6 * t + 3 + a], ordF(v[1]));
-			atomicMin(&L.cbox[6 * t + a], ordF(v[2]));
-			atomicMax(&L.cbox[6 * t + 3 + a], ordF(v[3]));
-		}
+	mergeBounds(bounds, bb, cb);
+	__syncthreads();
+	const int e = threadIdx.x;
+	if (e < 12) {
+		int *to = e < 6 ? box + e : cbox + e - 6;
+		if (e % 6 < 3) atomicMin(to, bounds[e]);
+		else atomicMax(to, bounds[e]);
 	}
 }
 
@@ -339,6 +368,7 @@ __global__ void __launch_bounds__(kThreads) k_level_bins(Level L, Prims P, const
 	Bins &g = L.bins[t];
 	for (int i = threadIdx.x; i < 3 * NB; i += kThreads) {
 		const int a = i / NB, k = i % NB;
+		L.blockCnt[(size_t) b * 3 * NB + i] = sb.cnt[a][k];
 		if (sb.cnt[a][k] == 0) continue;
 		atomicAdd(&g.cnt[a][k], sb.cnt[a][k]);
 		for (int e = 0; e < 3; e++) {
@@ -388,44 +418,40 @@ __device__ inline float splitScale(const Level &L, int t, const Box &cb) {
 	return ext > 0 ? NB / ext : 0.f;
 }
 
-__global__ void __launch_bounds__(kThreads) k_level_count(Level L, Prims P, const int *refs) {
-	__shared__ int part[kThreads / 64];
-	const int b = blockIdx.x, t = L.blockNode[b];
-	const Box cb	  = loadBox(L.cbox + 6 * t);
-	const float scale = splitScale(L, t, cb);
-	const int ax	  = L.axis[t] < 0 ? 0 : L.axis[t];
-	const int end	  = min(L.blockStart[b] + kChunk, L.first[t] + L.count[t]);
-	int n = 0;
-	for (int i = L.blockStart[b] + (int) threadIdx.x; i < end; i += kThreads) {
-		Box pb;
-		float c[3];
-		primBox(P, refs[i], pb, c);
-		n += goesLeft(L, t, cb, scale, i, c[ax]) ? 1 : 0;
+// Left references of block e of node t.
+__device__ inline int blockLefts(const Level &L, int t, int e) {
+	if (L.decision[t] != 0) {
+		const int size = min(kChunk, L.first[t] + L.count[t] - L.blockStart[e]);
+		return min(max(L.first[t] + L.count[t] / 2 - L.blockStart[e], 0), size);
 	}
-	for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o);
-	if (__lane_id() == 0) part[threadIdx.x / 64] = n;
-	__syncthreads();
-	if (threadIdx.x == 0) {
-		int s = 0;
-		for (int w = 0; w < kThreads / 64; w++) s += part[w];
-		L.blockLeft[b] = s;
-	}
+	const int *cnt = L.blockCnt + (size_t) e * 3 * NB + L.axis[t] * NB;
+	int n		   = 0;
+	for (int k = 0; k <= L.bin[t]; k++) n += cnt[k];
+	return n;
 }
 
-// Stable partition: thread j of the block owns references [8j, 8j + 8) of
-// the block's chunk, in order.
+// Stable partition: thread j of the block owns the references [per j, per j + per)
+// of the block's chunk, in order.  The bounds of a child that is a large node
+// itself are taken on the way.
 __global__ void __launch_bounds__(kThreads) k_level_scatter(Level L, Prims P, const int *refs, int *tmp) {
-	constexpr int per = kChunk / kThreads;
-	__shared__ int lefts[kThreads], earlier[kThreads / 64];
-	const int b = blockIdx.x, t = L.blockNode[b];
+	constexpr int per = kChunk / kThreads, waves = kThreads / 64;
+	__shared__ int lefts[waves], earlier[waves], bounds[24];
+	const int b = blockIdx.x, t = L.blockNode[b], lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 	const Box cb	  = loadBox(L.cbox + 6 * t);
 	const float scale = splitScale(L, t, cb);
 	const int ax	  = L.axis[t] < 0 ? 0 : L.axis[t];
 	const int first = L.first[t], end = min(L.blockStart[b] + kChunk, first + L.count[t]);
 	const int i0 = L.blockStart[b] + (int) threadIdx.x * per;
+	if (threadIdx.x < 24) bounds[threadIdx.x] = emptyBound(threadIdx.x);
 	int r[per];
 	bool left[per];
-	int nl = 0;
+	Box box[2], cen[2];
+#pragma unroll
+	for (int k = 0; k < 2; k++) {
+		box[k].reset();
+		cen[k].reset();
+	}
+#pragma unroll
 	for (int k = 0; k < per; k++) {
 		const int i = i0 + k;
 		r[k]		= i < end ? refs[i] : -1;
@@ -435,33 +461,56 @@ __global__ void __launch_bounds__(kThreads) k_level_scatter(Level L, Prims P, co
 			float c[3];
 			primBox(P, r[k], pb, c);
 			left[k] = goesLeft(L, t, cb, scale, i, c[ax]);
-			nl += left[k] ? 1 : 0;
+#pragma unroll
+			for (int side = 0; side < 2; side++) {
+				if (left[k] != (side == 0)) continue;
+				box[side].grow(pb);
+				growCentroid(cen[side], c);
+			}
 		}
 	}
-	// left references of the node's earlier blocks
+	// left references of the node's earlier blocks, of the block's earlier waves
+	// and of the wave's earlier lanes
 	int before = 0;
-	for (int e = L.blockBegin[t] + (int) threadIdx.x; e < b; e += kThreads) before += L.blockLeft[e];
+	for (int e = L.blockBegin[t] + (int) threadIdx.x; e < b; e += kThreads) before += blockLefts(L, t, e);
 	for (int o = 32; o > 0; o >>= 1) before += __shfl_xor(before, o);
-	if (__lane_id() == 0) earlier[threadIdx.x / 64] = before;
-	lefts[threadIdx.x] = nl;
+	int leftBefore = 0, waveLefts = 0;
+#pragma unroll
+	for (int k = 0; k < per; k++) {
+		const uint64_t m = __ballot(left[k]);
+		leftBefore += __popcll(m & ((1ull << lane) - 1));
+		waveLefts += __popcll(m);
+	}
+	if (lane == 0) {
+		earlier[wave] = before;
+		lefts[wave]	  = waveLefts;
+	}
 	__syncthreads();
 	before = 0;
-	for (int w = 0; w < kThreads / 64; w++) before += earlier[w];
-	// exclusive prefix over the threads (Hillis-Steele in LDS)
-	for (int o = 1; o < kThreads; o <<= 1) {
-		const int v = threadIdx.x >= (unsigned) o ? lefts[threadIdx.x - o] : 0;
-		__syncthreads();
-		lefts[threadIdx.x] += v;
-		__syncthreads();
+	for (int w = 0; w < waves; w++) {
+		before += earlier[w];
+		if (w < wave) leftBefore += lefts[w];
 	}
-	const int leftBefore  = lefts[threadIdx.x] - nl; // lefts of earlier threads of this block
-	const int blockBefore = i0 - L.blockStart[b];	  // references of earlier threads of this block
+	const int blockBefore = i0 - L.blockStart[b]; // references of earlier threads of this block
 	int lp = first + before + leftBefore;
 	int rp = first + L.nLeft[t] + (L.blockStart[b] - first - before) + (blockBefore - leftBefore);
+#pragma unroll
 	for (int k = 0; k < per; k++) {
 		if (i0 + k >= end) break;
 		if (left[k]) tmp[lp++] = r[k];
 		else tmp[rp++] = r[k];
+	}
+	const int sizes[2] = {L.nLeft[t], L.count[t] - L.nLeft[t]};
+#pragma unroll
+	for (int side = 0; side < 2; side++) {
+		if (sizes[side] <= kSmall) continue;
+		mergeBounds(bounds + 12 * side, box[side], cen[side]);
+	}
+	__syncthreads();
+	const int e = threadIdx.x;
+	if (e < 24 && sizes[e / 12] > kSmall) {
+		if (e % 6 < 3) atomicMin(&L.childBox[24 * t + e], bounds[e]);
+		else atomicMax(&L.childBox[24 * t + e], bounds[e]);
 	}
 }
 
@@ -476,6 +525,7 @@ __global__ void k_level_init(LevelList list, SmallTask *small, LevelCtl *ctl, in
 	list.count[0]	 = n;
 	list.node[0]	 = 0;
 	list.blockBegin[0] = 0;
+	for (int e = 0; e < 6; e++) list.box[e] = list.cbox[e] = emptyBound(e); // k_root_bounds fills them
 	list.blockBegin[1] = (n + kChunk - 1) / kChunk;
 	small[0]		 = SmallTask{0, 0, n, 1, 0};
 	*ctl			 = LevelCtl{large ? 1 : 0, (n + kChunk - 1) / kChunk, large ? 0 : 1, large ? 1 : 2 * n - 1, 0};
@@ -527,6 +577,10 @@ __global__ void __launch_bounds__(1024) k_level_next(Level L, int nNodes, LevelL
 				next.count[at.x]	  = c[k];
 				next.node[at.x]		  = node;
 				next.blockBegin[at.x] = at.y;
+				for (int e = 0; e < 6; e++) {
+					next.box[6 * at.x + e]	= L.childBox[24 * t + 12 * k + e];
+					next.cbox[6 * at.x + e] = L.childBox[24 * t + 12 * k + 6 + e];
+				}
 				at.x++;
 				at.y += (c[k] + kChunk - 1) / kChunk;
 			} else {
@@ -930,11 +984,10 @@ int buildBvh4Device(const float *pos, int64_t nVerts, const int32_t *idx, int64_
 		nRange = m.take<int2>(maxNodes2);
 		for (int k = 0; k < 2; k++) {
 			refs[k] = m.take<int>((size_t) n);
-			list[k] = LevelList{m.take<int>(maxT), m.take<int>(maxT), m.take<int>(maxT), m.take<int>(maxT + 1)};
+			list[k] = LevelList{m.take<int>(maxT), m.take<int>(maxT), m.take<int>(maxT), m.take<int>(maxT + 1), m.take<int>(6 * maxT), m.take<int>(6 * maxT)};
 		}
 		L		   = Level{};
-		L.box	   = m.take<int>(6 * maxT);
-		L.cbox	   = m.take<int>(6 * maxT);
+		L.childBox = m.take<int>(24 * maxT);
 		L.bins	   = m.take<Bins>(maxT);
 		L.decision = m.take<int>(maxT);
 		L.axis	   = m.take<int>(maxT);
@@ -942,7 +995,7 @@ int buildBvh4Device(const float *pos, int64_t nVerts, const int32_t *idx, int64_
 		L.nLeft	   = m.take<int>(maxT);
 		L.blockNode	 = m.take<int>(maxB);
 		L.blockStart = m.take<int>(maxB);
-		L.blockLeft	 = m.take<int>(maxB);
+		L.blockCnt	 = m.take<int>(3 * NB * maxB);
 		small		 = m.take<SmallTask>((size_t) n);
 		ctl			 = m.take<LevelCtl>(1);
 		total		 = m.take<int>(1);
@@ -963,6 +1016,9 @@ int buildBvh4Device(const float *pos, int64_t nVerts, const int32_t *idx, int64_
 	const Nodes2 N{nLo, nHi, nRange};
 	hipLaunchKernelGGL(k_prim_boxes, dim3((n + 255) / 256), dim3(256), 0, st, dPos, dIdx, n, pLo, pHi, refs[0]);
 	hipLaunchKernelGGL(k_level_init, dim3(1), dim3(1), 0, st, list[0], small, ctl, n);
+
+	if (n > kSmall)
+		hipLaunchKernelGGL(k_root_bounds, dim3(std::min(kRootBlocks, (n + kThreads - 1) / kThreads)), dim3(kThreads), 0, st, P, n, list[0].box, list[0].cbox);
 	BVHD_HIP(hipGetLastError());
 
 	// ---- large nodes, level by level: the lists stay on the device, the host
@@ -983,13 +1039,13 @@ int buildBvh4Device(const float *pos, int64_t nVerts, const int32_t *idx, int64_
 		L.count		 = list[cur].count;
 		L.node		 = list[cur].node;
 		L.blockBegin = list[cur].blockBegin;
+		L.box		 = list[cur].box;
+		L.cbox		 = list[cur].cbox;
 		const int *in = refs[levels & 1];
 		int *to		  = refs[(levels & 1) ^ 1];
 		hipLaunchKernelGGL(k_level_reset, dim3(T), dim3(256), 0, st, L, T);
-		hipLaunchKernelGGL(k_level_bounds, dim3(B), dim3(kThreads), 0, st, L, P, in);
 		hipLaunchKernelGGL(k_level_bins, dim3(B), dim3(kThreads), 0, st, L, P, in);
 		hipLaunchKernelGGL(k_level_split, dim3(T), dim3(64), 0, st, L, T, cost, maxLeaf);
-		hipLaunchKernelGGL(k_level_count, dim3(B), dim3(kThreads), 0, st, L, P, in);
 		hipLaunchKernelGGL(k_level_scatter, dim3(B), dim3(kThreads), 0, st, L, P, in, to);
 		hipLaunchKernelGGL(k_level_next, dim3(1), dim3(1024), 0, st, L, T, list[cur ^ 1], small, (levels & 1) ^ 1, N, ctl);
 		BVHD_HIP(hipGetLastError());

@@ -158,3 +158,11 @@ def test_subtree_sizes(krr, oracle, gpu, n, kind):
     assert infod["leaf_tris"] == n
     _assert_same_hits(gd, oracle.trace_closest(desc, rays))
     assert np.array_equal(vd, oracle.trace_any(desc, rays))
+
+
+@pytest.mark.parametrize("n", [2047, 2048, 2049, 3072, 4097, 9000])
+@pytest.mark.parametrize("kind", ["spread", "grid", "one_point"])
+def test_level_sizes(krr, oracle, gpu, n, kind):
+    """Nodes of several blocks of 1,024 references, whole and ragged, split by
+    bins and in the middle, with large and small children: as above."""
+    test_subtree_sizes(krr, oracle, gpu, n, kind)
