@@ -141,7 +141,7 @@ def test_nrc_on_1080p_field(krr, gpu):
 
 
 @pytest.mark.parametrize("res,sigma_t", [([1, 1, 1], [3.0, 3.0, 3.0]), ([2, 3, 2], [4.0, 4.0, 4.0]), ([5, 4, 6], [1.0, 4.0, 2.5]), ([5, 4, 6], [2.0, 2.0, 5.0])])
-def test_small_grid_media_match_checker(krr, oracle, gpu, res, sigma_t):
+def test_small_grid_media_match_oracle(krr, oracle, gpu, res, sigma_t):
     """Grids whose lookups are all, partly or never on the border, with empty
     voxels, grey media (one exponential for the three channels) and coloured
     ones."""

@@ -3,7 +3,7 @@
 Scenes of generated meshes around the block sizes the records are made in,
 with and without vertex normals, no light, one or many emissive triangles
 (normals agreeing with the winding and against it), beside an infinite light:
-both integrators against the checker.
+both integrators against the oracle.
 """
 import numpy as np
 import pytest
@@ -42,7 +42,7 @@ def _scene(krr, n, lights, flip, sky):
 
 @pytest.mark.parametrize("n,lights,flip,sky", [(1, 1, False, False), (2, 0, False, True), (255, 2, False, True), (256, 63, True, False),
                                                (257, 64, False, False), (700, 65, True, True)])
-def test_records_match_checker(krr, oracle, gpu, n, lights, flip, sky):
+def test_records_match_oracle(krr, oracle, gpu, n, lights, flip, sky):
     print(f"case: {n} triangles, {lights} lights, flip={flip}, sky={sky}", flush=True)
     s = _scene(krr, n, lights, flip, sky)
     g, gs = gpu_render(krr, gpu, s, 40, 30, {"spp": 2, "max_depth": 6}, frame_index=2)

@@ -106,7 +106,7 @@ def test_watertight_vertices_and_edges(krr, oracle, gpu):
 
 
 def test_full_scene_bvh_matches_checker_bvh(krr, oracle, gpu):
-    """1024 icospheres (1.31 M triangles): GPU hits equal the checker's own
+    """1024 icospheres (1.31 M triangles): GPU hits equal the oracle's own
     (independently built) BVH, itself pinned to brute force above."""
     print("case: 1.31M-triangle closest", flush=True)
     s = krr.Scene(icosphere_scene())
