@@ -1717,6 +1717,12 @@ struct PathGrid {
 	bool ordered = true;
 };
 
+// A persistent launch as a frame makes it: blocks, lanes of each wave that take
+// up paths, samples of a pixel one after the other.
+struct LaunchShape {
+	int blocks = 0, lanes = 0, samples = 0;
+};
+
 PathGrid pathGrid(int resident, int tb, int64_t paths, bool smallTree) {
 	PathGrid g;
 	const int64_t waves = (int64_t) resident * (tb / 64) / (smallTree ? 2 : 1);
@@ -1862,6 +1868,7 @@ struct krr_wf {
 	bool gridDense = false; // which form of the refill launch the grids were sized for
 	int gClosest = 1, gShadow = 1, gShade = 1;
 	PathGrid gMega;
+	LaunchShape lastShape; // of the last frame's persistent launch
 	bool beginPending	= false;
 	hipStream_t lastStream = nullptr;
 	krr_stats stats{};
@@ -2258,6 +2265,21 @@ int ldsNodeCount(const krr_wf *wf) {
 	return (int) std::min<int64_t>(wf->ldsNodes, wf->accel.nNodes);
 }
 
+// With every depth in the persistent launch, one launch runs all samples of
+// the frame; the radiance cache answers its queries between samples.  Paths of a
+// ray queue (camera = false) fill waves, a sample at a time.
+LaunchShape launchShape(const krr_wf *wf, const PathGrid &g, bool camera, bool nrc) {
+	return LaunchShape{g.blocks, camera ? g.lanes : 64, camera && !nrc ? wf->spp : 1};
+}
+
+Json shapeJson(const LaunchShape &s) {
+	Json o = Json::object();
+	o.set("blocks", Json((double) s.blocks));
+	o.set("lanes", Json((double) s.lanes));
+	o.set("samples", Json((double) s.samples));
+	return o;
+}
+
 // Kernel parameters of one frame (integrator.cpp:205-267 values).
 WfParams frameParams(const krr_wf *wf, int W, int H, int N, uint64_t frameIndex) {
 	WfParams P;
@@ -2583,6 +2605,7 @@ int krr_wf_get_params(const krr_wf *wf, char *buf, int32_t cap) {
 	j.set("bvh_builder", Json(std::string(wf->deviceBuilder ? "device" : "host")));
 	j.set("node_format", Json(std::string(wf->quantizedNodes ? "quantized" : "float")));
 	j.set("graph", Json(wf->useGraph));
+	if (wf->lastShape.blocks > 0) j.set("launch_in_force", shapeJson(wf->lastShape)); // of the last frame
 	if (wf->nrcOn) {
 		Json n = Json::object();
 		n.set("train_mod", Json((double) wf->nrcTrainMod));
@@ -2640,6 +2663,71 @@ int krr_wf_begin_frame(krr_wf *wf, const krr_camera *camera, uint64_t frame_inde
 	return KRR_OK;
 }
 
+} // extern "C"
+
+namespace {
+
+// How a frame of one camera is launched: what the kernels' variants depend on,
+// and with every depth in the persistent launch its shape.
+struct FrameLaunch {
+	TraceBvh bvh;
+	size_t lds;
+	bool media, count, plain, refill, dense;
+	PathGrid grid, gridNrc;
+	LaunchShape shape; // without the radiance cache's kernels
+};
+
+// The launch of a frame of N paths: krr_wf_render's, and the one the
+// autotuner times.  Grid sizes are computed once per shape, and the traversal
+// stack's overflow area is grown to hold them.
+int frameLaunch(krr_wf *wf, int N, FrameLaunch &L) {
+	wf->accel.stackLds = wf->stackLdsEntries; // before dev(): the kernels' LDS stack depth must match lds below
+	L.bvh			   = wf->accel.dev();
+	const int bs	   = wf->blockSize;
+	const unsigned gN  = (unsigned) ((N + bs - 1) / bs);
+	const int tb	   = wf->traceBlockSize;
+	const int gTmax	   = (N + tb - 1) / tb;
+	L.lds			   = stackLds(wf->accel, tb);
+	if ((size_t) (L.bvh.stackLds + kStackPad) * tb * sizeof(int) != L.lds) return krr::fail(KRR_ERR_INVALID_ARG, "krr_wf_render: stack layout mismatch");
+	L.count	 = wf->countTraversal;
+	L.media	 = wf->enableMedium && wf->sceneHasMedia;
+	L.plain	 = !wf->sceneTextured;
+	L.refill = refillLanesOf(wf) > 0;
+	L.dense	 = denseRefill(wf->accel, N);
+	const bool count = L.count, media = L.media;
+	const size_t lds = L.lds;
+	// persistent grid sizes (resident blocks), computed once per shape
+	const uint64_t shapeKey = ((uint64_t) N << 24) ^ ((uint64_t) tb << 12) ^ ((uint64_t) bs << 2) ^ ((uint64_t) wf->accel.stackSize << 50) ^ ((uint64_t) wf->stackLdsEntries << 43) ^
+							  (count ? 2 : 0) ^ (media ? 1 : 0) ^ (wf->nrcOn ? 4 : 0) ^ (L.plain ? 8 : 0) ^ (L.refill ? 16 : 0) ^
+							  ((uint64_t) ldsNodeCount(wf) << 5) ^ ((uint64_t) (wf->occupancy * 1024.f) << 32);
+	if (shapeKey != wf->gridKey || L.dense != wf->gridDense) {
+		// Counting variants use more registers: size each grid for the variant launched.
+		wf->gClosest = count ? persistentGrid(k_trace_closest_queue<true>, tb, lds, gTmax) : persistentGrid(k_trace_closest_queue<false>, tb, lds, gTmax);
+		if (media) wf->gShadow = count ? persistentGrid(k_shadow_tr<true>, tb, lds, gTmax) : persistentGrid(k_shadow_tr<false>, tb, lds, gTmax);
+		else wf->gShadow = count ? persistentGrid(k_trace_shadow<true>, tb, lds, gTmax) : persistentGrid(k_trace_shadow<false>, tb, lds, gTmax);
+		wf->gShade = media ? persistentGrid(k_shade<true>, bs, 0, (int) gN) : persistentGrid(k_shade<false>, bs, 0, (int) gN);
+		const size_t nodeBytes = (size_t) ldsNodeCount(wf) * sizeof(Bvh4Node);
+		auto mega = [&](bool nrc) {
+			const int resident = withMega<false>(media, count, nrc, L.plain, L.refill, L.dense, [&](auto k) { return decltype(k)::grid(tb, lds, 1 << 20, nodeBytes); });
+			return pathGrid(scaledGrid(resident, wf->occupancy), tb, N, !media && !L.refill);
+		};
+		wf->gMega = mega(false);
+		if (wf->nrcOn) wf->gMegaNrc = mega(true);
+		const int gMax = std::max(std::max(std::max(wf->gClosest, wf->gShadow), wf->gMega.blocks), wf->nrcOn ? wf->gMegaNrc.blocks : 0);
+		if (int rc = reserveOverflow(wf->ovf, wf->accel, (size_t) gMax * tb)) return rc;
+		wf->gridKey	  = shapeKey;
+		wf->gridDense = L.dense;
+	}
+	L.grid	  = wf->gMega;
+	L.gridNrc = wf->gMegaNrc;
+	L.shape	  = launchShape(wf, L.grid, wf->wavefrontDepths == 0, wf->nrcOn);
+	return KRR_OK;
+}
+
+} // namespace
+
+extern "C" {
+
 int krr_wf_render(krr_wf *wf, float *film_dev, void *hip_stream) {
 	krr::clearError();
 	if (!wf) return krr::fail(KRR_ERR_INVALID_ARG, "krr_wf_render: null handle");
@@ -2656,41 +2744,14 @@ int krr_wf_render(krr_wf *wf, float *film_dev, void *hip_stream) {
 					 wf->plen.as<uint8_t>()};
 	ShadowQueueDev sq{wf->shadowRay.as<float4>(), wf->shadowC.as<float4>(), wf->shadowExt.as<float4>()};
 	Counters *cnt	   = wf->counters.as<Counters>();
-	wf->accel.stackLds = wf->stackLdsEntries; // before dev(): the kernels' LDS stack depth must match lds below
-	const TraceBvh bvh = wf->accel.dev();
+	FrameLaunch L;
+	if (int rc = frameLaunch(wf, N, L)) return rc;
+	const TraceBvh bvh = L.bvh;
 	const int bs	   = wf->blockSize;
 	const unsigned gN  = (unsigned) ((N + bs - 1) / bs);
 	const int tb	   = wf->traceBlockSize;
-	const int gTmax	   = (N + tb - 1) / tb;
-	const size_t lds   = stackLds(wf->accel, tb);
-	if ((size_t) (bvh.stackLds + kStackPad) * tb * sizeof(int) != lds) return krr::fail(KRR_ERR_INVALID_ARG, "krr_wf_render: stack layout mismatch");
-	const bool count   = wf->countTraversal;
-	const bool media   = wf->enableMedium && wf->sceneHasMedia;
-	const bool plain   = !wf->sceneTextured;
-	const bool refill  = refillLanesOf(wf) > 0;
-	const bool dense   = denseRefill(wf->accel, N);
-	// persistent grid sizes (resident blocks), computed once per shape
-	const uint64_t shapeKey = ((uint64_t) N << 24) ^ ((uint64_t) tb << 12) ^ ((uint64_t) bs << 2) ^ ((uint64_t) wf->accel.stackSize << 50) ^ ((uint64_t) wf->stackLdsEntries << 43) ^
-							  (count ? 2 : 0) ^ (media ? 1 : 0) ^ (wf->nrcOn ? 4 : 0) ^ (plain ? 8 : 0) ^ (refill ? 16 : 0) ^
-							  ((uint64_t) ldsNodeCount(wf) << 5) ^ ((uint64_t) (wf->occupancy * 1024.f) << 32);
-	if (shapeKey != wf->gridKey || dense != wf->gridDense) {
-		// Counting variants use more registers: size each grid for the variant launched.
-		wf->gClosest = count ? persistentGrid(k_trace_closest_queue<true>, tb, lds, gTmax) : persistentGrid(k_trace_closest_queue<false>, tb, lds, gTmax);
-		if (media) wf->gShadow = count ? persistentGrid(k_shadow_tr<true>, tb, lds, gTmax) : persistentGrid(k_shadow_tr<false>, tb, lds, gTmax);
-		else wf->gShadow = count ? persistentGrid(k_trace_shadow<true>, tb, lds, gTmax) : persistentGrid(k_trace_shadow<false>, tb, lds, gTmax);
-		wf->gShade = media ? persistentGrid(k_shade<true>, bs, 0, (int) gN) : persistentGrid(k_shade<false>, bs, 0, (int) gN);
-		const size_t nodeBytes = (size_t) ldsNodeCount(wf) * sizeof(Bvh4Node);
-		auto mega = [&](bool nrc) {
-			const int resident = withMega<false>(media, count, nrc, plain, refill, dense, [&](auto k) { return decltype(k)::grid(tb, lds, 1 << 20, nodeBytes); });
-			return pathGrid(scaledGrid(resident, wf->occupancy), tb, N, !media && !refill);
-		};
-		wf->gMega = mega(false);
-		if (wf->nrcOn) wf->gMegaNrc = mega(true);
-		const int gMax = std::max(std::max(std::max(wf->gClosest, wf->gShadow), wf->gMega.blocks), wf->nrcOn ? wf->gMegaNrc.blocks : 0);
-		if (int rc = reserveOverflow(wf->ovf, wf->accel, (size_t) gMax * tb)) return rc;
-		wf->gridKey	  = shapeKey;
-		wf->gridDense = dense;
-	}
+	const size_t lds   = L.lds;
+	const bool count = L.count, media = L.media;
 	int *ovf = wf->ovf.as<int>();
 	const unsigned gTc = (unsigned) wf->gClosest, gTs = (unsigned) wf->gShadow, gS = (unsigned) wf->gShade;
 
@@ -2730,13 +2791,10 @@ int krr_wf_render(krr_wf *wf, float *film_dev, void *hip_stream) {
 		nrc.trainMod   = wf->nrcTrainMod;
 		nrc.phase	   = (int) (wf->frameIndex % (uint64_t) wf->nrcTrainMod);
 	}
-	// With every depth in the persistent launch, one launch runs all samples of
-	// the frame; the radiance cache answers its queries between samples.
-	const PathGrid &pg = wf->nrcOn ? wf->gMegaNrc : wf->gMega;
-	if (wf->wavefrontDepths == 0) {
-		P.fetchLanes = pg.lanes;
-		if (!wf->nrcOn) P.chain = wf->spp;
-	}
+	const PathGrid &pg = wf->nrcOn ? L.gridNrc : L.grid;
+	wf->lastShape	   = launchShape(wf, pg, wf->wavefrontDepths == 0, wf->nrcOn);
+	P.fetchLanes	   = wf->lastShape.lanes;
+	P.chain			   = wf->lastShape.samples;
 	if (!pg.ordered) px.order = nullptr;
 	for (int s = 0; s < wf->spp; s += P.chain) {
 		// with every depth in the persistent launch, it makes the camera rays itself
@@ -2760,7 +2818,7 @@ int krr_wf_render(krr_wf *wf, float *film_dev, void *hip_stream) {
 				timed(4, [&] {
 					const int camFetch = depth == 0 ? 1 : 0; // k_camera skipped: the kernel makes the camera rays
 					const int *cp	 = (const int *) &cnt->rayCount[cur];
-					withMega<false>(media, count, wf->nrcOn, plain, refill, dense, [&](auto k) {
+					withMega<false>(media, count, wf->nrcOn, L.plain, L.refill, L.dense, [&](auto k) {
 						decltype(k)::launch((unsigned) pg.blocks, tb, lds, st, P, wf->ds, bvh, cq, cp, px, ovf, cnt,
 											wf->nrcOn ? nrc : NrcDev{}, ViewsDev{}, depth, cam, camFetch);
 						return 0;
@@ -2843,6 +2901,7 @@ struct ViewsLaunch {
 	TraceBvh bvh;
 	size_t lds;
 	PathGrid grid;
+	LaunchShape shape;
 	bool media, count, nrc;
 };
 
@@ -2865,16 +2924,16 @@ int viewsLaunch(krr_wf *wf, int N, bool nrc, ViewsLaunch &L) {
 		if (int rc = reserveOverflow(wf->ovf, wf->accel, (size_t) wf->gMegaViews.blocks * tb)) return rc;
 		wf->viewsGridKey = key;
 	}
-	L.grid = wf->gMegaViews;
+	L.grid	= wf->gMegaViews;
+	L.shape = launchShape(wf, L.grid, true, wf->nrcOn);
 	return KRR_OK;
 }
 
 // Everything of one multi-view frame after the frame values are set:
 // beginFrame of all views, each sample in one persistent launch over all
 // views' pixels (plus the cache queries), accumulate, the cache's training,
-// the film write of every view.  `trial` stops after the first persistent
-// launch and writes no film (autotuner).
-int enqueueViews(krr_wf *wf, WfParams P, const ViewsLaunch &L, hipStream_t st, bool timing, bool trial) {
+// the film write of every view.
+int enqueueViews(krr_wf *wf, WfParams P, const ViewsLaunch &L, hipStream_t st, bool timing) {
 	const ViewsDev V = viewsDev(wf);
 	PixelStateDev px = viewsPx(wf);
 	Counters *cnt		   = wf->counters.as<Counters>();
@@ -2907,8 +2966,8 @@ int enqueueViews(krr_wf *wf, WfParams P, const ViewsLaunch &L, hipStream_t st, b
 	if (L.nrc) hipLaunchKernelGGL(k_nrc_begin, dim3(1), dim3(1), 0, st, cnt, wf->nrcBatch);
 	hipLaunchKernelGGL(k_begin_views, dim3(gN), dim3(wf->blockSize), 0, st, P, V, px);
 	int rc		 = KRR_OK;
-	P.fetchLanes = L.grid.lanes;
-	if (!L.nrc) P.chain = wf->spp; // as in krr_wf_render
+	P.fetchLanes = L.shape.lanes;
+	P.chain		 = L.shape.samples;
 	if (!L.grid.ordered) px.order = nullptr;
 	for (int s = 0; s < wf->spp; s += P.chain) {
 		hipLaunchKernelGGL(k_mega_begin, dim3(1), dim3(1), 0, st, cnt);
@@ -2929,7 +2988,6 @@ int enqueueViews(krr_wf *wf, WfParams P, const ViewsLaunch &L, hipStream_t st, b
 				return 0;
 			});
 		});
-		if (trial) return KRR_OK;
 		if (L.nrc) {
 			timed(5, [&] {
 				hipLaunchKernelGGL(k_nrc_targets, dim3(256), dim3(256), 0, st, nrc, (const int *) &cnt->nrcTrainDone, (const float4 *) px.L,
@@ -3040,6 +3098,7 @@ int krr_wf_render_views(krr_wf *wf, uint64_t frame_index, void *hip_stream) {
 	const WfParams P = frameParams(wf, 0, 0, wf->NV, frame_index);
 	ViewsLaunch L;
 	if (int rc = viewsLaunch(wf, wf->NV, wf->nrcOn, L)) return rc;
+	wf->lastShape = L.shape;
 	hipLaunchKernelGGL(k_set_frame, dim3(1), dim3(1), 0, st, wf->frameBuf.as<FrameDev>(), frameDev(wf, frame_index));
 	const bool timing = wf->timeKernels;
 	wf->spans.clear();
@@ -3053,7 +3112,7 @@ int krr_wf_render_views(krr_wf *wf, uint64_t frame_index, void *hip_stream) {
 			wf->dropGraph();
 			if (!wf->capStream) KRR_HIP(hipStreamCreateWithFlags(&wf->capStream, hipStreamNonBlocking));
 			KRR_HIP(hipStreamBeginCapture(wf->capStream, hipStreamCaptureModeThreadLocal));
-			int rc		 = enqueueViews(wf, P, L, wf->capStream, false, false);
+			int rc		 = enqueueViews(wf, P, L, wf->capStream, false);
 			hipGraph_t g = nullptr;
 			hipError_t e = hipStreamEndCapture(wf->capStream, &g);
 			if (rc || e != hipSuccess) {
@@ -3072,7 +3131,7 @@ int krr_wf_render_views(krr_wf *wf, uint64_t frame_index, void *hip_stream) {
 		KRR_HIP(hipGraphLaunch(wf->graphExec, st));
 	} else {
 		const int b = timing ? wf->mark(st) : -1;
-		if (int rc = enqueueViews(wf, P, L, st, timing, false)) return rc;
+		if (int rc = enqueueViews(wf, P, L, st, timing)) return rc;
 		if (timing) wf->spans.push_back({3, b, wf->mark(st)});
 	}
 	KRR_HIP(hipGetLastError());
@@ -3104,12 +3163,18 @@ int krr_wf_autotune(krr_wf *wf, int64_t trial_paths, char *report, int32_t cap, 
 		float occ;
 		int refill;
 		float ms;
+		LaunchShape shape;
 	};
 	std::vector<Trial> trials;
 	int rc = KRR_OK;
-	// One candidate: `runs` timed persistent launches over the first N paths
-	// of the frame (the views' pixels in order, or the first N pixels of the
-	// single view); the fastest run counts.
+	// One candidate: `runs` timed persistent launches over the first N pixels
+	// of the frame (the views' pixels in order, or those of the single view);
+	// the fastest run counts.  Each is the launch the whole frame makes at the
+	// candidate's settings (its kernel, blocks and lanes, and as many of its
+	// samples as trial_paths leave), but for the order of the paths, which trials
+	// of fewer paths than pixels have none of, and the radiance cache's
+	// recording.
+	auto samples = [&](const LaunchShape &shape) { return (int) std::min<int64_t>(shape.samples, std::max<int64_t>(1, trial_paths / N)); };
 	auto measure = [&](Trial &t, int runs) -> int {
 		wf->traceBlockSize	= t.tb;
 		wf->stackLdsEntries = t.lds;
@@ -3118,9 +3183,12 @@ int krr_wf_autotune(krr_wf *wf, int64_t trial_paths, char *report, int32_t cap, 
 		t.ms				= 1e30f;
 		for (int r = 0; r < runs; r++) {
 			if (views) {
-				const WfParams P = frameParams(wf, 0, 0, N, 1);
+				WfParams P = frameParams(wf, 0, 0, N, 1);
 				ViewsLaunch L;
-				if (int e = viewsLaunch(wf, N, false, L)) return e;
+				if (int e = viewsLaunch(wf, total, false, L)) return e;
+				t.shape		 = L.shape;
+				P.fetchLanes = t.shape.lanes;
+				P.chain		 = t.shape.samples = samples(L.shape);
 				hipLaunchKernelGGL(k_set_frame, dim3(1), dim3(1), 0, st, wf->frameBuf.as<FrameDev>(), frameDev(wf, 1));
 				// begin + one persistent launch, timed from its start
 				hipLaunchKernelGGL(k_reset_totals, dim3(1), dim3(1), 0, st, wf->counters.as<Counters>());
@@ -3138,27 +3206,24 @@ int krr_wf_autotune(krr_wf *wf, int64_t trial_paths, char *report, int32_t cap, 
 				});
 			} else {
 				WfParams P = frameParams(wf, wf->W, wf->H, N, wf->frameIndex);
-				wf->accel.stackLds = wf->stackLdsEntries;
-				const TraceBvh bvh = wf->accel.dev();
-				const size_t lds   = stackLds(wf->accel, t.tb);
-				const int maxBlocks = std::max(1, (N + t.tb - 1) / t.tb);
-				const size_t nodeBytes = (size_t) ldsNodeCount(wf) * sizeof(Bvh4Node);
-				int g = withMega<false>(media, false, false, !wf->sceneTextured, refillLanesOf(wf) > 0, denseRefill(wf->accel, N),
-										[&](auto k) { return decltype(k)::grid(t.tb, lds, maxBlocks, nodeBytes); });
-				g	  = scaledGrid(g, t.occ);
-				if (int e = reserveOverflow(wf->ovf, wf->accel, (size_t) g * t.tb)) return e;
+				FrameLaunch L;
+				if (int e = frameLaunch(wf, total, L)) return e;
+				const bool camera = wf->wavefrontDepths == 0; // else the first depths are launches of their own, and fill a queue
+				t.shape			  = L.shape;
+				P.fetchLanes	  = t.shape.lanes;
+				P.chain			  = t.shape.samples = samples(L.shape);
 				// trials may cover fewer paths than pixels: pixel order, no miss record
 				const PixelStateDev px{wf->L.as<float4>(), wf->pixel.as<float4>(), wf->rng.as<uint64_t>(), wf->channel.as<int>()};
 				Counters *cnt = wf->counters.as<Counters>();
 				const unsigned gN = (unsigned) ((N + 255) / 256);
 				hipLaunchKernelGGL(k_reset_totals, dim3(1), dim3(1), 0, st, cnt);
 				hipLaunchKernelGGL(k_begin_frame, dim3(gN), dim3(256), 0, st, P, px);
-				hipLaunchKernelGGL(k_camera, dim3(gN), dim3(256), 0, st, P, cameraDev(wf->cam), px, rayQueue(wf, 0), cnt);
+				if (!camera) hipLaunchKernelGGL(k_camera, dim3(gN), dim3(256), 0, st, P, cameraDev(wf->cam), px, rayQueue(wf, 0), cnt);
 				hipLaunchKernelGGL(k_mega_begin, dim3(1), dim3(1), 0, st, cnt);
 				KRR_HIP(hipEventRecord(e0, st));
-				withMega<false>(media, false, false, !wf->sceneTextured, refillLanesOf(wf) > 0, denseRefill(wf->accel, N), [&](auto k) {
-					decltype(k)::launch((unsigned) g, t.tb, lds, st, P, wf->ds, bvh, rayQueue(wf, 0), (const int *) &cnt->rayCount[0], px,
-										wf->ovf.as<int>(), cnt, NrcDev{}, ViewsDev{});
+				withMega<false>(L.media, false, false, L.plain, L.refill, L.dense, [&](auto k) {
+					decltype(k)::launch((unsigned) L.grid.blocks, t.tb, L.lds, st, P, wf->ds, L.bvh, rayQueue(wf, 0), (const int *) &cnt->rayCount[0], px,
+										wf->ovf.as<int>(), cnt, NrcDev{}, ViewsDev{}, 0, cameraDev(wf->cam), camera ? 1 : 0);
 					return 0;
 				});
 			}
@@ -3183,7 +3248,7 @@ int krr_wf_autotune(krr_wf *wf, int64_t trial_paths, char *report, int32_t cap, 
 	for (int ti = 0; ti < 3 && rc == KRR_OK; ti++)
 		for (int li = 0; li < 3 && rc == KRR_OK; li++)
 			for (int oi = 0; oi < 3 && rc == KRR_OK; oi++) {
-				Trial t{tbs[ti], ldss[li], occs[oi], refill0, 0.f};
+				Trial t{tbs[ti], ldss[li], occs[oi], refill0, 0.f, {}};
 				rc = measure(t, 3);
 				if (rc == KRR_OK) trials.push_back(t);
 			}
@@ -3191,7 +3256,7 @@ int krr_wf_autotune(krr_wf *wf, int64_t trial_paths, char *report, int32_t cap, 
 		const Trial shape = *std::min_element(trials.begin(), trials.end(), [](const Trial &a, const Trial &b) { return a.ms < b.ms; });
 		for (const int r : {0, 4, kDefaultRefillLanes, 12, 16}) {
 			if (r == refill0 || rc != KRR_OK) continue;
-			Trial t{shape.tb, shape.lds, shape.occ, r, 0.f};
+			Trial t{shape.tb, shape.lds, shape.occ, r, 0.f, {}};
 			rc = measure(t, 3);
 			if (rc == KRR_OK) trials.push_back(t);
 		}
@@ -3212,25 +3277,21 @@ int krr_wf_autotune(krr_wf *wf, int64_t trial_paths, char *report, int32_t cap, 
 	wf->gridKey = wf->viewsGridKey = ~0ull; // grids and the recorded frame follow the new shape
 	wf->dropGraph();
 	if (!views) wf->beginPending = true; // the trials used the frame's pixel state: seed it again
-	Json j = Json::object(), arr = Json::array();
-	for (const Trial &t : trials) {
+	auto entry = [](const Trial &t) {
 		Json o = Json::object();
 		o.set("trace_block_size", Json((double) t.tb));
 		o.set("stack_lds_entries", Json((double) t.lds));
 		o.set("occupancy", Json((double) t.occ));
 		o.set("refill_lanes", Json((double) t.refill));
 		o.set("ms", Json((double) t.ms));
-		arr.push(o);
-	}
-	Json b = Json::object();
-	b.set("trace_block_size", Json((double) best.tb));
-	b.set("stack_lds_entries", Json((double) best.lds));
-	b.set("occupancy", Json((double) best.occ));
-	b.set("refill_lanes", Json((double) best.refill));
-	b.set("ms", Json((double) best.ms));
+		o.set("launch", shapeJson(t.shape));
+		return o;
+	};
+	Json j = Json::object(), arr = Json::array();
+	for (const Trial &t : trials) arr.push(entry(t));
 	j.set("trial_paths", Json((double) N));
 	j.set("candidates", arr);
-	j.set("best", b);
+	j.set("best", entry(best));
 	const std::string out = j.dump();
 	if (report && cap > 0) {
 		const size_t n = std::min((size_t) cap - 1, out.size());
