@@ -1733,6 +1733,14 @@ PathGrid pathGrid(int resident, int tb, int64_t paths, bool smallTree) {
 	return g;
 }
 
+// Launch over a ray queue ("wavefront_depths"), whose rays fill waves: no more
+// blocks than the queue can hold rays for.
+PathGrid queueGrid(int resident, int tb, int64_t rays) {
+	PathGrid g;
+	g.blocks = (int) std::max<int64_t>(1, std::min<int64_t>(resident, (rays + tb - 1) / tb));
+	return g;
+}
+
 // A fraction of a persistent grid (at least one block).
 int scaledGrid(int g, float frac) { return std::max(1, (int) std::lround((double) g * (double) frac)); }
 
@@ -2266,10 +2274,10 @@ int ldsNodeCount(const krr_wf *wf) {
 }
 
 // With every depth in the persistent launch, one launch runs all samples of
-// the frame; the radiance cache answers its queries between samples.  Paths of a
-// ray queue (camera = false) fill waves, a sample at a time.
+// the frame; the radiance cache answers its queries between samples, and a ray
+// queue (camera = false) holds one sample's paths.
 LaunchShape launchShape(const krr_wf *wf, const PathGrid &g, bool camera, bool nrc) {
-	return LaunchShape{g.blocks, camera ? g.lanes : 64, camera && !nrc ? wf->spp : 1};
+	return LaunchShape{g.blocks, g.lanes, camera && !nrc ? wf->spp : 1};
 }
 
 Json shapeJson(const LaunchShape &s) {
@@ -2709,6 +2717,7 @@ int frameLaunch(krr_wf *wf, int N, FrameLaunch &L) {
 		const size_t nodeBytes = (size_t) ldsNodeCount(wf) * sizeof(Bvh4Node);
 		auto mega = [&](bool nrc) {
 			const int resident = withMega<false>(media, count, nrc, L.plain, L.refill, L.dense, [&](auto k) { return decltype(k)::grid(tb, lds, 1 << 20, nodeBytes); });
+			if (wf->wavefrontDepths > 0) return queueGrid(scaledGrid(resident, wf->occupancy), tb, N);
 			return pathGrid(scaledGrid(resident, wf->occupancy), tb, N, !media && !L.refill);
 		};
 		wf->gMega = mega(false);
