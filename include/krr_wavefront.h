@@ -290,7 +290,9 @@ typedef struct krr_wf krr_wf;
  *   nee (true), enable_medium (true), max_depth (10), rr (0.8),
  *   enable_clamp (false), clamp_max (1e3)
  * plus keys this library adds:
- *   spp (1)              samples per pixel per frame (UI-only in the reference)
+ *   spp (1)              samples per pixel per frame (UI-only in the
+ *                        reference); a launch runs up to 256 of them, and
+ *                        2^28 paths
  *   rr_min_depth (0)     first path depth at which Russian roulette applies
  *   legacy_spp_accumulate (false)  keep the reference's running-sum spp loop
  *   count_traversal (false)  count node visits / triangle tests
@@ -413,7 +415,7 @@ int krr_mk_destroy(krr_mk *mk);
 /* ---------------------------------------------------------------------- */
 /* Many camera views in one frame.  No reference counterpart: KiRaRay        */
 /* renders one view per frame (integrator.cpp:205-267); this batches views   */
-/* of uneven sizes into one persistent launch per sample.                    */
+/* of uneven sizes into one persistent launch.                               */
 /* ---------------------------------------------------------------------- */
 
 typedef struct krr_view {
@@ -426,8 +428,8 @@ typedef struct krr_view {
  * state for all views, at most 2^30 pixels in total. */
 int krr_wf_set_views(krr_wf *wf, const krr_view *views, int32_t n_views);
 /* One frame of every view: beginFrame + render (integrator.cpp:205-267) of
- * each view, all views' pixels in one persistent launch per sample, films
- * written.  View v seeds pixel (x, y) with PCG initstate
+ * each view, all views' pixels and samples in one persistent launch (or several,
+ * see spp; with the radiance cache one per sample), films written.  View v seeds pixel (x, y) with PCG initstate
  * interleave(x, y) | v << 32, so view 0 renders exactly what krr_wf_render
  * renders for the same camera, size and frame index.  With "graph" the
  * launches are recorded once (per views / scene / launch shape) and replayed;

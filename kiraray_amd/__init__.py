@@ -184,7 +184,7 @@ class WavefrontPathTracer:
 
     def set_views(self, views):
         """views: iterable of (camera, width, height, film_ptr); all are
-        rendered by render_views in one persistent launch per sample."""
+        rendered by render_views in one persistent launch."""
         views = list(views)
         arr = (krr_view * len(views))()
         for i, (cam, w, h, film) in enumerate(views):

@@ -2273,11 +2273,20 @@ int ldsNodeCount(const krr_wf *wf) {
 	return (int) std::min<int64_t>(wf->ldsNodes, wf->accel.nNodes);
 }
 
-// With every depth in the persistent launch, one launch runs all samples of
-// the frame; the radiance cache answers its queries between samples, and a ray
-// queue (camera = false) holds one sample's paths.
-LaunchShape launchShape(const krr_wf *wf, const PathGrid &g, bool camera, bool nrc) {
-	return LaunchShape{g.blocks, g.lanes, camera && !nrc ? wf->spp : 1};
+// With every depth in the persistent launch, a launch runs several samples of
+// the frame's N pixels; the radiance cache answers its queries between samples,
+// and a ray queue (camera = false) holds one sample's paths.
+//
+// A launch is not interrupted, so what it runs is bounded, by the samples a lane
+// chains and by the paths: 129 samples of a 1080p frame of the 1.31 M-triangle
+// field are one launch of 0.31 s, 256 of the 720p volume one of about 1.1 s (2 take 8.5 ms).  Every
+// launch waits for its longest pixel: 256 samples of the 256x256 Cornell box
+// take 24.6 ms in one launch and 26.9 ms in four.
+constexpr int kLaunchSamples	= 256;
+constexpr int64_t kLaunchPaths = (int64_t) 1 << 28;
+LaunchShape launchShape(const krr_wf *wf, const PathGrid &g, int N, bool camera, bool nrc) {
+	const int64_t most = std::min<int64_t>(kLaunchSamples, std::max<int64_t>(1, kLaunchPaths / N));
+	return LaunchShape{g.blocks, g.lanes, camera && !nrc ? (int) std::min<int64_t>(wf->spp, most) : 1};
 }
 
 Json shapeJson(const LaunchShape &s) {
@@ -2729,7 +2738,7 @@ int frameLaunch(krr_wf *wf, int N, FrameLaunch &L) {
 	}
 	L.grid	  = wf->gMega;
 	L.gridNrc = wf->gMegaNrc;
-	L.shape	  = launchShape(wf, L.grid, wf->wavefrontDepths == 0, wf->nrcOn);
+	L.shape	  = launchShape(wf, L.grid, N, wf->wavefrontDepths == 0, wf->nrcOn);
 	return KRR_OK;
 }
 
@@ -2801,11 +2810,11 @@ int krr_wf_render(krr_wf *wf, float *film_dev, void *hip_stream) {
 		nrc.phase	   = (int) (wf->frameIndex % (uint64_t) wf->nrcTrainMod);
 	}
 	const PathGrid &pg = wf->nrcOn ? L.gridNrc : L.grid;
-	wf->lastShape	   = launchShape(wf, pg, wf->wavefrontDepths == 0, wf->nrcOn);
+	wf->lastShape	   = launchShape(wf, pg, N, wf->wavefrontDepths == 0, wf->nrcOn);
 	P.fetchLanes	   = wf->lastShape.lanes;
-	P.chain			   = wf->lastShape.samples;
 	if (!pg.ordered) px.order = nullptr;
 	for (int s = 0; s < wf->spp; s += P.chain) {
+		P.chain = std::min(wf->lastShape.samples, wf->spp - s);
 		// with every depth in the persistent launch, it makes the camera rays itself
 		if (wf->wavefrontDepths > 0) hipLaunchKernelGGL(k_camera, dim3(gN), dim3(bs), 0, st, P, cam, px, rayQueue(wf, 0), cnt);
 		for (int depth = 0; depth <= wf->maxDepth; depth++) {
@@ -2934,7 +2943,7 @@ int viewsLaunch(krr_wf *wf, int N, bool nrc, ViewsLaunch &L) {
 		wf->viewsGridKey = key;
 	}
 	L.grid	= wf->gMegaViews;
-	L.shape = launchShape(wf, L.grid, true, wf->nrcOn);
+	L.shape = launchShape(wf, L.grid, N, true, wf->nrcOn);
 	return KRR_OK;
 }
 
@@ -2976,9 +2985,9 @@ int enqueueViews(krr_wf *wf, WfParams P, const ViewsLaunch &L, hipStream_t st, b
 	hipLaunchKernelGGL(k_begin_views, dim3(gN), dim3(wf->blockSize), 0, st, P, V, px);
 	int rc		 = KRR_OK;
 	P.fetchLanes = L.shape.lanes;
-	P.chain		 = L.shape.samples;
 	if (!L.grid.ordered) px.order = nullptr;
 	for (int s = 0; s < wf->spp; s += P.chain) {
+		P.chain = std::min(L.shape.samples, wf->spp - s);
 		hipLaunchKernelGGL(k_mega_begin, dim3(1), dim3(1), 0, st, cnt);
 		if (L.grid.ordered) { // the order of this sample's camera paths, from the last sample's path lengths (k_tile_keys)
 			const int nT = wf->vTiles, nBlk = (nT + kTileBlock - 1) / kTileBlock;

@@ -36,3 +36,38 @@ def test_queue_launches_are_no_larger_than_the_queue(krr, gpu, w, h):
     assert la == {"blocks": (w * h + 127) // 128, "lanes": 64, "samples": 1}
     assert lb["blocks"] > la["blocks"] and lb["lanes"] < 64 and lb["samples"] == 2
     assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("scene,spp,more", [("cornell", 257, {}), ("cornell", 300, {"legacy_spp_accumulate": True}), ("field", 256, {"refill_lanes": 8}),
+                                            ("field", 513, {"refill_lanes": 8})])
+def test_launches_run_a_bounded_number_of_samples(krr, gpu, scene, spp, more):
+    """A launch runs at most 256 samples of a pixel; the next one goes on with
+    the pixel's sampler and sum, so the film is that of a launch per sample."""
+    print(f"case: {scene} 31x17 {spp} spp {more}", flush=True)
+    s = krr.Scene(CORNELL if scene == "cornell" else icosphere_scene(count=64, level=2, res=(31, 17)))
+    params = dict({"spp": spp, "max_depth": 4}, **more)
+    a, la, sa = _frame(krr, gpu, s, 31, 17, params)
+    b, _, sb = _frame(krr, gpu, s, 31, 17, dict(params, wavefront_depths=1))
+    assert la["samples"] == min(spp, 256)
+    assert sa["closest_launches"] == -(-spp // 256)
+    assert sa["closest_rays"] == sb["closest_rays"] and sa["shadow_rays"] == sb["shadow_rays"]
+    assert np.array_equal(a, b)
+
+
+def test_views_run_a_bounded_number_of_samples(krr, gpu):
+    print("case: views, 260 spp", flush=True)
+    s = krr.Scene(icosphere_scene(count=64, level=2, res=(31, 17)))
+    a, _, sa = _frame(krr, gpu, s, 31, 17, {"spp": 260, "max_depth": 4})
+    for graph in (True, False):
+        wf = krr.WavefrontPathTracer({"spp": 260, "max_depth": 4, "graph": graph})
+        wf.set_scene(s)
+        film = gpu.DeviceBuffer(31 * 17 * 16)
+        wf.set_views([(s.camera(0), 31, 17, film.ptr)])
+        for _ in range(3):  # replays
+            wf.render_views(3, 0)
+            gpu.synchronize()
+            assert np.array_equal(a, film.to_numpy(np.float32, (17, 31, 4)))
+        st = wf.stats()
+        assert st["closest_launches"] == 2 and st["closest_rays"] == sa["closest_rays"]
+        assert wf.to_json()["launch_in_force"]["samples"] == 256
+        wf.close()
