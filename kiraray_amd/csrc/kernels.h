@@ -298,7 +298,7 @@ KRR_DEV RayItem cameraRay(const CameraDev &cam, int W, int H, int x, int y, Pcg 
 // This lane's traversal stack: its wave's rows of the block's LDS, overflow
 // slots of the grid (ovf holds (stack size - bvh.stackLds) * grid threads ints).
 KRR_DEV LaneStack laneStack(const TraceBvh &bvh, int *lds, int *ovf) {
-	return LaneStack{lds + (threadIdx.x >> 6) * (bvh.stackLds + kStackPad) * 64 + (threadIdx.x & 63),
+	return LaneStack{lds + (threadIdx.x >> 6) * stackRows(bvh.stackLds) * 64 + (threadIdx.x & 63),
 					 ovf + (size_t) blockIdx.x * blockDim.x + threadIdx.x, (int) (gridDim.x * blockDim.x), bvh.stackLds};
 }
 

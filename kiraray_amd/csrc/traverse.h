@@ -4,8 +4,8 @@
 // Each lane traverses its own ray through the 4-wide BVH (bvh.h): one node
 // fetch = seven 16-byte loads of one 128-byte line, four slab tests, hit
 // children (inner nodes and leaves) sorted front to back with the far ones
-// pushed on a per-lane stack in LDS (stride = block size, so the 64 lanes of
-// a wave hit 64 different banks); a leaf is one more step of the loop.
+// pushed on a per-lane stack in LDS (rows of a wave's 64 lanes, which hit 64
+// different banks); a leaf is one more step of the loop.
 //
 // Hit rule (shared with the CPU checker): the Woop-Benthin-Wald watertight
 // test (JCGT 2(1), 2013), hit iff t > 0 and t < tbest, or t == tbest with a
@@ -185,21 +185,22 @@ struct TraceResult {
 // keeps the traversal kernels at high occupancy; deep stacks are rare but stay
 // exact.  nLds is uniform over the launch.
 //
-// Each wave owns nLds + kStackPad rows of 64 ints, lane-fastest, so a wave's
-// 64 lanes hit 64 banks, entry e of a lane is e * 256 bytes from its first, and
-// the three entries a node can push go to constant offsets from one address.
+// Each wave owns nLds + 1 rows of 64 ints, lane-fastest, so a wave's 64 lanes
+// hit 64 banks, entry e of a lane is e * 256 bytes from its first, and the
+// three entries a node can push go to constant offsets from one address.
 // A push writes all three rows whatever the number of children to keep: the
-// valid ones come first, the rows above are overwritten by later pushes, and
-// the pad rows take them at the top of the area.  Lanes past nLds send their
-// wave through a path that also serves the overflow area; the common path has
-// one compare for it.  (A push at a time, each with its own address, bound and
+// valid ones come first, and the rows above are overwritten by later pushes.
+// A lane with fewer than three rows left sends its wave through a path that
+// also serves the overflow area; the common path has one compare for it.  (The
+// last row is read, and the value dropped, by lanes that pop from the overflow
+// area.)  (A push at a time, each with its own address, bound and
 // branch, took 21 vector instructions for the three; this takes 10.)  With the
 // loops per node kind below: 2^20 incoherent closest and 2^20 shadow rays in the
 // 1.31 M-triangle field 1369 against 1550 us, the 36-triangle Cornell box at
 // 256x256, 16 samples 3.91 against 4.18 ms, the field's 1080p frame 3.72
 // against 3.77 ms.
 constexpr int kShortStack = 16;
-constexpr int kStackPad	  = 3;
+constexpr int stackRows(int nLds) { return nLds + 1; }
 struct LaneStack {
 	int *lds; // this lane's entry 0
 	int *ovf;
@@ -214,7 +215,7 @@ struct LaneStack {
 	KRR_DEV void push(int &sp, bool h1, bool h2, bool h3, int c1, int c2, int c3) const {
 		const int e0 = h3 ? c3 : (h2 ? c2 : c1), e1 = h3 ? c2 : c1;
 		const int n	 = sp + (h1 ? 1 : 0) + (h2 ? 1 : 0) + (h3 ? 1 : 0);
-		if (__builtin_expect(__ballot(n > nLds) == 0, 1)) { // sp <= nLds: the three rows are inside the area
+		if (__builtin_expect(__ballot(sp > nLds - 3) == 0, 1)) {
 			int *p = lds + sp * 64;
 			p[0]   = e0;
 			p[64]  = e1;

@@ -1205,7 +1205,7 @@ k_megakernel_refill(WfParams P0, DevScene sc, TraceBvh bvh, RayQueueDev q, const
 	const LaneStack stack = laneStack(bvh, ldsStack, ovf);
 	WfParams P			  = P0;
 	// the top P.ldsNodes nodes of the tree, copied into LDS behind the stack
-	float4 *nodeLds = reinterpret_cast<float4 *>(ldsStack + (size_t) (bvh.stackLds + kStackPad) * blockDim.x);
+	float4 *nodeLds = reinterpret_cast<float4 *>(ldsStack + (size_t) stackRows(bvh.stackLds) * blockDim.x);
 	if (P.ldsNodes > 0) {
 		const float4 *src = reinterpret_cast<const float4 *>(bvh.nodes);
 		for (int i = (int) threadIdx.x; i < P.ldsNodes * 8; i += (int) blockDim.x) nodeLds[i] = src[i];
@@ -1470,9 +1470,7 @@ struct AccelData {
 	int maxDepth	= 0;
 	double buildSeconds = 0;
 	bool onDevice		= false; // built by the GPU builder
-	// entries kept in LDS: "stack_lds_entries" less the two rows the pad has
-	// beyond one, so that the LDS a setting takes does not depend on the pad
-	int ldsEntries() const { return std::min(stackSize, std::max(0, stackLds - (kStackPad - 1))); }
+	int ldsEntries() const { return std::min(stackSize, stackLds); }
 	TraceBvh dev() const {
 		return TraceBvh{nodes.as<Bvh4Node>(), tris.as<LeafTri>(), ldsEntries(), (int) std::min<int64_t>(INT32_MAX, nNodes + nLeafTris),
 						alphaTri.as<AlphaTri>(), alphaSrc.as<AlphaSrc>(), quantized ? qnodes.as<Bvh4QNode>() : nullptr};
@@ -1693,7 +1691,7 @@ template <class K> int persistentGrid(K kernel, int block, size_t lds, int maxBl
 
 // LDS bytes per block of the short traversal stack, and ints per grid thread
 // of its global overflow.
-size_t stackLds(const AccelData &a, int block) { return (size_t) (a.ldsEntries() + kStackPad) * block * sizeof(int); }
+size_t stackLds(const AccelData &a, int block) { return (size_t) stackRows(a.ldsEntries()) * block * sizeof(int); }
 size_t stackOverflowInts(const AccelData &a) { return (size_t) (a.stackSize - a.ldsEntries()); }
 
 // Launch of a persistent path kernel over `paths` pixels: the resident blocks,
@@ -1718,9 +1716,10 @@ struct PathGrid {
 };
 
 // A persistent launch as a frame makes it: blocks, lanes of each wave that take
-// up paths, samples of a pixel one after the other.
+// up paths, samples of a pixel one after the other, and the entries of a lane's
+// traversal stack that are in LDS.
 struct LaunchShape {
-	int blocks = 0, lanes = 0, samples = 0;
+	int blocks = 0, lanes = 0, samples = 0, stackLds = 0;
 };
 
 PathGrid pathGrid(int resident, int tb, int64_t paths, bool smallTree) {
@@ -2286,7 +2285,7 @@ constexpr int kLaunchSamples	= 256;
 constexpr int64_t kLaunchPaths = (int64_t) 1 << 28;
 LaunchShape launchShape(const krr_wf *wf, const PathGrid &g, int N, bool camera, bool nrc) {
 	const int64_t most = std::min<int64_t>(kLaunchSamples, std::max<int64_t>(1, kLaunchPaths / N));
-	return LaunchShape{g.blocks, g.lanes, camera && !nrc ? (int) std::min<int64_t>(wf->spp, most) : 1};
+	return LaunchShape{g.blocks, g.lanes, camera && !nrc ? (int) std::min<int64_t>(wf->spp, most) : 1, wf->accel.ldsEntries()};
 }
 
 Json shapeJson(const LaunchShape &s) {
@@ -2294,6 +2293,7 @@ Json shapeJson(const LaunchShape &s) {
 	o.set("blocks", Json((double) s.blocks));
 	o.set("lanes", Json((double) s.lanes));
 	o.set("samples", Json((double) s.samples));
+	o.set("stack_lds_entries", Json((double) s.stackLds));
 	return o;
 }
 
@@ -2705,7 +2705,7 @@ int frameLaunch(krr_wf *wf, int N, FrameLaunch &L) {
 	const int tb	   = wf->traceBlockSize;
 	const int gTmax	   = (N + tb - 1) / tb;
 	L.lds			   = stackLds(wf->accel, tb);
-	if ((size_t) (L.bvh.stackLds + kStackPad) * tb * sizeof(int) != L.lds) return krr::fail(KRR_ERR_INVALID_ARG, "krr_wf_render: stack layout mismatch");
+	if ((size_t) stackRows(L.bvh.stackLds) * tb * sizeof(int) != L.lds) return krr::fail(KRR_ERR_INVALID_ARG, "krr_wf_render: stack layout mismatch");
 	L.count	 = wf->countTraversal;
 	L.media	 = wf->enableMedium && wf->sceneHasMedia;
 	L.plain	 = !wf->sceneTextured;
@@ -3555,7 +3555,7 @@ int krr_mk_render(krr_mk *mk, float *film_dev, void *hip_stream) {
 		if (!mk->rays.p) KRR_HIP(mk->rays.alloc(256)); // the two counts, and the work counter on a line of its own
 		mk->gridKey = key;
 	}
-	if ((size_t) (bvh.stackLds + kStackPad) * tb * sizeof(int) != lds) return krr::fail(KRR_ERR_INVALID_ARG, "krr_mk_render: stack layout mismatch");
+	if ((size_t) stackRows(bvh.stackLds) * tb * sizeof(int) != lds) return krr::fail(KRR_ERR_INVALID_ARG, "krr_mk_render: stack layout mismatch");
 	PtArgs a;
 	a.sc		  = wf->ds;
 	a.bvh		  = bvh;

@@ -1,5 +1,6 @@
 """Shapes of the persistent launch ("launch_in_force"): blocks, lanes of a wave
-that take up paths, samples of a pixel per launch."""
+that take up paths, samples of a pixel per launch, entries of a lane's
+traversal stack in LDS."""
 import numpy as np
 import pytest
 
@@ -33,7 +34,7 @@ def test_queue_launches_are_no_larger_than_the_queue(krr, gpu, w, h):
     a, la, _ = _frame(krr, gpu, s, w, h, dict(params, wavefront_depths=1))
     b, lb, _ = _frame(krr, gpu, s, w, h, params)
     print("queue", la, "camera", lb, flush=True)
-    assert la == {"blocks": (w * h + 127) // 128, "lanes": 64, "samples": 1}
+    assert (la["blocks"], la["lanes"], la["samples"]) == ((w * h + 127) // 128, 64, 1)
     assert lb["blocks"] > la["blocks"] and lb["lanes"] < 64 and lb["samples"] == 2
     assert np.array_equal(a, b)
 
@@ -71,3 +72,17 @@ def test_views_run_a_bounded_number_of_samples(krr, gpu):
         assert st["closest_launches"] == 2 and st["closest_rays"] == sa["closest_rays"]
         assert wf.to_json()["launch_in_force"]["samples"] == 256
         wf.close()
+
+
+@pytest.mark.parametrize("entries", [0, 1, 2, 3, 4, 16, 96])
+def test_stack_entries_in_lds_are_the_setting(krr, gpu, entries):
+    """stack_lds_entries of each lane are kept in LDS, or all that the tree
+    needs (three per level and four)."""
+    print(f"case: stack_lds_entries={entries}", flush=True)
+    s = krr.Scene(icosphere_scene(count=64, level=2, res=(32, 32)))
+    accel = krr.Accel(s.desc)
+    need = 3 * accel.info()["max_depth"] + 4
+    accel.close()
+    _, launch, _ = _frame(krr, gpu, s, 32, 32, {"spp": 1, "max_depth": 3, "stack_lds_entries": entries})
+    print(launch, "needed", need, flush=True)
+    assert launch["stack_lds_entries"] == min(entries, need)
