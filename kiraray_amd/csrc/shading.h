@@ -98,7 +98,7 @@ struct DevScene {
 	const float *uv; // 2 per vertex (may be null)
 	const float *tan; // 3 per vertex (may be null)
 	const DevTexture *textures;
-	const float4 *tri;		// kTriRec per triangle: what a hit needs of it
+	const float4 *tri;		// kTriRec per triangle: what a hit needs of it (null where nothing reads it: uploadScene)
 	const float4 *lightTri; // kLightRec per light (area lights only): what a light sample needs of its triangle
 	float sceneRadius;
 	float bmin[3], binv[3]; // scene box: p -> (p - bmin) * binv maps it to [0,1]^3

@@ -80,7 +80,7 @@ __global__ void k_begin_frame(WfParams P, PixelStateDev px) {
 	px.rng[i]			= s.state;
 }
 
-// The records of every triangle and light (kTriRec, kLightRec).
+// The records of the triangles and lights (kTriRec, kLightRec).
 __global__ void k_tri_records(DevScene sc, int64_t n, float4 *out) {
 	const int64_t i = blockIdx.x * (int64_t) blockDim.x + threadIdx.x;
 	if (i >= n) return;
@@ -2238,20 +2238,24 @@ int uploadScene(krr_wf *wf, const krr_scene_desc *s) {
 		ds.bmin[a] = lo[a];
 		ds.binv[a] = hi[a] > lo[a] ? 1.f / (hi[a] - lo[a]) : 1.f;
 	}
-	KRR_HIP(wf->triRec.alloc((size_t) s->n_triangles * kTriRec * sizeof(float4)));
+	wf->sceneHasMedia = s->n_media > 0;
+	wf->sceneTextured = s->n_textures > 0 || wf->accel.alphaTri.p != nullptr;
+	for (int i = 0; i < s->n_meshes; i++) wf->sceneTextured |= s->meshes[i].has_tangents != 0;
+	for (int i = 0; i < s->n_infinite_lights; i++) wf->sceneTextured |= s->infinite_lights[i].image_rgba != nullptr;
+	// what reads triangle records (prepareSurfaceRecord): every hit of a scene
+	// without texture lookups, and the interfaces a shadow ray meets in media
+	const bool triRecords = !wf->sceneTextured || (wf->enableMedium && wf->sceneHasMedia);
+	if (triRecords) KRR_HIP(wf->triRec.alloc((size_t) s->n_triangles * kTriRec * sizeof(float4)));
+	else wf->triRec.release();
 	KRR_HIP(wf->lightRec.alloc(lights.size() * kLightRec * sizeof(float4)));
-	if (s->n_triangles > 0)
+	if (triRecords && s->n_triangles > 0)
 		hipLaunchKernelGGL(k_tri_records, dim3((unsigned) ((s->n_triangles + 255) / 256)), dim3(256), 0, nullptr, ds, s->n_triangles, wf->triRec.as<float4>());
 	if (!lights.empty()) hipLaunchKernelGGL(k_light_records, dim3((unsigned) ((lights.size() + 63) / 64)), dim3(64), 0, nullptr, ds, wf->lightRec.as<float4>());
 	KRR_HIP(hipGetLastError());
 	KRR_HIP(hipDeviceSynchronize());
 	ds.tri		= wf->triRec.as<float4>();
 	ds.lightTri = wf->lightRec.as<float4>();
-	wf->sceneHasMedia = s->n_media > 0;
-	wf->sceneTextured = s->n_textures > 0 || wf->accel.alphaTri.p != nullptr;
-	for (int i = 0; i < s->n_meshes; i++) wf->sceneTextured |= s->meshes[i].has_tangents != 0;
-	for (int i = 0; i < s->n_infinite_lights; i++) wf->sceneTextured |= s->infinite_lights[i].image_rgba != nullptr;
-	wf->haveScene	  = true;
+	wf->haveScene = true;
 	return KRR_OK;
 }
 

@@ -8,6 +8,7 @@ both integrators against the oracle.
 import numpy as np
 import pytest
 
+from conftest import icosphere_scene
 from test_gpu_megakernel import mk_render
 from test_gpu_render import assert_images_match, gpu_render
 
@@ -53,3 +54,35 @@ def test_records_match_oracle(krr, oracle, gpu, n, lights, flip, sky):
     o, os_ = oracle.render_megakernel(s.desc, s.camera(0), 40, 30, 2, spp=2, max_depth=6)
     assert gs["closest_rays"] == os_["closest_rays"] and gs["shadow_rays"] == os_["shadow_rays"]
     assert_images_match(g, o)
+
+
+def _free_bytes(gpu):
+    import ctypes as C
+    free, total = C.c_size_t(), C.c_size_t()
+    gpu.synchronize()
+    gpu.check(gpu.runtime().hipMemGetInfo(C.byref(free), C.byref(total)))
+    return free.value
+
+
+@pytest.mark.parametrize("media", [False, True])
+def test_triangle_records_only_where_they_are_read(krr, gpu, tmp_path, media):
+    """Scenes with texture lookups build hits from the vertex arrays: without
+    media nothing reads a triangle's record, and none is kept (96 bytes each,
+    of 328 K triangles)."""
+    print(f"case: device memory of a scene under an image environment, media={media}", flush=True)
+    np.save(tmp_path / "sky.npy", np.ones((4, 8, 3), np.float32))
+    cfg = icosphere_scene(count=256, level=3, res=(32, 32), media=media, grid_res=16)
+    used = []
+    for textured in (False, True, False, True):  # the first of a kind may also pay for the runtime's own memory
+        s = krr.Scene(dict(cfg, environment={"image": str(tmp_path / "sky.npy")}) if textured else cfg)
+        wf = krr.WavefrontPathTracer({"spp": 1, "max_depth": 3})
+        before = _free_bytes(gpu)
+        wf.set_scene(s)
+        used.append(before - _free_bytes(gpu))
+        wf.close()
+    records = 96 * s.n_triangles
+    print("bytes without / with textures", used[2:], "records", records, flush=True)
+    if media:
+        assert used[3] >= used[2]
+    else:
+        assert used[3] < used[2] - 0.8 * records
