@@ -243,6 +243,7 @@ struct Level {
 	int *blockCnt;				// the axes' bin counts of each block's references
 	int *childBox;				// per node 24 ints: bounds and centroid bounds of the left child, then the right
 	const int *blockBegin;		// first block of each node (n + 1 entries)
+	int *blockOff;				// left references of the node before each block (nodes of many blocks: k_level_offsets)
 };
 
 // One of the two node lists that the levels alternate between.
@@ -253,6 +254,7 @@ struct LevelList {
 // What the host reads between levels, and the running totals.
 struct LevelCtl {
 	int nodes, blocks;	 // of the next level
+	int most;			 // blocks of its largest node, if more than kThreads
 	int small, nextNode; // subtrees handed to k_small, binary nodes numbered so far
 	int bad;			 // a split left a side empty
 };
@@ -430,6 +432,40 @@ __device__ inline int blockLefts(const Level &L, int t, int e) {
 	return n;
 }
 
+// Nodes of at most kThreads blocks have their earlier blocks' left references
+// counted by each block of the scatter, one row per thread (a launch less).
+// Those of larger nodes are added up once: counted by each block, the work
+// grows with the square of the node.  Root's scatter 4.24 ms for 16.8 M triangles
+// that way, 0.72 ms and 0.10 ms for the sums this way; 4.2 M 0.32 against 0.19 and
+// 0.02 ms; 1.05 M 0.06 ms both.
+__device__ inline bool offsetsListed(const Level &L, int t) { return L.blockBegin[t + 1] - L.blockBegin[t] > kThreads; }
+
+__global__ void __launch_bounds__(1024) k_level_offsets(Level L) {
+	const int t = blockIdx.x;
+	if (!offsetsListed(L, t)) return;
+	__shared__ int part[16];
+	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, end = L.blockBegin[t + 1];
+	int carry = 0; // of the blocks before base
+	for (int base = L.blockBegin[t]; base < end; base += 1024) {
+		const int e	  = base + (int) threadIdx.x;
+		const int own = e < end ? blockLefts(L, t, e) : 0;
+		int incl	  = own;
+		for (int o = 1; o < 64; o <<= 1) {
+			const int u = __shfl_up(incl, o);
+			if (lane >= o) incl += u;
+		}
+		if (lane == 63) part[wave] = incl;
+		__syncthreads();
+		int before = carry;
+		for (int w = 0; w < 16; w++) {
+			if (w < wave) before += part[w];
+			carry += part[w];
+		}
+		if (e < end) L.blockOff[e] = before + incl - own;
+		__syncthreads();
+	}
+}
+
 // Stable partition: thread j of the block owns the references [per j, per j + per)
 // of the block's chunk, in order.  The bounds of a child that is a large node
 // itself are taken on the way.
@@ -471,8 +507,9 @@ __global__ void __launch_bounds__(kThreads) k_level_scatter(Level L, Prims P, co
 	}
 	// left references of the node's earlier blocks, of the block's earlier waves
 	// and of the wave's earlier lanes
-	int before = 0;
-	for (int e = L.blockBegin[t] + (int) threadIdx.x; e < b; e += kThreads) before += blockLefts(L, t, e);
+	int before		  = 0;
+	const bool listed = offsetsListed(L, t);
+	if (!listed && L.blockBegin[t] + (int) threadIdx.x < b) before = blockLefts(L, t, L.blockBegin[t] + (int) threadIdx.x);
 	for (int o = 32; o > 0; o >>= 1) before += __shfl_xor(before, o);
 	int leftBefore = 0, waveLefts = 0;
 #pragma unroll
@@ -486,7 +523,7 @@ __global__ void __launch_bounds__(kThreads) k_level_scatter(Level L, Prims P, co
 		lefts[wave]	  = waveLefts;
 	}
 	__syncthreads();
-	before = 0;
+	before = listed ? L.blockOff[b] : 0;
 	for (int w = 0; w < waves; w++) {
 		before += earlier[w];
 		if (w < wave) leftBefore += lefts[w];
@@ -528,7 +565,8 @@ __global__ void k_level_init(LevelList list, SmallTask *small, LevelCtl *ctl, in
 	for (int e = 0; e < 6; e++) list.box[e] = list.cbox[e] = emptyBound(e); // k_root_bounds fills them
 	list.blockBegin[1] = (n + kChunk - 1) / kChunk;
 	small[0]		 = SmallTask{0, 0, n, 1, 0};
-	*ctl			 = LevelCtl{large ? 1 : 0, (n + kChunk - 1) / kChunk, large ? 0 : 1, large ? 1 : 2 * n - 1, 0};
+	const int blocks = (n + kChunk - 1) / kChunk;
+	*ctl			 = LevelCtl{large ? 1 : 0, blocks, blocks, large ? 0 : 1, large ? 1 : 2 * n - 1, 0};
 }
 
 // Binary nodes of the level, the next level's list and the subtrees that are
@@ -536,8 +574,10 @@ __global__ void k_level_init(LevelList list, SmallTask *small, LevelCtl *ctl, in
 // block, 1024 nodes at a time, places by a scan.
 __global__ void __launch_bounds__(1024) k_level_next(Level L, int nNodes, LevelList next, SmallTask *small, int buf, Nodes2 N, LevelCtl *ctl) {
 	__shared__ int4 part[16];
+	__shared__ int most;
 	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 	const int node0 = ctl->nextNode, small0 = ctl->small;
+	if (threadIdx.x == 0) most = 0; // the loop's first barrier lies before its other uses
 	int4 carry		= make_int4(0, 0, 0, 0); // large children, their blocks, small children, their descendants
 	for (int base = 0; base < nNodes; base += 1024) {
 		const int t	 = base + (int) threadIdx.x;
@@ -583,6 +623,7 @@ __global__ void __launch_bounds__(1024) k_level_next(Level L, int nNodes, LevelL
 				}
 				at.x++;
 				at.y += (c[k] + kChunk - 1) / kChunk;
+				if (c[k] > kThreads * kChunk) atomicMax(&most, (c[k] + kChunk - 1) / kChunk);
 			} else {
 				small[small0 + at.z] = SmallTask{node, f[k], c[k], node0 + 2 * nNodes + at.w, buf};
 				at.z++;
@@ -595,6 +636,7 @@ __global__ void __launch_bounds__(1024) k_level_next(Level L, int nNodes, LevelL
 		next.blockBegin[carry.x] = carry.y;
 		ctl->nodes				 = carry.x;
 		ctl->blocks				 = carry.y;
+		ctl->most				 = most;
 		ctl->small				 = small0 + carry.z;
 		ctl->nextNode			 = node0 + 2 * nNodes + carry.w;
 	}
@@ -830,7 +872,9 @@ __global__ void __launch_bounds__(256) k_collapse_count(Nodes2 N, const int *lev
 }
 
 // The level's 4-wide nodes; the inner children's places in the next level are
-// the sum of the earlier blocks' counts and a scan within the block.
+// the sum of the earlier blocks' counts and a scan within the block.  (The sums
+// are few: 256 nodes a block; with the counts scanned by a launch of its own the
+// emissions of 16.8 M triangles took 1.24 ms as well.)
 __global__ void __launch_bounds__(256) k_collapse_emit(Nodes2 N, const int *level, int n, int levelBase, const int *blockSum, int nextBase,
 													   int *nextLevel, Bvh4Node *out, int *total) {
 	__shared__ int earlier[4], part[4];
@@ -996,6 +1040,7 @@ int buildBvh4Device(const float *pos, int64_t nVerts, const int32_t *idx, int64_
 		L.blockNode	 = m.take<int>(maxB);
 		L.blockStart = m.take<int>(maxB);
 		L.blockCnt	 = m.take<int>(3 * NB * maxB);
+		L.blockOff	 = m.take<int>(maxB);
 		small		 = m.take<SmallTask>((size_t) n);
 		ctl			 = m.take<LevelCtl>(1);
 		total		 = m.take<int>(1);
@@ -1046,6 +1091,7 @@ int buildBvh4Device(const float *pos, int64_t nVerts, const int32_t *idx, int64_
 		hipLaunchKernelGGL(k_level_reset, dim3(T), dim3(256), 0, st, L, T);
 		hipLaunchKernelGGL(k_level_bins, dim3(B), dim3(kThreads), 0, st, L, P, in);
 		hipLaunchKernelGGL(k_level_split, dim3(T), dim3(64), 0, st, L, T, cost, maxLeaf);
+		if (c.most > kThreads) hipLaunchKernelGGL(k_level_offsets, dim3(T), dim3(1024), 0, st, L);
 		hipLaunchKernelGGL(k_level_scatter, dim3(B), dim3(kThreads), 0, st, L, P, in, to);
 		hipLaunchKernelGGL(k_level_next, dim3(1), dim3(1024), 0, st, L, T, list[cur ^ 1], small, (levels & 1) ^ 1, N, ctl);
 		BVHD_HIP(hipGetLastError());

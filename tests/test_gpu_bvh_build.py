@@ -166,3 +166,28 @@ def test_level_sizes(krr, oracle, gpu, n, kind):
     """Nodes of several blocks of 1,024 references, whole and ragged, split by
     bins and in the middle, with large and small children: as above."""
     test_subtree_sizes(krr, oracle, gpu, n, kind)
+
+
+@pytest.mark.parametrize("n,kind", [(512 * 1024, "spread"), (512 * 1024 + 1, "spread"), (513 * 1024 + 1, "one_point"), (1500001, "spread")])
+def test_nodes_of_many_blocks(krr, gpu, n, kind):
+    """Nodes of more than 512 blocks of 1,024 references have the blocks'
+    left counts added up by a launch of its own: the host build's tree and
+    hits."""
+    print(f"case: device BVH of {n} triangles, {kind}", flush=True)
+    rng = np.random.default_rng(n)
+    c = rng.random((n, 1, 3), dtype=np.float32) if kind == "spread" else np.full((n, 1, 3), 0.5, np.float32)
+    edge = np.array([[0.05, 0.0, 0.0], [-0.025, 0.05, 0.0], [-0.025, -0.05, 0.0]], np.float32) * (0.2 if kind == "spread" else 1.0)
+    pos = np.ascontiguousarray((c + edge * (0.5 + rng.random((n, 1, 1), dtype=np.float32))).reshape(-1, 3), np.float32)
+    idx = np.arange(3 * n, dtype=np.int32).reshape(-1, 3)
+    desc, keep = _soup_desc(krr, pos, idx)
+    rays = _rays_towards_triangles(pos, idx, 5000 if kind == "spread" else 100, rng, np.array([-0.2, -0.2, -1.0]), np.array([1.2, 1.2, 2.0]), jitter=0.02)
+    gd, vd, infod = _gpu_closest(krr, gpu, _Desc(desc), rays, {"builder": "device"})
+    gh, vh, infoh = _gpu_closest(krr, gpu, _Desc(desc), rays, {"builder": "host"})
+    print("device", infod, "host", infoh, flush=True)
+    assert infod["leaf_tris"] == infoh["leaf_tris"] == n
+    if kind == "spread":
+        assert infod["nodes"] == infoh["nodes"] and infod["max_depth"] == infoh["max_depth"]
+    _assert_same_hits(gd, gh)
+    assert np.array_equal(vd, vh)
+    assert (gd["prim"] >= 0).mean() > 0.3
+    del keep
