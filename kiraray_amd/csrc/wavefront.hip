@@ -1701,17 +1701,20 @@ size_t stackOverflowInts(const AccelData &a) { return (size_t) (a.stackSize - a.
 // paths fill waves of 64, and each wave runs every stage for as long as its
 // slowest lane.  Spread over more waves, a path waits for fewer others: the
 // fewest lanes per wave, a power of two, that still hold every path at once in
-// the resident waves, or in half of them for small trees whose nodes sit in the
-// L1 (two waves then share a SIMD that four would crowd).  us per frame with 64
-// lanes / all resident waves / half of them: Cornell 64x64 704 / 445 / 420,
-// 256x256 2208 / 2332 / 2055; 1.31 M-triangle field 64x48 1069 / 526 / 559,
-// 160x90 1902 / 1417 / 1613, 320x180 1256 / 1141 / 1261; grid medium 240x135
-// 7119 / 4743 / 5622.
+// the resident waves, or (half) in half of them.  Half is for launches without
+// refill or media on small trees (smallTree), whose nodes sit in the L1: two
+// waves then share a SIMD that four would crowd.  us per frame with 64 lanes /
+// all resident waves / half of them: Cornell 64x64 704 / 445 / 420, 256x256
+// 2208 / 2332 / 2055, with refill_lanes 8 (three waves per SIMD) 64x64 - / 472 /
+// 514, 256x256 - / 769 / 793; 1.31 M-triangle field 64x48 1069 / 526 / 559,
+// 160x90 1902 / 1417 / 1613, 320x180 1256 / 1141 / 1261, with refill_lanes 0
+// 160x90 - / 939 / 1112, 320x180 - / 1442 / 1610; grid medium 240x135 7119 /
+// 4743 / 5622.
 struct PathGrid {
 	int blocks = 1, lanes = 64;
 	// The order the paths are taken up in (k_tile_keys) counts only when some
-	// wait for a lane; when every path starts at once, its six launches (25 us)
-	// are left out: 742 against 753 us for a 64x64 frame of 4 samples.
+	// wait for a lane; when every path starts at once, its six launches are left
+	// out: 742 against 753 us for a 64x64 frame of 4 samples.
 	bool ordered = true;
 };
 
@@ -1722,9 +1725,11 @@ struct LaunchShape {
 	int blocks = 0, lanes = 0, samples = 0, stackLds = 0;
 };
 
-PathGrid pathGrid(int resident, int tb, int64_t paths, bool smallTree) {
+bool smallTree(const AccelData &a) { return a.nNodes < kRefillMinNodes; }
+
+PathGrid pathGrid(int resident, int tb, int64_t paths, bool half) {
 	PathGrid g;
-	const int64_t waves = (int64_t) resident * (tb / 64) / (smallTree ? 2 : 1);
+	const int64_t waves = (int64_t) resident * (tb / 64) / (half ? 2 : 1);
 	while (g.lanes > 1 && waves * (g.lanes / 2) >= paths) g.lanes /= 2;
 	const int64_t perBlock = (int64_t) g.lanes * (tb / 64);
 	g.blocks  = (int) std::max<int64_t>(1, std::min<int64_t>(resident, (paths + perBlock - 1) / perBlock));
@@ -2450,8 +2455,6 @@ int krr_accel_build(const krr_scene_desc *scene, const char *json_opts, krr_acce
 // counter and stack overflow area: calls on one accel must not overlap.
 static constexpr int kAccelBlock = 128;
 
-static bool smallTree(const AccelData &a) { return a.nNodes < kRefillMinNodes; }
-
 int krr_accel_trace_closest(krr_accel *accel, const float *rays_dev, int64_t n, krr_hit *hits_dev, void *hip_stream) {
 	krr::clearError();
 	if (!accel || n < 0 || (n > 0 && (!rays_dev || !hits_dev))) return krr::fail(KRR_ERR_INVALID_ARG, "krr_accel_trace_closest: bad argument");
@@ -2652,6 +2655,7 @@ int krr_wf_set_scene(krr_wf *wf, const krr_scene_desc *scene) {
 	KRR_HIP(hipDeviceSynchronize());
 	wf->haveScene = false;
 	wf->sceneVersion++;
+	wf->gridKey = wf->viewsGridKey = ~0ull; // the grids depend on the tree
 	wf->dropGraph();
 	int rc		  = uploadScene(wf, scene);
 	if (rc) return rc;
@@ -2731,7 +2735,7 @@ int frameLaunch(krr_wf *wf, int N, FrameLaunch &L) {
 		auto mega = [&](bool nrc) {
 			const int resident = withMega<false>(media, count, nrc, L.plain, L.refill, L.dense, [&](auto k) { return decltype(k)::grid(tb, lds, 1 << 20, nodeBytes); });
 			if (wf->wavefrontDepths > 0) return queueGrid(scaledGrid(resident, wf->occupancy), tb, N);
-			return pathGrid(scaledGrid(resident, wf->occupancy), tb, N, !media && !L.refill);
+			return pathGrid(scaledGrid(resident, wf->occupancy), tb, N, !media && !L.refill && smallTree(wf->accel));
 		};
 		wf->gMega = mega(false);
 		if (wf->nrcOn) wf->gMegaNrc = mega(true);
@@ -2942,7 +2946,7 @@ int viewsLaunch(krr_wf *wf, int N, bool nrc, ViewsLaunch &L) {
 		const size_t nodeBytes = (size_t) ldsNodeCount(wf) * sizeof(Bvh4Node);
 		const int resident = withMega<true>(L.media, L.count, nrc, !wf->sceneTextured, refillLanesOf(wf) > 0, false,
 											[&](auto k) { return decltype(k)::grid(tb, L.lds, 1 << 20, nodeBytes); });
-		wf->gMegaViews = pathGrid(scaledGrid(resident, wf->occupancy), tb, N, !L.media && refillLanesOf(wf) == 0);
+		wf->gMegaViews = pathGrid(scaledGrid(resident, wf->occupancy), tb, N, !L.media && refillLanesOf(wf) == 0 && smallTree(wf->accel));
 		if (int rc = reserveOverflow(wf->ovf, wf->accel, (size_t) wf->gMegaViews.blocks * tb)) return rc;
 		wf->viewsGridKey = key;
 	}

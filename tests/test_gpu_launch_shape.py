@@ -86,3 +86,23 @@ def test_stack_entries_in_lds_are_the_setting(krr, gpu, entries):
     _, launch, _ = _frame(krr, gpu, s, 32, 32, {"spp": 1, "max_depth": 3, "stack_lds_entries": entries})
     print(launch, "needed", need, flush=True)
     assert launch["stack_lds_entries"] == min(entries, need)
+
+
+@pytest.mark.parametrize("scene,refill,media,half", [("cornell", 0, False, True), ("cornell", 8, False, False), ("field", 0, False, False),
+                                                     ("field", 8, False, False), ("field", 0, True, False)])
+@pytest.mark.parametrize("w,h", [(64, 48), (131, 77)])
+def test_lanes_that_take_up_paths(krr, gpu, scene, refill, media, half, w, h):
+    """Small frames take the fewest lanes per wave that hold their paths in the
+    resident waves, or in half of them for small trees without refill or media."""
+    print(f"case: {scene} refill={refill} media={media} {w}x{h}", flush=True)
+    s = krr.Scene(CORNELL if scene == "cornell" else icosphere_scene(count=64, level=2, res=(w, h), media=media, grid_res=16))
+    params = {"spp": 1, "max_depth": 2, "refill_lanes": refill, "trace_block_size": 128}
+    _, full, _ = _frame(krr, gpu, s, 1024, 768, params)
+    _, small, _ = _frame(krr, gpu, s, w, h, params)
+    assert full["lanes"] == 64  # more paths than lanes: every resident block
+    waves = full["blocks"] * 2 // (2 if half else 1)
+    lanes = 64
+    while lanes > 1 and waves * (lanes // 2) >= w * h:
+        lanes //= 2
+    print("full", full, "small", small, flush=True)
+    assert small["lanes"] == lanes and small["blocks"] == -(-w * h // (2 * lanes))
