@@ -262,16 +262,18 @@ __global__ void k_trace_closest_queue(TraceBvh bvh, const float4 *__restrict__ r
 	}
 }
 
-__global__ void k_accel_begin(Counters *cnt) { cnt->work[0] = 0; }
+// taken: places of the trace that its waves start with (firstShare).
+__global__ void k_accel_begin(Counters *cnt, int taken) { cnt->work[0] = taken; }
 
 // Trace of a caller's ray array (krr_accel_trace_closest / _any): closest hit
 // records, or a visibility flag per ray.  A persistent grid with ray refill, as
 // in the persistent path launch: the rays of a wave advance together until
 // fewer than kTraceLanes of 64 are still traversing, then the others write
-// their result and take the next rays (one atomic per wave).  Waves of 64 rays
+// their result and take the next rays of the wave's share.  Waves of 64 rays
 // run to their end, each as long as its longest, took 1369 us for 2^20
 // incoherent closest and 2^20 shadow rays in the 1.31 M-triangle field; this
-// takes 1231 us (16 lanes: 1239, 32: 1278, 48: 1621, each ray to its end: 1267).
+// took 1231 us with an atomic per refill (16 lanes: 1239, 32: 1278, 48: 1621,
+// each ray to its end: 1267) and takes 1186 us with shares.
 // What bounds it is the L1: a node visit reads seven 16-byte pieces per lane,
 // each lane from a line of its own.
 // With fewer rays than resident lanes, fewer lanes of each wave take rays
@@ -283,16 +285,15 @@ __global__ void __launch_bounds__(128) k_trace_rays(TraceBvh bvh, const float4 *
 	extern __shared__ int ldsStack[];
 	const LaneStack stack = laneStack(bvh, ldsStack, ovf);
 	uint32_t nv = 0, nt = 0;
-	bool going = false, exhausted = false;
+	bool going = false;
 	int ray = -1;
 	f3 o, d;
 	TravState ts;
+	WorkShare share = firstShare(fetchLanes, count);
 	while (true) {
-		if (!exhausted) {
-			const bool need = ray < 0 && laneId() < fetchLanes;
-			const int i		= wavePush(&cnt->work[0], need);
-			if (__ballot(need && i >= count)) exhausted = true;
-			if (need && i < count) {
+		if (!share.empty()) {
+			const int i = takePlace(share, ray < 0 && laneId() < fetchLanes, &cnt->work[0], fetchLanes, count);
+			if (i >= 0) {
 				const float4 a = rays[2 * i], b = rays[2 * i + 1];
 				o	  = f3(a.x, a.y, a.z);
 				d	  = f3(b.x, b.y, b.z);
@@ -304,7 +305,7 @@ __global__ void __launch_bounds__(128) k_trace_rays(TraceBvh bvh, const float4 *
 		const int nActive = __popcll(__ballot(ray >= 0));
 		if (nActive == 0) break;
 		// at most the number of rays in flight: each round finishes at least one
-		const int minLanes = exhausted ? 1 : max(1, (nActive * kTraceLanes) >> 6);
+		const int minLanes = share.empty() ? 1 : max(1, (nActive * kTraceLanes) >> 6);
 		traverseSteps<false, true>(bvh, o, d, ANY, going, ts, stack, minLanes, nv, nt, nullptr, 0, kDefaultLeafShare);
 		if (ray >= 0 && !going) {
 			if (ANY) reinterpret_cast<int *>(out)[ray] = ts.prim < 0 ? 1 : 0;
@@ -2467,7 +2468,7 @@ int krr_accel_trace_closest(krr_accel *accel, const float *rays_dev, int64_t n, 
 	if (int rc = reserveOverflow(accel->ovf, accel->a, (size_t) g.blocks * tb)) return rc;
 	hipStream_t st = (hipStream_t) hip_stream;
 	Counters *cnt  = accel->counters.as<Counters>();
-	hipLaunchKernelGGL(k_accel_begin, dim3(1), dim3(1), 0, st, cnt);
+	hipLaunchKernelGGL(k_accel_begin, dim3(1), dim3(1), 0, st, cnt, g.blocks * (tb / 64) * g.lanes);
 	hipLaunchKernelGGL(k_trace_rays<false>, dim3(g.blocks), dim3(tb), lds, st, accel->a.dev(), (const float4 *) rays_dev, (void *) hits_dev, (int) n, g.lanes,
 					   accel->ovf.as<int>(), cnt);
 	KRR_HIP(hipGetLastError());
@@ -2542,7 +2543,7 @@ int krr_accel_trace_closest_noalloc(krr_accel *accel, const float *rays_dev, int
 	int *ovf	   = reinterpret_cast<int *>(reinterpret_cast<unsigned char *>(base) + kScratchCounterBytes);
 	hipStream_t st = (hipStream_t) hip_stream;
 	// the ray counter starts at zero on every call (a kernel, not a memset)
-	hipLaunchKernelGGL(k_accel_begin, dim3(1), dim3(1), 0, st, cnt);
+	hipLaunchKernelGGL(k_accel_begin, dim3(1), dim3(1), 0, st, cnt, g.blocks * (tb / 64) * g.lanes);
 	hipLaunchKernelGGL(k_trace_rays<false>, dim3(g.blocks), dim3(tb), lds, st, accel->a.dev(), (const float4 *) rays_dev, (void *) hits_dev, (int) n, g.lanes, ovf,
 					   cnt);
 	KRR_HIP(hipGetLastError());
@@ -2561,7 +2562,7 @@ int krr_accel_trace_any(krr_accel *accel, const float *rays_dev, int64_t n, int3
 	if (int rc = reserveOverflow(accel->ovf, accel->a, (size_t) g.blocks * tb)) return rc;
 	hipStream_t st = (hipStream_t) hip_stream;
 	Counters *cnt  = accel->counters.as<Counters>();
-	hipLaunchKernelGGL(k_accel_begin, dim3(1), dim3(1), 0, st, cnt);
+	hipLaunchKernelGGL(k_accel_begin, dim3(1), dim3(1), 0, st, cnt, g.blocks * (tb / 64) * g.lanes);
 	hipLaunchKernelGGL(k_trace_rays<true>, dim3(g.blocks), dim3(tb), lds, st, accel->a.dev(), (const float4 *) rays_dev, (void *) visible_dev, (int) n, g.lanes,
 					   accel->ovf.as<int>(), cnt);
 	KRR_HIP(hipGetLastError());

@@ -1,0 +1,46 @@
+"""Places of a persistent launch handed out to waves and lanes: no ray is left
+out or taken twice, for counts below, at and beyond what the launch's waves
+start with, and for the grid that the fixed scratch holds."""
+import numpy as np
+import pytest
+
+from conftest import CORNELL
+from test_gpu_trace import _assert_same_hits
+
+pytestmark = pytest.mark.gpu
+
+HIT = np.dtype([("t", "<f4"), ("prim", "<i4"), ("b1", "<f4"), ("b2", "<f4")])
+
+
+@pytest.fixture(scope="module")
+def rays(krr, oracle):
+    s = krr.Scene(CORNELL)
+    rng = np.random.default_rng(3)
+    n = 600001
+    r = np.zeros((n, 8), np.float32)
+    r[:, 0:3] = rng.random((n, 3), dtype=np.float32) * [0.8, 1.6, 0.8] + [-0.4, 0.2, -0.4]
+    r[:, 3] = np.where(rng.random(n) < 0.3, 0.5, np.inf)
+    r[:, 4:7] = rng.standard_normal((n, 3), dtype=np.float32)
+    return s, r, oracle.trace_closest(s.desc, r), oracle.trace_any(s.desc, r)
+
+
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 127, 128, 129, 4095, 4097, 131071, 131073, 262143, 262144, 262145, 524287, 524289, 600001])
+def test_every_ray_is_traced_once(krr, gpu, rays, n):
+    print(f"case: {n} rays", flush=True)
+    s, r, closest, visible = rays
+    accel = krr.Accel(s.desc)
+    d = gpu.DeviceBuffer.from_numpy(r[:n])
+    hits, vis = gpu.DeviceBuffer(16 * n), gpu.DeviceBuffer(4 * n)
+    for k in range(2):  # a second pass finds the counter set anew
+        for buf, size in ((hits, 16 * n), (vis, 4 * n)):
+            buf.copy_from_numpy(np.full(size, 0xA5, np.uint8))
+        accel.trace_closest(d.ptr, n, hits.ptr, 0)
+        accel.trace_any(d.ptr, n, vis.ptr, 0)
+        gpu.synchronize()
+        _assert_same_hits(hits.to_numpy(HIT, (n,)), closest[:n])
+        assert np.array_equal(vis.to_numpy(np.int32, (n,)), visible[:n])
+    hits.copy_from_numpy(np.full(16 * n, 0xA5, np.uint8))
+    accel.trace_closest_noalloc(d.ptr, n, hits.ptr, 0)
+    gpu.synchronize()
+    _assert_same_hits(hits.to_numpy(HIT, (n,)), closest[:n])
+    accel.close()
