@@ -176,16 +176,18 @@ KRR_DEV int wavePush(int *counter, bool want) {
 // 1.31 M-triangle field 251 against 375 us.
 struct WorkShare {
 	int next, end; // places the wave holds
+	int first;	   // of its last share
 	bool more;	   // places are left beyond every share taken so far
 	KRR_DEV bool empty() const { return next >= end && !more; }
 };
 KRR_DEV WorkShare firstShare(int size, int count) {
 	const int waves = (int) (blockDim.x >> 6), wave = (int) (blockIdx.x * waves + (threadIdx.x >> 6));
 	const int first = __builtin_amdgcn_readfirstlane(min(wave * size, count));
-	return WorkShare{first, min(first + size, count), (int) gridDim.x * waves * size < count};
+	return WorkShare{first, min(first + size, count), first, (int) gridDim.x * waves * size < count};
 }
 // The next place for each lane with need (at most `size` of them), -1 when there
-// is none left.  Called by every lane of the wave.
+// is none left.  Called by every lane of the wave.  Without a counter a wave's
+// shares are waves * size places apart.
 KRR_DEV int takePlace(WorkShare &s, bool need, int *counter, int size, int count) {
 	const uint64_t mask	 = __ballot(need);
 	const uint64_t below = laneId() == 0 ? 0ull : (mask & (~0ull >> (64 - laneId())));
@@ -193,8 +195,10 @@ KRR_DEV int takePlace(WorkShare &s, bool need, int *counter, int size, int count
 	int place = rank < have ? s.next + rank : -1;
 	if (n > have && s.more) {
 		int base = 0;
-		if (laneId() == 0) base = atomicAdd(counter, size);
-		base = __builtin_amdgcn_readfirstlane(base);
+		if (!counter) base = min(s.first + (int) (gridDim.x * (blockDim.x >> 6)) * size, count);
+		else if (laneId() == 0) base = atomicAdd(counter, size);
+		base	= __builtin_amdgcn_readfirstlane(base);
+		s.first = base;
 		if (rank >= have && base + rank - have < count) place = base + rank - have;
 		s.end  = min(base + size, count);
 		s.next = min(base + n - have, s.end);

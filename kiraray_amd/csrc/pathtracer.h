@@ -20,6 +20,7 @@ struct PtArgs {
 	int *ovf;			  // traversal stack overflow: (stack size - LDS entries) * grid * tb ints
 	unsigned long long *rays; // [0] closest rays, [1] shadow rays (added to)
 	int *work;				  // next place to take up: pixel i % 64 of tile i / 64
+	bool fixedShares;		  // each wave's places are given: the kernel without the counter
 	int fetchLanes;			  // lanes of a wave that take up pixels
 	int refillLanes;		  // a traversal round ends below this many traversing lanes of 64 (0: rays run to their end)
 	int tilesX, nTiles;		  // 8 x 8-pixel tiles
@@ -31,6 +32,6 @@ struct PtArgs {
 hipError_t launchPathTracer(const PtArgs &a, int grid, int tb, size_t lds, hipStream_t st);
 
 // Resident blocks per CU of the kernel for this block size and LDS (>= 1).
-int pathTracerBlocksPerCU(int tb, size_t lds, bool textured);
+int pathTracerBlocksPerCU(int tb, size_t lds, bool textured, bool fixedShares);
 
 } // namespace krr

@@ -115,7 +115,9 @@ KRR_DEV void pathVertex(const PtArgs &A, const TravState &h, const f3 &d, Pcg &r
 	next = p.thp.any();
 }
 
-template <bool TEX> __global__ void __launch_bounds__(256) k_path_tracer(PtArgs A) {
+// FIXED: each wave's places are given shares (WorkShare without a counter),
+// taken up half a wave at a time; else a counter's, as lanes end.
+template <bool TEX, bool FIXED> __global__ void __launch_bounds__(256) k_path_tracer(PtArgs A) {
 	extern __shared__ int ldsStack[];
 	const LaneStack stack = laneStack(A.bvh, ldsStack, A.ovf);
 	uint32_t nClosest = 0, nShadow = 0, nv = 0, nt = 0;
@@ -125,12 +127,23 @@ template <bool TEX> __global__ void __launch_bounds__(256) k_path_tracer(PtArgs 
 	PtPath p;
 	f3 color, o, d, no, nd, contrib; // the ray in flight, and while it is a shadow ray the path's next one
 	TravState ts;
+	const int places = A.nTiles * 64;
+	WorkShare share	 = FIXED ? firstShare(A.fetchLanes, places) : WorkShare{};
 	while (true) {
 		if (!exhausted) {
 			const bool need = !active && left == 0 && laneId() < A.fetchLanes;
-			const int i		= wavePush(A.work, need);
-			if (__ballot(need && i >= A.nTiles * 64)) exhausted = true;
-			if (need && i < A.nTiles * 64) {
+			int i;
+			if constexpr (!FIXED) {
+				i = wavePush(A.work, need);
+				if (__ballot(need && i >= places)) exhausted = true;
+			} else {
+				i = -1;
+				if (2 * __popcll(__ballot(need)) >= A.fetchLanes) {
+					i		  = takePlace(share, need, nullptr, A.fetchLanes, places);
+					exhausted = share.empty();
+				}
+			}
+			if (need && (!FIXED || i >= 0) && i < places) {
 				const int tile = i >> 6;
 				x = (tile % A.tilesX) * 8 + (i & 7);
 				y = (tile / A.tilesX) * 8 + ((i >> 3) & 7);
@@ -206,17 +219,21 @@ __global__ void k_path_tracer_clear(unsigned long long *rays, int *work) {
 	if (threadIdx.x == 2) *work = 0;
 }
 
+template <class F> static void withPathTracer(bool textured, bool fixed, F &&f) {
+	if (textured) fixed ? f(k_path_tracer<true, true>) : f(k_path_tracer<true, false>);
+	else fixed ? f(k_path_tracer<false, true>) : f(k_path_tracer<false, false>);
+}
+
 hipError_t launchPathTracer(const PtArgs &a, int grid, int tb, size_t lds, hipStream_t st) {
 	hipLaunchKernelGGL(k_path_tracer_clear, dim3(1), dim3(64), 0, st, a.rays, a.work);
-	if (a.textured) hipLaunchKernelGGL(k_path_tracer<true>, dim3(grid), dim3(tb), lds, st, a);
-	else hipLaunchKernelGGL(k_path_tracer<false>, dim3(grid), dim3(tb), lds, st, a);
+	withPathTracer(a.textured, a.fixedShares, [&](auto k) { hipLaunchKernelGGL(k, dim3(grid), dim3(tb), lds, st, a); });
 	return hipGetLastError();
 }
 
-int pathTracerBlocksPerCU(int tb, size_t lds, bool textured) {
-	int nb = 0;
-	const hipError_t e = textured ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_path_tracer<true>, tb, lds)
-								  : hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_path_tracer<false>, tb, lds);
+int pathTracerBlocksPerCU(int tb, size_t lds, bool textured, bool fixedShares) {
+	int nb		 = 0;
+	hipError_t e = hipSuccess;
+	withPathTracer(textured, fixedShares, [&](auto k) { e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k, tb, lds); });
 	if (e != hipSuccess || nb < 1) nb = 1;
 	return nb;
 }

@@ -3536,6 +3536,26 @@ int krr_mk_begin_frame(krr_mk *mk, const krr_camera *camera, uint64_t frame_inde
 	return KRR_OK;
 }
 
+} // extern "C"
+
+namespace {
+
+// Megakernel frames whose waves take given shares of the pixels, half a wave at
+// a time, instead of refilling lanes one by one from a counter: short paths (one
+// sample, trees below 2 MB of nodes) ended too many lanes too often for the
+// counter's 4 ns per refill, and mixed camera rays into other rays' rounds.
+// us per frame of pixels in whole tiles a wave without any refill / from the
+// counter / given: 5 K triangles 640x360 273 / 326 / 268, 1920x1080 580 / 1046 /
+// 548; 20 K 1920x1080 1007 / 1178 / 844; 30 K 1255 / 1205 / 1020; 40 K (25 K nodes)
+// 1474 / 1244 / -; Cornell 640x360 375 / 335 / 323, 1920x1080 1279 / 1324 / 1061,
+// but 300x300 207 / 261 / 246.  Four samples of a pixel make few refills: 853x479
+// of 5 K 890 / 900 / 1039, Cornell 1490 / 995 / 1376.
+bool fixedShares(const AccelData &a, int spp) { return spp == 1 && a.nNodes < 1 << 14; }
+
+} // namespace
+
+extern "C" {
+
 int krr_mk_render(krr_mk *mk, float *film_dev, void *hip_stream) {
 	krr::clearError();
 	if (!mk) return krr::fail(KRR_ERR_INVALID_ARG, "krr_mk_render: null handle");
@@ -3558,7 +3578,7 @@ int krr_mk_render(krr_mk *mk, float *film_dev, void *hip_stream) {
 		int dev = 0, cus = 0;
 		KRR_HIP(hipGetDevice(&dev));
 		KRR_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-		const int resident = scaledGrid(pathTracerBlocksPerCU(tb, lds, wf->sceneTextured) * std::max(cus, 1), mk->occupancy);
+		const int resident = scaledGrid(pathTracerBlocksPerCU(tb, lds, wf->sceneTextured, fixedShares(wf->accel, mk->spp)) * std::max(cus, 1), mk->occupancy);
 		mk->grid		   = pathGrid(resident, tb, (int64_t) nTiles * 64, smallTree(wf->accel));
 		if (int rc = reserveOverflow(mk->ovf, wf->accel, (size_t) mk->grid.blocks * tb)) return rc;
 		if (!mk->rays.p) KRR_HIP(mk->rays.alloc(256)); // the two counts, and the work counter on a line of its own
@@ -3581,6 +3601,7 @@ int krr_mk_render(krr_mk *mk, float *film_dev, void *hip_stream) {
 	a.rays		  = mk->rays.as<unsigned long long>();
 	a.work		  = mk->rays.as<int>() + 32;
 	a.fetchLanes  = mk->grid.lanes;
+	a.fixedShares = fixedShares(wf->accel, mk->spp);
 	a.refillLanes = refillLanesOf(wf);
 	a.tilesX	  = tilesX;
 	a.nTiles	  = nTiles;

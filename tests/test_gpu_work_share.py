@@ -4,7 +4,7 @@ start with, and for the grid that the fixed scratch holds."""
 import numpy as np
 import pytest
 
-from conftest import CORNELL
+from conftest import CORNELL, icosphere_scene
 from test_gpu_trace import _assert_same_hits
 
 pytestmark = pytest.mark.gpu
@@ -44,3 +44,28 @@ def test_every_ray_is_traced_once(krr, gpu, rays, n):
     gpu.synchronize()
     _assert_same_hits(hits.to_numpy(HIT, (n,)), closest[:n])
     accel.close()
+
+
+@pytest.mark.parametrize("w,h,spp", [(1, 1, 1), (8, 8, 1), (9, 7, 1), (65, 33, 2), (500, 301, 1), (1031, 517, 1), (1031, 517, 2)])
+@pytest.mark.parametrize("spheres", [0, 16, 160])
+def test_every_pixel_is_rendered_once(krr, gpu, w, h, spp, spheres):
+    """The megakernel pass hands out pixels as given shares (one sample, small
+    trees) or from a counter; a launch held to few blocks makes many shares
+    of each wave's.  The same film and rays, and no pixel left out."""
+    print(f"case: {spheres} spheres {w}x{h} {spp} spp", flush=True)
+    s = krr.Scene(icosphere_scene(count=spheres, level=2, res=(w, h)) if spheres else CORNELL)
+    out = []
+    for occupancy in (1.0, 0.05, 0.002):
+        mk = krr.MegakernelPathTracer({"spp": spp, "max_depth": 5, "occupancy": occupancy})
+        mk.set_scene(s.desc)
+        mk.resize(w, h)
+        film = gpu.DeviceBuffer.from_numpy(np.full((h, w, 4), np.nan, np.float32))
+        for frame in (3, 4):
+            mk.begin_frame(s.camera(0), frame)
+            mk.render(film.ptr, 0)
+        st = mk.stats()
+        out.append((film.to_numpy(np.float32, (h, w, 4)), st["closest_rays"], st["shadow_rays"]))
+        mk.close()
+    assert np.isfinite(out[0][0]).all() and out[0][1] >= w * h * spp
+    for o in out[1:]:
+        assert np.array_equal(o[0], out[0][0]) and o[1:] == out[0][1:]
