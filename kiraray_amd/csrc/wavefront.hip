@@ -1472,6 +1472,8 @@ struct AccelData {
 	double buildSeconds = 0;
 	bool onDevice		= false; // built by the GPU builder
 	int ldsEntries() const { return std::min(stackSize, stackLds); }
+	// bytes of the nodes that the traversal reads
+	int64_t nodeBytes() const { return nNodes * (int64_t) (quantized ? sizeof(Bvh4QNode) : sizeof(Bvh4Node)); }
 	TraceBvh dev() const {
 		return TraceBvh{nodes.as<Bvh4Node>(), tris.as<LeafTri>(), ldsEntries(), (int) std::min<int64_t>(INT32_MAX, nNodes + nLeafTris),
 						alphaTri.as<AlphaTri>(), alphaSrc.as<AlphaSrc>(), quantized ? qnodes.as<Bvh4QNode>() : nullptr};
@@ -1785,13 +1787,16 @@ template <bool VIEWS, bool REFILL, class F> auto withMegaR(bool media, bool coun
 }
 
 // Single-view frames that take the refill launch's 4-wave form: at least three
-// times the paths it has lanes, so that lanes are refilled for most of the
-// launch, and nodes of 2 MB, half an L2.  ms with 3 / 4 waves: 1.31 M triangles
+// times the paths it has lanes (of 16 waves per CU, and of the share of them
+// that `occupancy` launches), so that lanes are refilled for most of the launch,
+// and 2 MB of the nodes it reads, half an L2.  ms with 3 / 4 waves: 1.31 M triangles
 // 640x360 1.40 / 1.48, 960x540 1.64 / 1.79, 1100x700 1.87 / 1.87, 1280x720
 // 1.99 / 1.94, 1920x1080 3.58 / 3.39 and with two samples 6.22 / 5.69; 82 K
 // triangles 1280x720 1.10 / 1.10, 1920x1080 1.88 / 1.84; 20 K triangles 1920x1080
 // 1.44 / 1.47.
-bool denseRefill(const AccelData &a, int64_t paths) { return paths >= 3 << 18 && a.nNodes >= 1 << 14; }
+bool denseRefill(const AccelData &a, int64_t paths, int cus, float occupancy) {
+	return (double) paths >= 3.0 * 1024 * cus * (double) occupancy && a.nodeBytes() >= (int64_t) 2 << 20;
+}
 
 // The persistent kernel for these flags; the refill launch for scenes
 // without media when refill_lanes > 0.
@@ -1862,6 +1867,7 @@ struct krr_wf {
 	}
 	// scene
 	bool haveScene = false;
+	int cus		   = 256; // of the scene's device
 	AccelData accel;
 	DevBuf pos, nrm, idx, triMesh, meshes, materials, lights, media;
 	std::vector<std::unique_ptr<DevBuf>> mediumBufs, imageBufs, textureBufs;
@@ -2657,6 +2663,9 @@ int krr_wf_set_scene(krr_wf *wf, const krr_scene_desc *scene) {
 	wf->haveScene = false;
 	wf->sceneVersion++;
 	wf->gridKey = wf->viewsGridKey = ~0ull; // the grids depend on the tree
+	int dev						   = 0;
+	KRR_HIP(hipGetDevice(&dev));
+	KRR_HIP(hipDeviceGetAttribute(&wf->cus, hipDeviceAttributeMultiprocessorCount, dev));
 	wf->dropGraph();
 	int rc		  = uploadScene(wf, scene);
 	if (rc) return rc;
@@ -2719,7 +2728,7 @@ int frameLaunch(krr_wf *wf, int N, FrameLaunch &L) {
 	L.media	 = wf->enableMedium && wf->sceneHasMedia;
 	L.plain	 = !wf->sceneTextured;
 	L.refill = refillLanesOf(wf) > 0;
-	L.dense	 = denseRefill(wf->accel, N);
+	L.dense	 = denseRefill(wf->accel, N, wf->cus, wf->occupancy);
 	const bool count = L.count, media = L.media;
 	const size_t lds = L.lds;
 	// persistent grid sizes (resident blocks), computed once per shape
@@ -3550,7 +3559,7 @@ namespace {
 // 1474 / 1244 / -; Cornell 640x360 375 / 335 / 323, 1920x1080 1279 / 1324 / 1061,
 // but 300x300 207 / 261 / 246.  Four samples of a pixel make few refills: 853x479
 // of 5 K 890 / 900 / 1039, Cornell 1490 / 995 / 1376.
-bool fixedShares(const AccelData &a, int spp) { return spp == 1 && a.nNodes < 1 << 14; }
+bool fixedShares(const AccelData &a, int spp) { return spp == 1 && a.nodeBytes() < (int64_t) 2 << 20; }
 
 } // namespace
 

@@ -106,3 +106,27 @@ def test_lanes_that_take_up_paths(krr, gpu, scene, refill, media, half, w, h):
         lanes //= 2
     print("full", full, "small", small, flush=True)
     assert small["lanes"] == lanes and small["blocks"] == -(-w * h // (2 * lanes))
+
+
+@pytest.mark.parametrize("more,dense_from", [({}, 3.0), ({"occupancy": 0.5}, 1.5), ({"node_format": "quantized"}, None)])
+def test_four_waves_per_simd_for_many_paths(krr, gpu, more, dense_from):
+    """The refill launch's 4-wave form takes frames of three times the paths it
+    has lanes, on as many lanes as the device and "occupancy" give it, over 2 MB
+    of nodes as they are read (18,000 nodes: not when quantised)."""
+    import ctypes as C
+    print(f"case: waves per SIMD {more}", flush=True)
+    cus = C.c_int()
+    f = gpu.runtime().hipDeviceGetAttribute
+    gpu.check(f(C.byref(cus), 63, 0))  # hipDeviceAttributeMultiprocessorCount
+    lanes, share = cus.value * 1024, more.get("occupancy", 1.0)
+    s = krr.Scene(icosphere_scene(count=110, level=2, res=(64, 64)))
+    accel = krr.Accel(s.desc)
+    nodes = accel.info()["nodes"]
+    accel.close()
+    assert 1 << 14 <= nodes < 1 << 15
+    params = dict({"spp": 1, "max_depth": 1, "trace_block_size": 64, "refill_lanes": 8}, **more)
+    for paths, dense in ((3 * lanes, True), (3 * lanes - 64, dense_from != 3.0), (3 * lanes // 2, dense_from == 1.5), (3 * lanes // 2 - 64, False)):
+        _, launch, _ = _frame(krr, gpu, s, 64, paths // 64, params)
+        waves = launch["blocks"] / (cus.value * 4 * share)  # per SIMD
+        print(paths, launch, waves, flush=True)
+        assert waves == (4 if dense and dense_from else 3)
