@@ -680,9 +680,7 @@ struct SurfaceInteraction {
 // tangent is the mesh's interpolated tangent made orthogonal to n when the
 // mesh has tangents (shading.h:140-145), else getPerpendicular(n); a normal
 // map (shading.h:187-203) then tilts the frame on meshes with texture
-// coordinates.  TEX = false: no mesh has tangents and no material a normal
-// map (the lookups are compiled out).
-template <bool TEX = true>
+// coordinates.
 KRR_DEV void prepareSurfaceInteraction(const DevScene &sc, int prim, float b1, float b2, const f3 &rayDir, int rayMedium,
 									   SurfaceInteraction &it) {
 	const DevMesh m = sc.meshes[sc.triMesh[prim]];
@@ -694,7 +692,7 @@ KRR_DEV void prepareSurfaceInteraction(const DevScene &sc, int prim, float b1, f
 	it.p = b0 * p0 + b1 * p1 + b2 * p2;
 	if (m.hasNormals) it.n = normalize(b0 * loadV(sc.nrm, v0) + b1 * loadV(sc.nrm, v1) + b2 * loadV(sc.nrm, v2));
 	else it.n = normalize(cross(p1 - p0, p2 - p0));
-	if (TEX && m.hasTangents) {
+	if (m.hasTangents) {
 		it.tangent = normalize(b0 * loadV(sc.tan, v0) + b1 * loadV(sc.tan, v1) + b2 * loadV(sc.tan, v2));
 		it.tangent = normalize(it.tangent - it.n * dot(it.n, it.tangent));
 	} else it.tangent = getPerpendicular(it.n);
@@ -711,7 +709,7 @@ KRR_DEV void prepareSurfaceInteraction(const DevScene &sc, int prim, float b1, f
 	if (m.hasUV) { // shading.h:147-149: b0 t0 + b1 t1 + b2 t2
 		it.u = b0 * sc.uv[2 * v0] + b1 * sc.uv[2 * v1] + b2 * sc.uv[2 * v2];
 		it.v = b0 * sc.uv[2 * v0 + 1] + b1 * sc.uv[2 * v1 + 1] + b2 * sc.uv[2 * v2 + 1];
-		if (TEX && it.material >= 0) {
+		if (it.material >= 0) {
 			const int tn = sc.materials[it.material].texNormal;
 			if (tn >= 0) { // rgbToNormal (shading.h:32): 2 rgb - 1, in the (T, B, N) frame
 				const DevTexture t = sc.textures[tn];
@@ -750,10 +748,11 @@ KRR_DEV void prepareSurfaceRecord(const DevScene &sc, int prim, float b1, float 
 	it.u = it.v = 0.f;
 }
 
-// prepareSurfaceInteraction by the scene's kind.
+// prepareSurfaceInteraction by the scene's kind; TEX = false: no mesh has
+// tangents and no material a texture.
 template <bool TEX>
 KRR_DEV void surfaceAt(const DevScene &sc, int prim, float b1, float b2, const f3 &rayDir, int rayMedium, SurfaceInteraction &it) {
-	if constexpr (TEX) prepareSurfaceInteraction<true>(sc, prim, b1, b2, rayDir, rayMedium, it);
+	if constexpr (TEX) prepareSurfaceInteraction(sc, prim, b1, b2, rayDir, rayMedium, it);
 	else prepareSurfaceRecord(sc, prim, b1, b2, rayDir, rayMedium, it);
 }
 
