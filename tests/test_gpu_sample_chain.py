@@ -43,12 +43,24 @@ def test_chained_samples_in_media(krr, gpu):
                                           (301, 203, 1, {"refill_lanes": 12, "trace_block_size": 256}), (40, 30, 1, {"nrc": {"train_mod": 4}})])
 def test_few_paths_in_many_waves(krr, gpu, w, h, spp, more):
     """Frames of fewer paths than the launch has lanes are spread over more
-    waves with fewer lanes each; a launch held to few blocks ("occupancy")
-    fills its waves.  Both trace the same paths."""
+    waves with fewer lanes each.  Launches that fill their waves trace the
+    same paths: those over a ray queue (wavefront_depths 1) and, with the
+    radiance cache, those held to few blocks ("occupancy")."""
     print(f"case: field {w}x{h} {spp} spp {more}", flush=True)
     s = krr.Scene(icosphere_scene(count=64, level=2, res=(w, h)))
     params = dict({"spp": spp, "max_depth": 8, "refill_lanes": 8}, **more)
-    a, sa = gpu_render(krr, gpu, s, w, h, params)
-    b, sb = gpu_render(krr, gpu, s, w, h, dict(params, occupancy=0.01))
-    assert sa["closest_rays"] == sb["closest_rays"] and sa["shadow_rays"] == sb["shadow_rays"]
+    out = []
+    for p in (params, dict(params, **({"occupancy": 0.01} if "nrc" in more else {"wavefront_depths": 1}))):
+        wf = krr.WavefrontPathTracer(p)
+        wf.set_scene(s)
+        wf.resize(w, h)
+        film = gpu.DeviceBuffer(w * h * 16)
+        wf.begin_frame(s.camera(0), 1)
+        wf.render(film.ptr, 0)
+        st = wf.stats()
+        out.append((film.to_numpy(np.float32, (h, w, 4)), st["closest_rays"], st["shadow_rays"], wf.to_json()["launch_in_force"]["lanes"]))
+        wf.close()
+    (a, ca, sa, lanes), (b, cb, sb, full) = out
+    assert lanes < 64 and full == 64
+    assert ca == cb and sa == sb
     assert np.array_equal(a, b)
