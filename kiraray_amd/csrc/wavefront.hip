@@ -1740,14 +1740,6 @@ PathGrid pathGrid(int resident, int tb, int64_t paths, bool half) {
 	return g;
 }
 
-// Launch over a ray queue ("wavefront_depths"), whose rays fill waves: no more
-// blocks than the queue can hold rays for.
-PathGrid queueGrid(int resident, int tb, int64_t rays) {
-	PathGrid g;
-	g.blocks = (int) std::max<int64_t>(1, std::min<int64_t>(resident, (rays + tb - 1) / tb));
-	return g;
-}
-
 // A fraction of a persistent grid (at least one block).
 int scaledGrid(int g, float frac) { return std::max(1, (int) std::lround((double) g * (double) frac)); }
 
@@ -2290,18 +2282,18 @@ int ldsNodeCount(const krr_wf *wf) {
 
 // With every depth in the persistent launch, a launch runs several samples of
 // the frame's N pixels; the radiance cache answers its queries between samples,
-// and a ray queue (camera = false) holds one sample's paths.
+// and the paths of a ray queue (camera = false) fill waves, a sample at a time.
 //
 // A launch is not interrupted, so what it runs is bounded, by the samples a lane
 // chains and by the paths: 129 samples of a 1080p frame of the 1.31 M-triangle
-// field are one launch of 0.31 s, 256 of the 720p volume one of about 1.1 s (2 take 8.5 ms).  Every
-// launch waits for its longest pixel: 256 samples of the 256x256 Cornell box
-// take 24.6 ms in one launch and 26.9 ms in four.
+// field are one launch of 0.31 s, 256 of the 720p volume one of about 1.1 s (2 take
+// 8.5 ms).  Every launch waits for its longest pixel: 256 samples of the 256x256
+// Cornell box take 24.6 ms in one launch and 26.9 ms in four.
 constexpr int kLaunchSamples	= 256;
 constexpr int64_t kLaunchPaths = (int64_t) 1 << 28;
 LaunchShape launchShape(const krr_wf *wf, const PathGrid &g, int N, bool camera, bool nrc) {
 	const int64_t most = std::min<int64_t>(kLaunchSamples, std::max<int64_t>(1, kLaunchPaths / N));
-	return LaunchShape{g.blocks, g.lanes, camera && !nrc ? (int) std::min<int64_t>(wf->spp, most) : 1, wf->accel.ldsEntries()};
+	return LaunchShape{g.blocks, camera ? g.lanes : 64, camera && !nrc ? (int) std::min<int64_t>(wf->spp, most) : 1, wf->accel.ldsEntries()};
 }
 
 Json shapeJson(const LaunchShape &s) {
@@ -2744,7 +2736,6 @@ int frameLaunch(krr_wf *wf, int N, FrameLaunch &L) {
 		const size_t nodeBytes = (size_t) ldsNodeCount(wf) * sizeof(Bvh4Node);
 		auto mega = [&](bool nrc) {
 			const int resident = withMega<false>(media, count, nrc, L.plain, L.refill, L.dense, [&](auto k) { return decltype(k)::grid(tb, lds, 1 << 20, nodeBytes); });
-			if (wf->wavefrontDepths > 0) return queueGrid(scaledGrid(resident, wf->occupancy), tb, N);
 			return pathGrid(scaledGrid(resident, wf->occupancy), tb, N, !media && !L.refill && smallTree(wf->accel));
 		};
 		wf->gMega = mega(false);

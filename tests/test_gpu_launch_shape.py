@@ -24,21 +24,6 @@ def _frame(krr, gpu, scene, w, h, params, frame_index=3):
     return out, launch, stats
 
 
-@pytest.mark.parametrize("w,h", [(5, 3), (64, 48), (301, 200)])
-def test_queue_launches_are_no_larger_than_the_queue(krr, gpu, w, h):
-    """Rays of a queue fill waves, so a launch over one needs a block per
-    trace_block_size rays; camera paths of a small frame take more."""
-    print(f"case: queue launch {w}x{h}", flush=True)
-    s = krr.Scene(icosphere_scene(count=64, level=2, res=(w, h)))
-    params = {"spp": 2, "max_depth": 5, "trace_block_size": 128}
-    a, la, _ = _frame(krr, gpu, s, w, h, dict(params, wavefront_depths=1))
-    b, lb, _ = _frame(krr, gpu, s, w, h, params)
-    print("queue", la, "camera", lb, flush=True)
-    assert (la["blocks"], la["lanes"], la["samples"]) == ((w * h + 127) // 128, 64, 1)
-    assert lb["blocks"] > la["blocks"] and lb["lanes"] < 64 and lb["samples"] == 2
-    assert np.array_equal(a, b)
-
-
 @pytest.mark.parametrize("scene,spp,more", [("cornell", 257, {}), ("cornell", 300, {"legacy_spp_accumulate": True}), ("field", 256, {"refill_lanes": 8}),
                                             ("field", 513, {"refill_lanes": 8})])
 def test_launches_run_a_bounded_number_of_samples(krr, gpu, scene, spp, more):
