@@ -320,7 +320,8 @@ typedef struct krr_wf krr_wf;
  *                            launch uses (in-flight path capacity)
  *   refill_lanes (-1)        persistent launch without media: a wave's
  *                            traversal round ends once fewer than this many
- *                            of its 64 lanes are still traversing; the
+ *                            of its 64 lanes (in proportion, of those that
+ *                            have a path) are still traversing; the
  *                            others shade or take their next ray, and the
  *                            unfinished rays resume in the next round (0: each
  *                            ray runs to its end; 1..64; -1: 8 for trees of
