@@ -69,3 +69,33 @@ def test_every_pixel_is_rendered_once(krr, gpu, w, h, spp, spheres):
     assert np.isfinite(out[0][0]).all() and out[0][1] >= w * h * spp
     for o in out[1:]:
         assert np.array_equal(o[0], out[0][0]) and o[1:] == out[0][1:]
+
+
+@pytest.mark.parametrize("n", [1000, 48601, 300000])
+def test_both_traces_share_one_overflow_area(krr, gpu, n):
+    """Closest hits and then as many shadow rays on a new accel allocate the
+    stack's overflow area once: free device memory does not change between."""
+    import ctypes as C
+    print(f"case: {n} rays, one allocation", flush=True)
+    s = krr.Scene(icosphere_scene(count=160, level=2, res=(32, 32)))
+    rng = np.random.default_rng(n)
+    r = np.zeros((n, 8), np.float32)
+    r[:, 0:3], r[:, 3], r[:, 4:7] = rng.random((n, 3)), np.inf, rng.standard_normal((n, 3))
+    d, hits, vis = gpu.DeviceBuffer.from_numpy(r), gpu.DeviceBuffer(16 * n), gpu.DeviceBuffer(4 * n)
+
+    def free():
+        gpu.synchronize()
+        f, t = C.c_size_t(), C.c_size_t()
+        gpu.check(gpu.runtime().hipMemGetInfo(C.byref(f), C.byref(t)))
+        return f.value
+
+    seen = []
+    for _ in range(3):
+        accel = krr.Accel(s.desc, {"stack_lds_entries": 0})
+        accel.trace_closest(d.ptr, n, hits.ptr, 0)
+        a = free()
+        accel.trace_any(d.ptr, n, vis.ptr, 0)
+        seen.append((a, free()))
+        accel.close()
+    print(seen, flush=True)
+    assert all(a == b for a, b in seen)
